@@ -221,6 +221,31 @@ int sa_score_stats(int dtype, const void* q, const void* k, const int64_t* q_len
                    double* out, void* stream);
 
 /*
+ * SelectiveMHA's training attention (modules/selective_attention.py:86-95,
+ * 125-144), fp32: out_i = softmax_j(scale q_i . k_j + [j != i] log_gate_j) v_j
+ * over j <= i (causal) or every j, and its backward, without the score matrix.
+ *   q, k, v, dout: (batch, heads, len, head_dim) fp32 by element strides:
+ *     `strides` holds batch, head and row strides of q, k, v (9 values; the
+ *     backward: of q, k, v, dout, 12), multiples of 4, the last dimension
+ *     contiguous, 16-byte aligned; read on the host during the call
+ *   log_gate (batch, heads, len) contiguous, -inf for dropped keys
+ *   out, dq, dk, dv (batch, heads, len, head_dim) contiguous, 16-byte aligned
+ *   row_max, row_rcp (batch, heads, len): the softmax's maximum and 1 / sum,
+ *     written by the forward and read by the backward
+ *   dlog_gate (batch, heads, len); delta (batch, heads, len): scratch
+ * head_dim 32, 64, 96 or 128.  Deterministic.
+ */
+int sa_gated_attn_train_fwd(const float* q, const float* k, const float* v, const float* log_gate,
+                            const int64_t* strides, int batch, int heads, int len, int head_dim,
+                            int causal, float scale, float* out, float* row_max, float* row_rcp,
+                            void* stream);
+int sa_gated_attn_train_bwd(const float* q, const float* k, const float* v, const float* log_gate,
+                            const float* out, const float* dout, const float* row_max,
+                            const float* row_rcp, const int64_t* strides, int batch, int heads,
+                            int len, int head_dim, int causal, float scale, float* dq, float* dk,
+                            float* dv, float* dlog_gate, float* delta, void* stream);
+
+/*
  * Small-batch linear layer of the decode steps (nn.Linear with x of at most 8
  * rows): y (M, N) = bf16(x (M, K) . W (N, K)^T + bias (N,)), bf16, fp32
  * accumulation; M in 1..8, K % 8 == 0, K <= 4096, x and W 16-byte aligned; bias may

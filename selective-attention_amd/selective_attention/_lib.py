@@ -52,6 +52,10 @@ SIGNATURES: dict[str, list] = {
     "sa_silu_mul_bf16": [_vp, _vp, _i64, _vp, _vp],
     "sa_score_stats_workspace_size": [_i, _i, _i],
     "sa_score_stats": [_i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp, _sz, _vp, _vp],
+    "sa_gated_attn_train_fwd": [_vp, _vp, _vp, _vp, ctypes.POINTER(_i64), _i, _i, _i, _i, _i, _f,
+                                _vp, _vp, _vp, _vp],
+    "sa_gated_attn_train_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.POINTER(_i64), _i,
+                                _i, _i, _i, _i, _f, _vp, _vp, _vp, _vp, _vp, _vp],
     "sa_gemv_bf16": [_vp, _vp, _vp, _i, _i, _i, _vp, _vp],
     "sa_gemv_bf16_multi": [_vp, _vp, _i, _i, _i, ctypes.POINTER(_vp), ctypes.POINTER(_vp),
                            ctypes.POINTER(_i), ctypes.POINTER(_vp), _vp],

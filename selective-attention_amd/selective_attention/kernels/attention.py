@@ -9,6 +9,7 @@ softmax (modules/selective_attention.py:99-144): an optional per-key bias
 """
 from __future__ import annotations
 
+import ctypes
 import math
 
 import torch
@@ -185,3 +186,55 @@ def score_stats(q, k, q_lengths=None, k_lengths=None, causal=True, softmax_scale
               Lq, Lk, D, 1 if causal else 0, scale, _lib.ptr(ws), nbytes, _lib.ptr(out),
               _lib.stream_of(q))
     return out
+
+
+TRAIN_HEAD_DIMS = (32, 64, 96, 128)
+
+
+def _train_rows(t: torch.Tensor) -> torch.Tensor:
+    """t (batch, heads, len, head_dim) fp32 as the training kernels read it: any
+    batch / head / row strides that keep rows 16-byte aligned, else a copy."""
+    st = t.stride()
+    if st[3] != 1 or any(x % 4 for x in st[:3]) or t.data_ptr() % 16 != 0:
+        t = t.clone(memory_format=torch.contiguous_format)
+    return t
+
+
+def _strides(*tensors):
+    vals = [x for t in tensors for x in t.stride()[:3]]
+    return (ctypes.c_int64 * len(vals))(*vals)
+
+
+def gated_attn_train_forward(q, k, v, log_gate, causal):
+    """q, k, v (batch, heads, len, head_dim) float32, head_dim in
+    TRAIN_HEAD_DIMS; log_gate (batch, heads, len) float32.  Returns out
+    (batch, heads, len, head_dim) and the softmax's row maximum and 1 / sum,
+    each (batch, heads, len)."""
+    require_device(q, k, v, log_gate)
+    b, H, L, D = q.shape
+    q, k, v = _train_rows(q), _train_rows(k), _train_rows(v)
+    lg = log_gate.contiguous()
+    out = torch.empty((b, H, L, D), dtype=torch.float32, device=q.device)
+    stats = torch.empty((2, b, H, L), dtype=torch.float32, device=q.device)
+    _lib.call("sa_gated_attn_train_fwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(lg),
+              _strides(q, k, v), b, H, L, D, 1 if causal else 0, D ** -0.5, _lib.ptr(out),
+              _lib.ptr(stats[0]), _lib.ptr(stats[1]), _lib.stream_of(q))
+    return out, stats
+
+
+def gated_attn_train_backward(q, k, v, log_gate, out, stats, dout, causal):
+    """(dq, dk, dv, dlog_gate) of gated_attn_train_forward for the upstream
+    gradient dout (batch, heads, len, head_dim) float32."""
+    require_device(q, k, v, log_gate, out, stats, dout)
+    b, H, L, D = q.shape
+    q, k, v, dout = _train_rows(q), _train_rows(k), _train_rows(v), _train_rows(dout)
+    lg = log_gate.contiguous()
+    dq, dk, dv = (torch.empty((b, H, L, D), dtype=torch.float32, device=q.device)
+                  for _ in range(3))
+    dlg = torch.empty((b, H, L), dtype=torch.float32, device=q.device)
+    delta = torch.empty_like(dlg)
+    _lib.call("sa_gated_attn_train_bwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(lg),
+              _lib.ptr(out), _lib.ptr(dout), _lib.ptr(stats[0]), _lib.ptr(stats[1]),
+              _strides(q, k, v, dout), b, H, L, D, 1 if causal else 0, D ** -0.5, _lib.ptr(dq),
+              _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(dlg), _lib.ptr(delta), _lib.stream_of(q))
+    return dq, dk, dv, dlg

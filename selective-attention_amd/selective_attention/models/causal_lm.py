@@ -7,9 +7,8 @@ Precision: to_bf16() puts the matmul weights and activations in bfloat16
 and keeps the SSM's A_log / delta_bias / D and conv weights, the RMSNorm
 weights and the attention score statistics in float32 (all are per-channel
 vectors); RoPE's frequencies and angles are fp32 whatever the module dtype.
-Not built: training through SelectiveMHA (no attention backward kernel),
-the gate-analysis statistics and compute_attn_gate_threshold (calibration
-runs on analysis histograms, outside the kernel path).
+Not built: the gate-analysis statistics and compute_attn_gate_threshold
+(calibration runs on analysis histograms, outside the kernel path).
 """
 from __future__ import annotations
 

@@ -19,8 +19,7 @@ Training (:197-277): the per-head std of the valid scores comes from the
 in-kernel statistics (ScoreStdFn: count, sum and sum of squares reduced
 without a score matrix, differentiable), score_std_ema takes the running
 average, the log-gate is log(gate) * std * penalty, and the gated softmax
-runs densely in torch under autograd (this package has no attention
-backward kernel).
+runs forward and backward in fp32 kernels (gated_attention_train).
 """
 from __future__ import annotations
 

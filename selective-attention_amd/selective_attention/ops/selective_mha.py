@@ -26,15 +26,16 @@ ops:
   in-kernel reduction score_stats (count, sum, sum of squares, no score
   matrix); its backward carries d std_h / d s_ij = (s_ij - mean_h) /
   (count_h std_h) to q and k by query chunks.
-* gated_attention_train, cross_attention_train: the training attention
-  itself, the reference's dense gated softmax under autograd (there is no
-  attention backward kernel here), in fp32.
+* gated_attention_train: the training attention itself, the reference's gated
+  softmax, forward and backward in fp32 kernels without a score matrix.
+* cross_attention_train: the cross-attention's, dense under autograd, in fp32.
 """
 from __future__ import annotations
 
 import torch
 
-from ..kernels.attention import score_stats
+from ..kernels.attention import (TRAIN_HEAD_DIMS, gated_attn_train_backward,
+                                 gated_attn_train_forward, score_stats)
 from ..kernels.lm_ops import paged_kv_append, paged_kv_build
 from .attention import attn_varlen, paged_decode_attn
 
@@ -99,20 +100,70 @@ class ScoreStdFn(torch.autograd.Function):
         return dq.to(q.dtype), dk.to(k.dtype), None, None, None, None
 
 
-def gated_attention_train(q_rot, k_rot, v, log_gate, causal=True):
-    """SelectiveMHA's training attention (modules/selective_attention.py:86-95,
-    125-144): softmax_j(scale q_i . k_j + [j != i] log_gate_j) v_j with keys
-    after the query at -inf when causal; dense, in fp32, under autograd.
-    q_rot, k_rot, v (batch, heads, seq_len, head_dim); log_gate (batch,
-    heads, seq_len).  Returns (batch, heads, seq_len, head_dim) float32."""
-    L, D = q_rot.shape[-2], q_rot.shape[-1]
-    s = torch.matmul(q_rot.float(), k_rot.float().transpose(-2, -1).contiguous()) * D ** -0.5
+def _gated_attention_dense(q, k, v, log_gate, causal):
+    """gated_attention_train as dense torch ops on float32 tensors."""
+    L, D = q.shape[-2], q.shape[-1]
+    s = torch.matmul(q, k.transpose(-2, -1).contiguous()) * D ** -0.5
     diag = torch.eye(L, dtype=torch.bool, device=s.device)
-    s = torch.where(diag, s, s + log_gate.float()[:, :, None, :])
+    s = torch.where(diag, s, s + log_gate[:, :, None, :])
     if causal:
         s = s.masked_fill(~torch.tril(torch.ones(L, L, dtype=torch.bool, device=s.device)),
                           float("-inf"))
-    return torch.matmul(torch.softmax(s, dim=-1), v.float())
+    return torch.matmul(torch.softmax(s, dim=-1), v)
+
+
+class GatedAttnTrainFn(torch.autograd.Function):
+    """gated_attention_train on the fp32 MFMA kernels.  A backward that is itself
+    recorded (create_graph) differentiates the dense form instead."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, log_gate, causal):
+        out, stats = gated_attn_train_forward(q, k, v, log_gate, causal)
+        ctx.save_for_backward(q, k, v, log_gate, out, stats)
+        ctx.causal = causal
+        return out
+
+    @staticmethod
+    def backward(ctx, dout):
+        q, k, v, log_gate, out, stats = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            need = ctx.needs_input_grad[:4]
+            dense = _gated_attention_dense(q, k, v, log_gate, ctx.causal)
+            wanted = [t for t, n in zip((q, k, v, log_gate), need) if n]
+            grads = iter(torch.autograd.grad(dense, wanted, dout, create_graph=True))
+            return tuple(next(grads) if n else None for n in need) + (None,)
+        return gated_attn_train_backward(q, k, v, log_gate, out, stats, dout, ctx.causal) + (None,)
+
+
+def _train_kernel_ok(q, k, v, log_gate) -> bool:
+    """Whether the training kernels take this call: plain device tensors of equal
+    shapes (the dense form broadcasts), a head_dim they are built for, and
+    nothing that has to see the dense form's own ops (autocast, tracing,
+    functorch transforms, forward-mode AD, dispatch modes)."""
+    ts = (q, k, v, log_gate)
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
+                and t.is_floating_point() and t.device == q.device for t in ts)
+            and q.dim() == 4 and q.shape == k.shape == v.shape and log_gate.shape == q.shape[:3]
+            and q.shape[-1] in TRAIN_HEAD_DIMS and 0 < q.numel()
+            and q.shape[0] * q.shape[1] * ((q.shape[2] + 63) // 64) < 2 ** 31
+            and not torch.is_autocast_enabled("cuda")
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def gated_attention_train(q_rot, k_rot, v, log_gate, causal=True):
+    """SelectiveMHA's training attention (modules/selective_attention.py:86-95,
+    125-144): softmax_j(scale q_i . k_j + [j != i] log_gate_j) v_j with keys
+    after the query at -inf when causal; in fp32, under autograd, on the
+    training kernels (no score matrix), or densely where they do not apply.
+    q_rot, k_rot, v (batch, heads, seq_len, head_dim); log_gate (batch,
+    heads, seq_len).  Returns (batch, heads, seq_len, head_dim) float32."""
+    if _train_kernel_ok(q_rot, k_rot, v, log_gate):
+        return GatedAttnTrainFn.apply(q_rot.float(), k_rot.float(), v.float(), log_gate.float(),
+                                      bool(causal))
+    return _gated_attention_dense(q_rot.float(), k_rot.float(), v.float(), log_gate.float(), causal)
 
 
 def selective_mha_prefill(q_rot: torch.Tensor, k_rot: torch.Tensor, v: torch.Tensor,
