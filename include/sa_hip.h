@@ -221,6 +221,27 @@ int sa_score_stats(int dtype, const void* q, const void* k, const int64_t* q_len
                    double* out, void* stream);
 
 /*
+ * The same statistics without visiting every pair (Gram matrices of the keys),
+ * and the gradient of the per-head std.  `out` (heads, 3) as sa_score_stats;
+ * `std` (heads,) fp32 or NULL: sqrt(max(sum^2 / n - (sum / n)^2, 0)).
+ * sa_score_std_bwd: for stats = out of sa_score_moments and std_grad (heads,)
+ * fp32, dq and dk (shapes and dtype of q and k) of std_grad . std; a head of
+ * std 0 passes no gradient.  Sizes must be positive; q, k, dq, dk and the
+ * workspace (sa_score_moments_workspace_size bytes) 16-byte aligned.
+ * Deterministic.
+ */
+size_t sa_score_moments_workspace_size(int batch, int heads, int q_len, int k_len, int head_dim);
+int sa_score_moments(int dtype, const void* q, const void* k, const int64_t* q_length,
+                     const int64_t* k_length, int batch, int heads, int q_len, int k_len,
+                     int head_dim, int causal, float scale, void* workspace, size_t workspace_bytes,
+                     double* out, float* std, void* stream);
+int sa_score_std_bwd(int dtype, const void* q, const void* k, const int64_t* q_length,
+                     const int64_t* k_length, int batch, int heads, int q_len, int k_len,
+                     int head_dim, int causal, float scale, const double* stats,
+                     const float* std_grad, void* dq, void* dk, void* workspace,
+                     size_t workspace_bytes, void* stream);
+
+/*
  * SelectiveMHA's training attention (modules/selective_attention.py:86-95,
  * 125-144), fp32: out_i = softmax_j(scale q_i . k_j + [j != i] log_gate_j) v_j
  * over j <= i (causal) or every j, and its backward, without the score matrix.

@@ -33,6 +33,7 @@
 // for the same (elementwise passes over 0.5 GB score matrices, and products
 // over the masked half).
 #include "common.h"
+#include "fp32_tile.h"
 #include "prof.h"
 
 namespace sa {
@@ -43,8 +44,6 @@ struct TrainDims {
   float scale;
   long q[3], k[3], v[3], d[3];   // element strides of batch, head, row
 };
-
-constexpr int kRows = 64;   // rows of a tile, and rows a block owns
 
 // block -> (batch * H + head, tile index): the tile index runs from the
 // longest walk to the shortest over the whole launch, every other run of
@@ -61,85 +60,13 @@ __device__ __forceinline__ void block_tile(int bid, int nblocks, int nbh, bool l
   if (last_longest) tile = ntiles - 1 - tile;
 }
 
-// tile rows r0 .. r0 + 63 of x (row stride ld elements), zero past L, as
-// D / 16 float4 per thread
-template <int D>
-struct TileRegs {
-  float4 r[D / 16];
-};
-template <int D>
-__device__ __forceinline__ void tile_load(TileRegs<D>& t, const float* x, long ld, int r0, int L,
-                                          int tid) {
-#pragma unroll
-  for (int p = 0; p < D / 16; ++p) {
-    const int idx = tid + 256 * p, row = idx / (D / 4), c = 4 * (idx % (D / 4));
-    const int g = r0 + row;
-    t.r[p] = g < L ? *reinterpret_cast<const float4*>(x + g * ld + c) : float4{0.f, 0.f, 0.f, 0.f};
-  }
-}
-template <int D>
-__device__ __forceinline__ void tile_store(const TileRegs<D>& t, float* lds, int tid) {
-#pragma unroll
-  for (int p = 0; p < D / 16; ++p) {
-    const int idx = tid + 256 * p, row = idx / (D / 4), c = 4 * (idx % (D / 4));
-    *reinterpret_cast<float4*>(lds + row * (D + 4) + c) = t.r[p];
-  }
-}
-
-// one row of D floats as a score operand: lane group g holds elements
-// 16 s + 4 g + i
-template <int D>
-__device__ __forceinline__ void row_frag(v4f (&f)[D / 16], const float* row, int lg, bool ok) {
-#pragma unroll
-  for (int s = 0; s < D / 16; ++s)
-    f[s] = ok ? *reinterpret_cast<const v4f*>(row + 16 * s + 4 * lg) : v4f{0.f, 0.f, 0.f, 0.f};
-}
-
-__device__ __forceinline__ v4f mfma_f32(float a, float b, const v4f& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-// acc[t] (rows 16 t + 4 g + i of the LDS tile, column li) = tile . f^T
-template <int D>
-__device__ __forceinline__ void score_tile(v4f (&acc)[4], const float* lds, const v4f (&f)[D / 16],
-                                           int li, int lg) {
-#pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int s = 0; s < D / 16; ++s) {
-    v4f a[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-      a[t] = *reinterpret_cast<const v4f*>(lds + (16 * t + li) * (D + 4) + 16 * s + 4 * lg);
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) acc[t] = mfma_f32(a[t][i], f[s][i], acc[t]);
-  }
-}
-
-// out[dt] (d = 16 dt + 4 g + i, column li) += tile^T . w, w[t][i] the weight
-// of tile row 16 t + 4 g + i
-template <int D>
-__device__ __forceinline__ void weigh_tile(v4f (&out)[D / 16], const float* lds, const v4f (&w)[4],
-                                           int li, int lg) {
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float* row = lds + (16 * t + 4 * lg + i) * (D + 4) + li;
-#pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) out[dt] = mfma_f32(row[16 * dt], w[t][i], out[dt]);
-    }
-}
-
 __device__ __forceinline__ float expf_fast(float x) { return fast_exp2(x * kLog2e); }
 
 // ---------------------------------------------------------------------------
 // forward: out, and per query the softmax's maximum and 1 / sum
 // ---------------------------------------------------------------------------
 template <int D, bool CAUSAL>
-__global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void attn_train_fwd_kernel(
+__global__ __launch_bounds__(256, D <= 64 ? (CAUSAL ? 3 : 2) : 1) void attn_train_fwd_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v,
     const float* __restrict__ log_gate, TrainDims dm, float* __restrict__ out,
     float* __restrict__ smax, float* __restrict__ srcp) {

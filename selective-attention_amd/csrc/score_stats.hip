@@ -20,7 +20,25 @@
 // into bf16 hi + lo (products hi*hi + lo*hi + hi*lo).  Per-lane tile sums
 // are fp32, running sums fp64; each block writes (count, sum, sum^2) and
 // score_stats_reduce sums those in a fixed order (deterministic).
+//
+// The moments without the pairs (sa_score_moments, sa_score_std_bwd).  The
+// scores are bilinear, so over a set of keys with M = sum k k^T and
+// kappa = sum k the sum of a query's scores is scale q . kappa and the sum of
+// their squares scale^2 q . M q; the gradient of the std,
+//   g_ij = coef (s_ij - mean),   dq_i = scale sum_j g_ij k_j,
+// is scale coef (scale M q_i - mean kappa), and dk_j the same over the queries.
+// Causal attention needs M over the keys before each query: Gram matrices
+// of 256-row chunks (score_gram_kernel), their exclusive prefix (suffix for
+// dk) over the chunks (score_gram_scan_kernel), and in score_apply_kernel
+// the chunk's own pairs as 64x64 score tiles.  Work per row: 4 D^2 FLOP for
+// the Gram matrix and its product and 160 pairs on average, against L / 2
+// pairs.  All products are fp32 MFMA (bf16 inputs are widened); at b 4, H 8,
+// L 2048, D 64, fp32: statistics 51 us (Gram 12, scan 5, apply 33; the pass
+// over every pair 202), gradient 123 us (the same in torch ops by query chunks
+// of the dense scores 2.7 ms).  sa_score_stats keeps the pass over every pair
+// for callers that size its workspace without the key length and head_dim.
 #include "common.h"
+#include "fp32_tile.h"
 #include "prof.h"
 
 namespace sa {
@@ -127,10 +145,12 @@ __global__ __launch_bounds__(256) void score_stats_kernel(const T* __restrict__ 
   }
 }
 
-// out[h] = (count, sum, sum^2) over batch rows and query blocks of head h
+// out[h] = (count, sum, sum^2) over batch rows and query blocks of head h, and
+// (when std is given) the population std sqrt(max(sum^2 / n - (sum / n)^2, 0))
 __global__ __launch_bounds__(256) void score_stats_reduce_kernel(const double* __restrict__ part,
                                                                  int batch, int H, int nqb,
-                                                                 double* __restrict__ out) {
+                                                                 double* __restrict__ out,
+                                                                 float* __restrict__ std) {
   __shared__ double red[256][3];
   const int h = blockIdx.x, tid = threadIdx.x;
   double a[3] = {0.0, 0.0, 0.0};
@@ -152,6 +172,316 @@ __global__ __launch_bounds__(256) void score_stats_reduce_kernel(const double* _
     __syncthreads();
   }
   if (tid < 3) out[h * 3 + tid] = red[0][tid];
+  if (std && tid == 0) {
+    const double n = fmax(red[0][0], 1.0), mean = red[0][1] / n;
+    const double var = red[0][2] / n - mean * mean;
+    std[h] = static_cast<float>(sqrt(var < 0.0 ? 0.0 : var));   // a NaN stays one
+  }
+}
+
+// ---------------------------------------------------------------------------
+// moments through Gram matrices
+// ---------------------------------------------------------------------------
+constexpr int kChunk = 256;   // rows of a Gram matrix
+enum class Pairs { kBefore, kAfter, kAll };   // keys y <= x, y >= x, every y
+
+__device__ __forceinline__ int row_count(const int64_t* length, int b, int L) {
+  return length ? static_cast<int>(min(max(length[b], int64_t{0}), int64_t{L})) : L;
+}
+
+// one chunk's sum y y^T (D x D) followed by sum y (D); rows past the length
+// count as zero.  The 16x16 result tiles go round the four waves.
+template <typename T, int D>
+__global__ __launch_bounds__(256) void score_gram_kernel(const T* __restrict__ y,
+                                                         const int64_t* __restrict__ length, int H,
+                                                         int L, int nc, float* __restrict__ gram) {
+  constexpr int NT = D / 16, NP = NT * NT / 4;
+  __shared__ __align__(16) float yt[kRows * (D + 4)];
+  const int bh = blockIdx.x / nc, c = blockIdx.x % nc;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, lg = lane >> 4;
+  const int len = row_count(length, bh / H, L);
+  const T* yh = y + static_cast<long>(bh) * L * D;
+  float* out = gram + static_cast<long>(blockIdx.x) * (D * D + D);
+  v4f acc[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+  float sum = 0.f;
+  TileRegs<D> yr;
+  const int r1 = min(kChunk * (c + 1), len);   // (may lie before the chunk: zeros are written)
+  tile_load<D>(yr, yh, D, kChunk * c, r1, tid);
+  for (int r0 = kChunk * c; r0 < r1; r0 += kRows) {
+    __syncthreads();
+    tile_store<D>(yr, yt, tid);
+    __syncthreads();
+    if (r0 + kRows < r1) tile_load<D>(yr, yh, D, r0 + kRows, r1, tid);
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float* row = yt + (16 * t + 4 * lg + i) * (D + 4) + li;
+        float a[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) a[n] = row[16 * n];
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+          // tile pair w + 4 j; w is wave-uniform, so the selects are scalar
+          const int p = w + 4 * j;
+          float x = 0.f, z = 0.f;
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            x = p / NT == n ? a[n] : x;
+            z = p % NT == n ? a[n] : z;
+          }
+          acc[j] = mfma_f32(x, z, acc[j]);
+        }
+      }
+    if (tid < D)
+      for (int r = 0; r < kRows; ++r) sum += yt[r * (D + 4) + tid];
+  }
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    const int p = w + 4 * j;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      out[(16 * (p / NT) + 4 * lg + i) * D + 16 * (p % NT) + li] = acc[j][i];
+  }
+  if (tid < D) out[D * D + tid] = sum;
+}
+
+// over the chunks of one (batch row, head), in place: each slot becomes the sum
+// of the slots before it (kBefore), after it (kAfter); kAll: slot 0 the total
+template <Pairs PAIRS>
+__global__ __launch_bounds__(256) void score_gram_scan_kernel(float* __restrict__ gram, int nc,
+                                                              int size) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= size) return;
+  float* g = gram + static_cast<long>(blockIdx.y) * nc * size + i;
+  float run = 0.f;
+  for (int c0 = 0; c0 < nc; c0 += 8) {
+    float t[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = min(c0 + u, nc - 1);
+      t[u] = g[static_cast<long>(PAIRS == Pairs::kAfter ? nc - 1 - c : c) * size];
+    }
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int c = c0 + u;
+      if (c < nc) {
+        if (PAIRS != Pairs::kAll) g[static_cast<long>(PAIRS == Pairs::kAfter ? nc - 1 - c : c) * size] = run;
+        run += t[u];
+      }
+    }
+  }
+  if (PAIRS == Pairs::kAll) g[0] = run;
+}
+
+// 64 rows x against the rows y they pair with.  STATS: (count, sum, sum^2) of
+// the scores.  Otherwise the gradient of the std:
+//   dx_i = scale sum_j coef (s_ij - mean) y_j
+template <typename T, int D, Pairs PAIRS, bool STATS>
+__global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void score_apply_kernel(
+    const T* __restrict__ x, const T* __restrict__ y, const int64_t* __restrict__ x_length,
+    const int64_t* __restrict__ y_length, int H, int Lx, int Ly, int nc, float scale,
+    const float* __restrict__ gram, const double* __restrict__ stats, const float* __restrict__ g,
+    double* __restrict__ part, T* __restrict__ dx) {
+  constexpr int NT = D / 16;
+  __shared__ __align__(16) float yt[kRows * (D + 4)];
+  __shared__ double red[4][3];
+  const int nxb = (Lx + kRows - 1) / kRows;
+  const int xb = blockIdx.x % nxb, bh = blockIdx.x / nxb, b = bh / H, h = bh % H;
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, lg = lane >> 4;
+  const int xlen = row_count(x_length, b, Lx), ylen = row_count(y_length, b, Ly);
+  const T* yh = y + static_cast<long>(bh) * Ly * D;
+  const int xi = kRows * xb + 16 * w + li;
+  const long row = static_cast<long>(bh) * Lx + min(xi, Lx - 1);
+  v4f xf[NT], acc[NT];
+  row_frag<D>(xf, x + row * D, lg, xi < xlen);
+#pragma unroll
+  for (int i = 0; i < NT; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
+
+  float coef = 0.f, mean = 0.f;
+  if (!STATS) {
+    const double n = fmax(stats[3 * h], 1.0), mu = stats[3 * h + 1] / n;
+    const double var = stats[3 * h + 2] / n - mu * mu, sd = sqrt(var < 0.0 ? 0.0 : var);
+    coef = sd > 0.0 ? static_cast<float>(static_cast<double>(g[h]) / (n * sd)) : 0.f;
+    mean = static_cast<float>(mu);
+  }
+
+  // rows y outside the chunk, through their Gram matrix
+  const int c = PAIRS == Pairs::kAll ? 0 : kRows * xb / kChunk;
+  const bool outside = PAIRS == Pairs::kAll || (PAIRS == Pairs::kBefore ? c > 0 : c + 1 < nc);
+  double s1 = 0.0, s2 = 0.0;
+  if (outside) {
+    const float* gm = gram + (static_cast<long>(bh) * nc + c) * (D * D + D);
+#pragma unroll
+    for (int s = 0; s < NT; ++s) {
+      v4f a[NT];
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+        a[n] = *reinterpret_cast<const v4f*>(gm + (16 * n + li) * D + 16 * s + 4 * lg);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = mfma_f32(a[n][i], xf[s][i], acc[n]);
+    }
+    float t1 = 0.f, t2 = 0.f;
+#pragma unroll
+    for (int s = 0; s < NT; ++s) {
+      const v4f kap = *reinterpret_cast<const v4f*>(gm + D * D + 16 * s + 4 * lg);
+      if (STATS) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          t1 = fmaf(xf[s][i], kap[i], t1);
+          t2 = fmaf(xf[s][i], acc[s][i], t2);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[s][i] = coef * (scale * acc[s][i] - mean * kap[i]);
+      }
+    }
+    s1 = static_cast<double>(t1) * scale;
+    s2 = static_cast<double>(t2) * scale * scale;
+  }
+
+  // the chunk's own pairs: tiles of 64 rows y
+  if (PAIRS != Pairs::kAll) {
+    const int first = PAIRS == Pairs::kBefore ? c * (kChunk / kRows) : xb;
+    const int last = PAIRS == Pairs::kBefore ? xb : min((c + 1) * (kChunk / kRows), nxb) - 1;
+    TileRegs<D> yr;
+    tile_load<D>(yr, yh, D, kRows * first, ylen, tid);
+    for (int t0 = first; t0 <= last; ++t0) {
+      __syncthreads();
+      tile_store<D>(yr, yt, tid);
+      __syncthreads();
+      if (t0 < last) tile_load<D>(yr, yh, D, kRows * (t0 + 1), ylen, tid);
+      v4f s[4];
+      score_tile<D>(s, yt, xf, li, lg);
+      // rows past a length are zero on either side and add nothing; the pair
+      // order matters in the diagonal tile alone
+      float t1 = 0.f, t2 = 0.f;
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int yi = kRows * t0 + 16 * t + 4 * lg + i;
+          const bool ok = t0 != xb || (PAIRS == Pairs::kBefore ? yi <= xi : yi >= xi);
+          const float v = s[t][i] * scale;
+          if (STATS) {
+            t1 += ok ? v : 0.f;
+            t2 += ok ? v * v : 0.f;
+          } else {
+            s[t][i] = ok ? coef * (v - mean) : 0.f;
+          }
+        }
+      if (STATS) {
+        s1 += t1;
+        s2 += t2;
+      } else {
+        weigh_tile<D>(acc, yt, s, li, lg);
+      }
+    }
+  }
+  if (!STATS) {
+    if (xi >= Lx) return;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+      store4(dx + row * D + 16 * i + 4 * lg,
+             xi < xlen ? acc[i] * scale : v4f{0.f, 0.f, 0.f, 0.f});
+    return;
+  }
+  double n = xi < xlen && lg == 0 ? (PAIRS == Pairs::kAll ? ylen : min(xi + 1, ylen)) : 0.0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    s1 += __shfl_xor(s1, o, 64);
+    s2 += __shfl_xor(s2, o, 64);
+    n += __shfl_xor(n, o, 64);
+  }
+  if (lane == 0) {
+    red[w][0] = n;
+    red[w][1] = s1;
+    red[w][2] = s2;
+  }
+  __syncthreads();
+  if (tid < 3)
+    part[static_cast<long>(blockIdx.x) * 3 + tid] =
+        ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
+}
+
+// Gram matrices of y and their scan; nothing to do for causal rows of one chunk
+template <typename T, int D, Pairs PAIRS>
+int launch_gram(const T* y, const int64_t* length, int batch, int H, int L, float* gram,
+                hipStream_t s) {
+  const int nc = (L + kChunk - 1) / kChunk, size = D * D + D;
+  if (PAIRS != Pairs::kAll && nc == 1) return 0;
+  {
+    ProfScope prof_("score_gram", s);
+    hipLaunchKernelGGL((score_gram_kernel<T, D>), dim3(static_cast<unsigned>(batch) * H * nc),
+                       dim3(256), 0, s, y, length, H, L, nc, gram);
+    SA_CHECK_LAUNCH("score_gram");
+  }
+  if (nc == 1) return 0;
+  // (batch row, head) in y, at most 65535 of them a launch
+  const int rows = batch * H;
+  for (int r0 = 0; r0 < rows; r0 += 65535) {
+    ProfScope prof_("score_gram_scan", s);
+    hipLaunchKernelGGL((score_gram_scan_kernel<PAIRS>),
+                       dim3((size + 255) / 256, min(rows - r0, 65535)), dim3(256), 0, s,
+                       gram + static_cast<long>(r0) * nc * size, nc, size);
+    SA_CHECK_LAUNCH("score_gram_scan");
+  }
+  return 0;
+}
+
+template <typename T, int D, Pairs PAIRS, bool STATS>
+int launch_apply(const T* x, const T* y, const int64_t* x_length, const int64_t* y_length,
+                 int batch, int H, int Lx, int Ly, float scale, float* gram, const double* stats,
+                 const float* g, double* part, T* dx, hipStream_t s) {
+  const int rc = launch_gram<T, D, PAIRS>(y, y_length, batch, H, Ly, gram, s);
+  if (rc) return rc;
+  const int nc = (Ly + kChunk - 1) / kChunk;
+  const unsigned blocks = static_cast<unsigned>(batch) * H * ((Lx + kRows - 1) / kRows);
+  ProfScope prof_(STATS ? "score_moments" : "score_std_bwd", s);
+  hipLaunchKernelGGL((score_apply_kernel<T, D, PAIRS, STATS>), dim3(blocks), dim3(256), 0, s, x, y,
+                     x_length, y_length, H, Lx, Ly, nc, scale, gram, stats, g, part, dx);
+  SA_CHECK_LAUNCH(STATS ? "score_moments" : "score_std_bwd");
+  return 0;
+}
+
+template <typename T, int D>
+int launch_moments(const void* q, const void* k, const int64_t* ql, const int64_t* kl, int batch,
+                   int H, int Lq, int Lk, int causal, float scale, double* part, float* gram,
+                   double* out, float* std, hipStream_t s) {
+  const T *qt = static_cast<const T*>(q), *kt = static_cast<const T*>(k);
+  const int rc =
+      causal ? launch_apply<T, D, Pairs::kBefore, true>(qt, kt, ql, kl, batch, H, Lq, Lk, scale,
+                                                        gram, nullptr, nullptr, part, nullptr, s)
+             : launch_apply<T, D, Pairs::kAll, true>(qt, kt, ql, kl, batch, H, Lq, Lk, scale, gram,
+                                                     nullptr, nullptr, part, nullptr, s);
+  if (rc) return rc;
+  ProfScope prof_("score_stats_reduce", s);
+  hipLaunchKernelGGL(score_stats_reduce_kernel, dim3(H), dim3(256), 0, s, part, batch, H,
+                     (Lq + kRows - 1) / kRows, out, std);
+  SA_CHECK_LAUNCH("score_stats_reduce");
+  return 0;
+}
+
+template <typename T, int D>
+int launch_std_bwd(const void* q, const void* k, const int64_t* ql, const int64_t* kl, int batch,
+                   int H, int Lq, int Lk, int causal, float scale, const double* stats,
+                   const float* g, float* gram, void* dq, void* dk, hipStream_t s) {
+  const T *qt = static_cast<const T*>(q), *kt = static_cast<const T*>(k);
+  T *dqt = static_cast<T*>(dq), *dkt = static_cast<T*>(dk);
+  if (causal) {
+    const int rc = launch_apply<T, D, Pairs::kBefore, false>(
+        qt, kt, ql, kl, batch, H, Lq, Lk, scale, gram, stats, g, nullptr, dqt, s);
+    return rc ? rc : launch_apply<T, D, Pairs::kAfter, false>(kt, qt, kl, ql, batch, H, Lk, Lq,
+                                                              scale, gram, stats, g, nullptr, dkt, s);
+  }
+  const int rc = launch_apply<T, D, Pairs::kAll, false>(qt, kt, ql, kl, batch, H, Lq, Lk, scale,
+                                                        gram, stats, g, nullptr, dqt, s);
+  return rc ? rc : launch_apply<T, D, Pairs::kAll, false>(kt, qt, kl, ql, batch, H, Lk, Lq, scale,
+                                                          gram, stats, g, nullptr, dkt, s);
 }
 
 template <typename T, int D>
@@ -168,7 +498,8 @@ int launch_score_stats(const void* q, const void* k, const int64_t* q_length, co
     SA_CHECK_LAUNCH("score_stats");
   }
   ProfScope prof_("score_stats_reduce", s);
-  hipLaunchKernelGGL(score_stats_reduce_kernel, dim3(H), dim3(256), 0, s, part, batch, H, nqb, out);
+  hipLaunchKernelGGL(score_stats_reduce_kernel, dim3(H), dim3(256), 0, s, part, batch, H, nqb, out,
+                     nullptr);
   SA_CHECK_LAUNCH("score_stats_reduce");
   return 0;
 }
@@ -215,7 +546,7 @@ extern "C" int sa_score_stats(int dtype, const void* q, const void* k, const int
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (batch == 0 || q_len == 0 || k_len == 0) {   // no pairs: the reduction writes zeros
     hipLaunchKernelGGL(sa::score_stats_reduce_kernel, dim3(heads), dim3(256), 0, s, nullptr, 0,
-                       heads, 0, out);
+                       heads, 0, out, nullptr);
     SA_CHECK_LAUNCH("score_stats_reduce");
     return 0;
   }
@@ -233,4 +564,77 @@ extern "C" int sa_score_stats(int dtype, const void* q, const void* k, const int
                                            k_len, causal, scale, part, out, s);
   sa_set_error("sa_score_stats: unsupported dtype %d", dtype);
   return 1;
+}
+
+namespace {
+// doubles of the block partials, rounded up so that the Gram matrices behind
+// them stay 16-byte aligned
+size_t moments_part(int batch, int heads, int q_len) {
+  return (static_cast<size_t>(batch) * heads * ((q_len + sa::kRows - 1) / sa::kRows) * 3 + 1) &
+         ~static_cast<size_t>(1);
+}
+int check_moments(const char* what, int dtype, const void* q, const void* k, int batch, int heads,
+                  int q_len, int k_len, int head_dim, int causal) {
+  SA_CHECK_ARG(batch > 0 && heads > 0 && q_len > 0 && k_len > 0, "%s: bad sizes b=%d H=%d Lq=%d Lk=%d",
+               what, batch, heads, q_len, k_len);
+  SA_CHECK_ARG(!causal || q_len == k_len, "%s: causal needs q_len == k_len", what);
+  SA_CHECK_ARG(dtype == sa::kBF16 || dtype == sa::kF32, "%s: unsupported dtype %d", what, dtype);
+  SA_CHECK_ARG(head_dim == 32 || head_dim == 64 || head_dim == 96 || head_dim == 128,
+               "%s: head_dim %d not supported (32, 64, 96, 128)", what, head_dim);
+  SA_CHECK_ARG(q && k && ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k)) & 15) == 0,
+               "%s: q and k must be non-null and 16-byte aligned", what);
+  SA_CHECK_ARG(static_cast<int64_t>(batch) * heads * ((max(q_len, k_len) + sa::kRows - 1) / sa::kRows) <
+                   (1LL << 31), "%s: too many blocks", what);
+  return 0;
+}
+}  // namespace
+
+extern "C" size_t sa_score_moments_workspace_size(int batch, int heads, int q_len, int k_len,
+                                                  int head_dim) {
+  if (batch <= 0 || heads <= 0 || q_len <= 0 || k_len <= 0 || head_dim <= 0) return 0;
+  const size_t nc = (static_cast<size_t>(max(q_len, k_len)) + sa::kChunk - 1) / sa::kChunk;
+  return moments_part(batch, heads, q_len) * sizeof(double) +
+         static_cast<size_t>(batch) * heads * nc * (head_dim * head_dim + head_dim) * sizeof(float);
+}
+
+#define SA_MOMENTS_CASE(DD, FN, ...)                        case DD:                                                    return dtype == sa::kBF16 ? sa::FN<sa::bf16, DD>(__VA_ARGS__) : sa::FN<float, DD>(__VA_ARGS__)
+#define SA_MOMENTS_DISPATCH(FN, ...)         switch (head_dim) {                          SA_MOMENTS_CASE(32, FN, __VA_ARGS__);      SA_MOMENTS_CASE(64, FN, __VA_ARGS__);      SA_MOMENTS_CASE(96, FN, __VA_ARGS__);      SA_MOMENTS_CASE(128, FN, __VA_ARGS__);     default: return 1;                       }
+
+extern "C" int sa_score_moments(int dtype, const void* q, const void* k, const int64_t* q_length,
+                                const int64_t* k_length, int batch, int heads, int q_len, int k_len,
+                                int head_dim, int causal, float scale, void* workspace,
+                                size_t workspace_bytes, double* out, float* std, void* stream) {
+  if (check_moments("sa_score_moments", dtype, q, k, batch, heads, q_len, k_len, head_dim, causal))
+    return 1;
+  SA_CHECK_ARG(out, "sa_score_moments: null tensor pointer");
+  const size_t need = sa_score_moments_workspace_size(batch, heads, q_len, k_len, head_dim);
+  SA_CHECK_ARG(workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && workspace_bytes >= need,
+               "sa_score_moments: 16-byte aligned workspace of %zu B needed, %zu B given", need,
+               workspace_bytes);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  double* part = static_cast<double*>(workspace);
+  float* gram = reinterpret_cast<float*>(part + moments_part(batch, heads, q_len));
+  SA_MOMENTS_DISPATCH(launch_moments, q, k, q_length, k_length, batch, heads, q_len, k_len, causal,
+                      scale, part, gram, out, std, s)
+}
+
+extern "C" int sa_score_std_bwd(int dtype, const void* q, const void* k, const int64_t* q_length,
+                                const int64_t* k_length, int batch, int heads, int q_len, int k_len,
+                                int head_dim, int causal, float scale, const double* stats,
+                                const float* std_grad, void* dq, void* dk, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  if (check_moments("sa_score_std_bwd", dtype, q, k, batch, heads, q_len, k_len, head_dim, causal))
+    return 1;
+  SA_CHECK_ARG(stats && std_grad && dq && dk &&
+                   ((reinterpret_cast<uintptr_t>(dq) | reinterpret_cast<uintptr_t>(dk)) & 15) == 0,
+               "sa_score_std_bwd: tensor pointers must be non-null, dq and dk 16-byte aligned");
+  const size_t need = sa_score_moments_workspace_size(batch, heads, q_len, k_len, head_dim);
+  SA_CHECK_ARG(workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && workspace_bytes >= need,
+               "sa_score_std_bwd: 16-byte aligned workspace of %zu B needed, %zu B given", need,
+               workspace_bytes);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  float* gram = reinterpret_cast<float*>(static_cast<double*>(workspace) +
+                                         moments_part(batch, heads, q_len));
+  SA_MOMENTS_DISPATCH(launch_std_bwd, q, k, q_length, k_length, batch, heads, q_len, k_len, causal,
+                      scale, stats, std_grad, gram, dq, dk, s)
 }

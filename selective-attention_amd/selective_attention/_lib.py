@@ -52,6 +52,11 @@ SIGNATURES: dict[str, list] = {
     "sa_silu_mul_bf16": [_vp, _vp, _i64, _vp, _vp],
     "sa_score_stats_workspace_size": [_i, _i, _i],
     "sa_score_stats": [_i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp, _sz, _vp, _vp],
+    "sa_score_moments_workspace_size": [_i, _i, _i, _i, _i],
+    "sa_score_moments": [_i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp, _sz, _vp, _vp,
+                         _vp],
+    "sa_score_std_bwd": [_i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp, _vp, _vp, _vp,
+                         _vp, _sz, _vp],
     "sa_gated_attn_train_fwd": [_vp, _vp, _vp, _vp, ctypes.POINTER(_i64), _i, _i, _i, _i, _i, _f,
                                 _vp, _vp, _vp, _vp],
     "sa_gated_attn_train_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.POINTER(_i64), _i,
@@ -82,7 +87,8 @@ RESTYPES = {"sa_last_error": ctypes.c_char_p, "sa_profile_enable": None, "sa_ssd
             "sa_paged_decode_noalloc_limit": ctypes.c_size_t,
             "sa_ssm_conv_bwd_workspace_size": ctypes.c_size_t,
             "sa_ssm_gate_bwd_workspace_size": ctypes.c_size_t,
-            "sa_score_stats_workspace_size": ctypes.c_size_t}
+            "sa_score_stats_workspace_size": ctypes.c_size_t,
+            "sa_score_moments_workspace_size": ctypes.c_size_t}
 
 DTYPE_F32 = 0
 DTYPE_BF16 = 1

@@ -188,6 +188,54 @@ def score_stats(q, k, q_lengths=None, k_lengths=None, causal=True, softmax_scale
     return out
 
 
+def score_moments(q, k, q_lengths=None, k_lengths=None, causal=True):
+    """score_stats at softmax_scale head_dim^-0.5 through Gram matrices of the
+    keys (no pass over every pair), with the std it gives: returns (stats
+    (heads, 3) float64, std (heads,) float32)."""
+    from .common import act_dtype_code
+    if (q.dim() != 4 or k.dim() != 4 or q.shape[:2] != k.shape[:2] or q.shape[3] != k.shape[3]
+            or q.dtype != k.dtype or (causal and q.shape[2] != k.shape[2])
+            or q.numel() == 0 or k.numel() == 0):
+        stats = score_stats(q, k, q_lengths, k_lengths, causal)     # refused, or no pairs
+        return stats, torch.zeros(stats.shape[0], dtype=torch.float32, device=q.device)
+    require_device(q, k, q_lengths, k_lengths)
+    b, H, Lq, D = q.shape
+    Lk = k.shape[2]
+    code = act_dtype_code(q.dtype)
+    q, k = q.contiguous(), k.contiguous()
+    ql = None if q_lengths is None else q_lengths.to(torch.int64).contiguous()
+    kl = None if k_lengths is None else k_lengths.to(torch.int64).contiguous()
+    stats = torch.empty((H, 3), dtype=torch.float64, device=q.device)
+    std = torch.empty((H,), dtype=torch.float32, device=q.device)
+    nbytes = _lib.load().sa_score_moments_workspace_size(b, H, Lq, Lk, D)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=q.device)
+    _lib.call("sa_score_moments", code, _lib.ptr(q), _lib.ptr(k), _lib.ptr(ql), _lib.ptr(kl), b, H,
+              Lq, Lk, D, 1 if causal else 0, D ** -0.5, _lib.ptr(ws), nbytes, _lib.ptr(stats),
+              _lib.ptr(std), _lib.stream_of(q))
+    return stats, std
+
+
+def score_std_backward(q, k, q_lengths, k_lengths, causal, stats, std_grad):
+    """(dq, dk) of the std of score_moments for its upstream gradient (heads,)."""
+    from .common import act_dtype_code
+    require_device(q, k, q_lengths, k_lengths, stats, std_grad)
+    b, H, Lq, D = q.shape
+    Lk = k.shape[2]
+    q, k = q.contiguous(), k.contiguous()
+    dq, dk = torch.empty_like(q), torch.empty_like(k)
+    if min(b, H, Lq, Lk) == 0:
+        return dq.zero_(), dk.zero_()
+    ql = None if q_lengths is None else q_lengths.to(torch.int64).contiguous()
+    kl = None if k_lengths is None else k_lengths.to(torch.int64).contiguous()
+    g = std_grad.to(torch.float32).contiguous()
+    nbytes = _lib.load().sa_score_moments_workspace_size(b, H, Lq, Lk, D)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=q.device)
+    _lib.call("sa_score_std_bwd", act_dtype_code(q.dtype), _lib.ptr(q), _lib.ptr(k), _lib.ptr(ql),
+              _lib.ptr(kl), b, H, Lq, Lk, D, 1 if causal else 0, D ** -0.5, _lib.ptr(stats),
+              _lib.ptr(g), _lib.ptr(dq), _lib.ptr(dk), _lib.ptr(ws), nbytes, _lib.stream_of(q))
+    return dq, dk
+
+
 TRAIN_HEAD_DIMS = (32, 64, 96, 128)
 
 

@@ -22,10 +22,10 @@ ops:
   removes pages whose keys every head has dropped, without moving data.
 
 * ScoreStdFn: the per-head std of the valid scores that SelectiveMHA's
-  training forward scales the log-gate by (:234-247).  Its forward is the
-  in-kernel reduction score_stats (count, sum, sum of squares, no score
-  matrix); its backward carries d std_h / d s_ij = (s_ij - mean_h) /
-  (count_h std_h) to q and k by query chunks.
+  training forward scales the log-gate by (:234-247), from the count, sum and
+  sum of squares that Gram matrices of the keys give (score_moments); its
+  backward carries d std_h / d s_ij = (s_ij - mean_h) / (count_h std_h) to q
+  and k the same way.
 * gated_attention_train: the training attention itself, the reference's gated
   softmax, forward and backward in fp32 kernels without a score matrix.
 * cross_attention_train: the cross-attention's, dense under autograd, in fp32.
@@ -35,7 +35,7 @@ from __future__ import annotations
 import torch
 
 from ..kernels.attention import (TRAIN_HEAD_DIMS, gated_attn_train_backward,
-                                 gated_attn_train_forward, score_stats)
+                                 gated_attn_train_forward, score_moments, score_std_backward)
 from ..kernels.lm_ops import paged_kv_append, paged_kv_build
 from .attention import attn_varlen, paged_decode_attn
 
@@ -69,35 +69,43 @@ class ScoreStdFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, q_lengths=None, k_lengths=None, causal=True, chunk=256):
-        st = score_stats(q, k, q_lengths, k_lengths, causal)
-        cnt = st[:, 0].clamp(min=1)
-        mean = st[:, 1] / cnt
-        std = (st[:, 2] / cnt - mean * mean).clamp(min=0).sqrt()
-        ctx.save_for_backward(q, k, mean, std, cnt)
+        stats, std = score_moments(q, k, q_lengths, k_lengths, causal)
+        ctx.save_for_backward(q, k, stats)
         ctx.q_lengths, ctx.k_lengths, ctx.causal, ctx.chunk = q_lengths, k_lengths, causal, chunk
-        return std.to(torch.float32)
+        return std
 
     @staticmethod
     def backward(ctx, g):
-        q, k, mean, std, cnt = ctx.saved_tensors
-        Lq, D = q.shape[2], q.shape[3]
-        Lk = k.shape[2]
-        scale = D ** -0.5
-        coef = torch.where(std > 0, g.double() / (cnt * std.clamp(min=1e-300)),
-                           torch.zeros_like(std)).float()[None, :, None, None]
-        mu = mean.float()[None, :, None, None]
-        kf = k.float()
-        dq = torch.zeros(q.shape, dtype=torch.float32, device=q.device)
-        dk = torch.zeros(k.shape, dtype=torch.float32, device=k.device)
-        for i0 in range(0, Lq, ctx.chunk):
-            i1 = min(Lq, i0 + ctx.chunk)
-            qc = q[:, :, i0:i1].float()
-            s = torch.matmul(qc, kf.transpose(-2, -1).contiguous()) * scale
-            valid = _valid_pairs(Lk, ctx.q_lengths, ctx.k_lengths, ctx.causal, i0, i1, q.device)
-            gs = torch.where(valid, (s - mu) * coef, torch.zeros((), device=q.device))
-            dq[:, :, i0:i1] = torch.matmul(gs, kf) * scale
-            dk += torch.matmul(gs.transpose(-2, -1).contiguous(), qc) * scale
-        return dq.to(q.dtype), dk.to(k.dtype), None, None, None, None
+        q, k, stats = ctx.saved_tensors
+        if torch.is_grad_enabled():      # a recorded backward: torch ops by query chunks
+            dq, dk = _score_std_backward_dense(q, k, stats, g, ctx)
+        else:
+            dq, dk = score_std_backward(q, k, ctx.q_lengths, ctx.k_lengths, ctx.causal, stats, g)
+        return dq, dk, None, None, None, None
+
+
+def _score_std_backward_dense(q, k, stats, g, ctx):
+    cnt = stats[:, 0].clamp(min=1)
+    mean = stats[:, 1] / cnt
+    std = (stats[:, 2] / cnt - mean * mean).clamp(min=0).sqrt()
+    Lq, D = q.shape[2], q.shape[3]
+    Lk = k.shape[2]
+    scale = D ** -0.5
+    coef = torch.where(std > 0, g.double() / (cnt * std.clamp(min=1e-300)),
+                       torch.zeros_like(std)).float()[None, :, None, None]
+    mu = mean.float()[None, :, None, None]
+    kf = k.float()
+    dq, dk = [], torch.zeros(k.shape, dtype=torch.float32, device=k.device)
+    for i0 in range(0, Lq, ctx.chunk):
+        i1 = min(Lq, i0 + ctx.chunk)
+        qc = q[:, :, i0:i1].float()
+        s = torch.matmul(qc, kf.transpose(-2, -1).contiguous()) * scale
+        valid = _valid_pairs(Lk, ctx.q_lengths, ctx.k_lengths, ctx.causal, i0, i1, q.device)
+        gs = torch.where(valid, (s - mu) * coef, torch.zeros((), device=q.device))
+        dq.append(torch.matmul(gs, kf) * scale)
+        dk = dk + torch.matmul(gs.transpose(-2, -1).contiguous(), qc) * scale
+    dq = torch.cat(dq, dim=2) if dq else torch.zeros(q.shape, device=q.device)
+    return dq.to(q.dtype), dk.to(k.dtype)
 
 
 def _gated_attention_dense(q, k, v, log_gate, causal):

@@ -110,6 +110,50 @@ def test_second_derivative_matches_dense():
         assert float((a.double() - e).norm() / e.norm()) < 1e-4
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,b,H,Lq,Lk,D,causal,ql,kl", [
+    (torch.float32, 2, 2, 1, 1, 64, True, None, None),
+    (torch.float32, 2, 3, 255, 255, 64, True, [255, 130], [255, 130]),
+    (torch.float32, 1, 2, 257, 257, 128, True, None, None),
+    (torch.bfloat16, 3, 2, 600, 600, 64, True, [600, 256, 0], [600, 256, 0]),
+    (torch.float32, 2, 2, 2500, 2500, 32, True, [2500, 1030], [2400, 1100]),
+    (torch.bfloat16, 2, 2, 70, 300, 96, False, None, [300, 17]),
+    (torch.float32, 1, 3, 530, 65, 64, False, [400], [65]),
+])
+def test_score_std_through_gram_matrices(dtype, b, H, Lq, Lk, D, causal, ql, kl):
+    """Counts exact; std and its gradient against the fp64 oracle at the edges of
+    the 64-row tiles and 256-row chunks.  fp32 sums of at most 2500 rows:
+    2500^0.5 * 2^-24 = 3e-6 relative on a Gram entry, 1e-5 with the products."""
+    from oracle import attn as ref
+    g = torch.Generator().manual_seed(Lq)
+    q = (torch.randn(b, H, Lq, D, generator=g) + 0.2).to(dtype)
+    k = (torch.randn(b, H, Lk, D, generator=g) + 0.1).to(dtype)
+    go = torch.randn(H, generator=g)
+    lens = [None if x is None else torch.tensor(x) for x in (ql, kl)]
+    dev = [None if x is None else x.cuda() for x in lens]
+    qd, kd = q.cuda().requires_grad_(True), k.cuda().requires_grad_(True)
+    std = M.ScoreStdFn.apply(qd, kd, *dev, causal)
+    stats, _ = M.score_moments(qd.detach(), kd.detach(), *dev, causal)
+    got = torch.autograd.grad(std, (qd, kd), go.cuda(), retain_graph=True)
+    q64, k64 = q.double().requires_grad_(True), k.double().requires_grad_(True)
+    want_stats = ref.score_stats(q64, k64, D ** -0.5, *lens, causal)
+    want = ref.score_std(want_stats)
+    assert torch.equal(stats[:, 0].cpu(), want_stats[:, 0].detach())
+    torch.testing.assert_close(std.detach().cpu().double(), want.detach(), rtol=1e-5, atol=1e-6)
+    wg = torch.autograd.grad(want, (q64, k64), go.double())
+    rel = 1e-5 if dtype == torch.float32 else 2 ** -8
+    if float(want.detach().min()) > 1e-3:      # (a single pair has std 0: no gradient)
+        for a, e in zip(got, wg):
+            assert float((a.double().cpu() - e).norm() / e.norm()) < rel
+    else:
+        assert all(float(a.abs().max()) < 1e-3 for a in got)
+    # a recorded backward takes the torch form: the same gradients
+    rec = torch.autograd.grad(std, (qd, kd), go.cuda(), create_graph=True)
+    for a, e in zip(got, rec):
+        assert rec[0].requires_grad
+        torch.testing.assert_close(a.float(), e.detach().float(), rtol=2 * rel, atol=1e-6)
+
+
 def test_dense_form_on_the_cpu():
     q, k, v, lg, do = inputs(1, 2, 20, 64, device="cpu", seed=6)
     assert not M._train_kernel_ok(q, k, v, lg)
