@@ -335,10 +335,11 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 // inclusive prefix sum across the 64 lanes of a wave
-__device__ __forceinline__ float wave_incl_scan(float v, int lane) {
+template <typename F>
+__device__ __forceinline__ F wave_incl_scan(F v, int lane) {
 #pragma unroll
   for (int o = 1; o < 64; o <<= 1) {
-    float t = __shfl_up(v, o, 64);
+    const F t = __shfl_up(v, o, 64);
     if (lane >= o) v += t;
   }
   return v;

@@ -1,5 +1,5 @@
-// 64-row fp32 tiles on v_mfma_f32_16x16x4_f32, shared by the training
-// attention and the score statistics: a row-major LDS tile of row length
+// fp32 tiles on v_mfma_f32_16x16x4_f32, shared by the training attention, the
+// score statistics and the fp32 SSD scan: a row-major LDS tile of row length
 // D + 4 floats serves both as the row operand of a score product (16-byte
 // reads) and, transposed, as the weighted sum of its rows (dword reads); both
 // are free of bank conflicts at that row length.
@@ -24,26 +24,26 @@ __device__ __forceinline__ void store4(bf16* p, const v4f& v) {
   *reinterpret_cast<uint2*>(p) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
 }
 
-// tile rows r0 .. r0 + 63 of x (row stride ld elements), zero past L, as
-// D / 16 float4 per thread
-template <int D>
+// tile rows r0 .. r0 + R - 1 of x (row stride ld elements), zero at and past
+// row L, as R D / 1024 float4 per thread of a 256-thread block
+template <int D, int R = kRows>
 struct TileRegs {
-  float4 r[D / 16];
+  float4 r[R * D / 1024];
 };
-template <int D, typename T>
-__device__ __forceinline__ void tile_load(TileRegs<D>& t, const T* x, long ld, int r0, int L,
+template <int D, int R, typename T>
+__device__ __forceinline__ void tile_load(TileRegs<D, R>& t, const T* x, long ld, int r0, int L,
                                           int tid) {
 #pragma unroll
-  for (int p = 0; p < D / 16; ++p) {
+  for (int p = 0; p < R * D / 1024; ++p) {
     const int idx = tid + 256 * p, row = idx / (D / 4), c = 4 * (idx % (D / 4));
     const int g = r0 + row;
     t.r[p] = g < L ? load4_f32(x + g * ld + c) : float4{0.f, 0.f, 0.f, 0.f};
   }
 }
-template <int D>
-__device__ __forceinline__ void tile_store(const TileRegs<D>& t, float* lds, int tid) {
+template <int D, int R>
+__device__ __forceinline__ void tile_store(const TileRegs<D, R>& t, float* lds, int tid) {
 #pragma unroll
-  for (int p = 0; p < D / 16; ++p) {
+  for (int p = 0; p < R * D / 1024; ++p) {
     const int idx = tid + 256 * p, row = idx / (D / 4), c = 4 * (idx % (D / 4));
     *reinterpret_cast<float4*>(lds + row * (D + 4) + c) = t.r[p];
   }
@@ -64,32 +64,43 @@ __device__ __forceinline__ v4f mfma_f32(float a, float b, const v4f& c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// acc[t] (rows 16 t + 4 g + i of the LDS tile, column li) = tile . f^T
-template <int D>
-__device__ __forceinline__ void score_tile(v4f (&acc)[4], const float* lds, const v4f (&f)[D / 16],
-                                           int li, int lg) {
+template <int N>
+__device__ __forceinline__ void zero_frag(v4f (&f)[N]) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int i = 0; i < N; ++i) f[i] = v4f{0.f, 0.f, 0.f, 0.f};
+}
+
+// acc[t] (rows 16 t + 4 g + i of the LDS tile, column li) += tile . f^T over
+// the first 16 NT rows
+template <int D, int NT>
+__device__ __forceinline__ void score_add(v4f (&acc)[NT], const float* lds, const v4f (&f)[D / 16],
+                                          int li, int lg) {
 #pragma unroll
   for (int s = 0; s < D / 16; ++s) {
-    v4f a[4];
+    v4f a[NT];
 #pragma unroll
-    for (int t = 0; t < 4; ++t)
+    for (int t = 0; t < NT; ++t)
       a[t] = *reinterpret_cast<const v4f*>(lds + (16 * t + li) * (D + 4) + 16 * s + 4 * lg);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int t = 0; t < 4; ++t) acc[t] = mfma_f32(a[t][i], f[s][i], acc[t]);
+      for (int t = 0; t < NT; ++t) acc[t] = mfma_f32(a[t][i], f[s][i], acc[t]);
   }
+}
+template <int D, int NT>
+__device__ __forceinline__ void score_tile(v4f (&acc)[NT], const float* lds, const v4f (&f)[D / 16],
+                                           int li, int lg) {
+  zero_frag(acc);
+  score_add<D>(acc, lds, f, li, lg);
 }
 
 // out[dt] (d = 16 dt + 4 g + i, column li) += tile^T . w, w[t][i] the weight
 // of tile row 16 t + 4 g + i
-template <int D>
-__device__ __forceinline__ void weigh_tile(v4f (&out)[D / 16], const float* lds, const v4f (&w)[4],
+template <int D, int NT>
+__device__ __forceinline__ void weigh_tile(v4f (&out)[D / 16], const float* lds, const v4f (&w)[NT],
                                            int li, int lg) {
 #pragma unroll
-  for (int t = 0; t < 4; ++t)
+  for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float* row = lds + (16 * t + 4 * lg + i) * (D + 4) + li;

@@ -62,8 +62,9 @@ __device__ __forceinline__ void frag_col_sums(const float (&v)[2][2][4], float (
 struct BwdWs {
   size_t dS, dCB, ddt_part, xB_part, xC_part, rsum, qpart, ddc_part, dA_part, db_part;
   size_t dyp, dSp, dcbp, total;   // bf16 planes of the fused path
+  size_t f32_cb, f32_dCB, f32_part;   // fp32 tile path
   int ptiles, ntiles, ttiles, per_bh;
-  bool fused;
+  bool fused, f32;
 };
 
 inline size_t al256(size_t x) { return (x + 255) & ~static_cast<size_t>(255); }
@@ -92,6 +93,16 @@ inline BwdWs bwd_layout(const SsdDims& d, size_t mt_bytes) {
   w.dyp = o;       o = al256(o + (w.fused ? bhc * d.Lc * 64 * 2 * 2 : 0));
   w.dSp = o;       o = al256(o + (w.fused ? bhc * PN * 2 * 2 : 0));
   w.dcbp = o;      o = al256(o + (w.fused ? bncg * w.ttiles * w.ttiles * 2 * 64 * 64 * 2 : 0));
+  // the fp32 tile path: C B^T, dCB per share of the heads, dB / dC per share
+  w.f32 = mt_bytes == 4 && ssd_f32_shape_ok(d);
+  if (w.f32) {
+    const size_t cb = bncg * d.Lc * d.Lc * 4;
+    const int bs = ssd_f32_dbdc_shares(d);
+    w.f32_cb = region;
+    w.f32_dCB = al256(w.f32_cb + cb);
+    w.f32_part = al256(w.f32_dCB + cb * ssd_f32_dcb_shares(d));
+    o = al256(w.f32_part + (bs > 1 ? static_cast<size_t>(bs) * 2 * d.b * d.L * d.G * d.N * 4 : 0));
+  }
   if (o < generic_end) o = generic_end;
   w.ddt_part = o;  o = al256(o + bhc * w.ptiles * d.Lc * 4);
   w.xB_part = o;   o = al256(o + bhc * w.ntiles * d.Lc * 4);
@@ -689,10 +700,11 @@ __global__ __launch_bounds__(256) void chunk_dbdc_bwd_kernel(
 // exclusive prefix and writes the block total to *total
 // exclusive prefix sums of three values at once (one pair of barriers);
 // wt3 holds 4 waves x 3 floats
-__device__ __forceinline__ void block_excl_scan3(const float (&v)[3], float* wt3, float (&base)[3],
-                                                 float (&tot)[3]) {
+template <typename F>
+__device__ __forceinline__ void block_excl_scan3(const F (&v)[3], F* wt3, F (&base)[3],
+                                                 F (&tot)[3]) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  float incl[3];
+  F incl[3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     incl[i] = wave_incl_scan(v[i], lane);
@@ -702,7 +714,7 @@ __device__ __forceinline__ void block_excl_scan3(const float (&v)[3], float* wt3
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     base[i] = incl[i] - v[i];
-    tot[i] = 0.f;
+    tot[i] = 0;
     for (int w = 0; w < 4; ++w) {
       if (w < wid) base[i] += wt3[w * 3 + i];
       tot[i] += wt3[w * 3 + i];
@@ -712,7 +724,8 @@ __device__ __forceinline__ void block_excl_scan3(const float (&v)[3], float* wt3
 }
 
 // block sums of two values at once
-__device__ __forceinline__ void block_sum2(float& a, float& b, float* wt3) {
+template <typename F>
+__device__ __forceinline__ void block_sum2(F& a, F& b, F* wt3) {
   a = wave_sum(a);
   b = wave_sum(b);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -726,12 +739,13 @@ __device__ __forceinline__ void block_sum2(float& a, float& b, float* wt3) {
   __syncthreads();
 }
 
-__device__ __forceinline__ float block_sum(float v, float* wtot) {
+template <typename F>
+__device__ __forceinline__ F block_sum(F v, F* wtot) {
   v = wave_sum(v);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane == 0) wtot[wid] = v;
   __syncthreads();
-  const float s = wtot[0] + wtot[1] + wtot[2] + wtot[3];
+  const F s = wtot[0] + wtot[1] + wtot[2] + wtot[3];
   __syncthreads();
   return s;
 }
@@ -762,8 +776,9 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(
     const float* __restrict__ rsum, const float* __restrict__ qpart,
     const float* __restrict__ ddc_part, T* __restrict__ ddelta_raw, float* __restrict__ dA_part,
     float* __restrict__ db_part, SsdDims d, int ptiles, int ntiles, int xctiles, int ttiles,
-    int rtiles, int per_bh, int has_init, int softplus, float lo, float hi) {
-  __shared__ float wtot[4 * 3];
+    int rtiles, int per_bh, int has_init, int softplus, float lo, float hi, int qlower) {
+  typedef typename CumsumAcc<T>::type Acc;
+  __shared__ Acc wtot[4 * 3];
   const int h = blockIdx.x % d.H;
   const int c = (blockIdx.x / d.H) % d.nc;
   const int b = blockIdx.x / (d.H * d.nc);
@@ -776,16 +791,19 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(
 
   // every global load is issued here, ahead of the block reductions (a
   // barrier orders memory, so loads placed after one wait for it)
-  float ddc = 0.f;
+  Acc ddc = 0;
   for (int k = threadIdx.x; k < per_bh; k += 256) ddc += ddc_part[bhc * per_bh + k];
   // loads from clamped (valid) positions, unconditionally, so that they are
   // all in flight together; positions past Lc, qlim or lim are masked after
-  float qr[PER], xb[PER], xc[PER], zv[PER], dtv[PER], ddtd[PER];
+  float qr[PER], xb[PER], zv[PER], dtv[PER], ddtd[PER];
+  Acc xc[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int t = tb + j;
     const int tl = min(t, d.Lc - 1), tq = min(t, qlim - 1);
-    const float q = sum_parts<4>(qpart + bhc * ttiles * d.Lc + tl, d.Lc, ttiles);
+    // column sums: partials of the row tiles k >= t / 64 (qlower), or of every one
+    const int q0 = qlower ? tl / 64 : 0;
+    const float q = sum_parts<4>(qpart + (bhc * ttiles + q0) * d.Lc + tl, d.Lc, ttiles - q0);
     const float x1 = sum_parts<2>(xB_part + bhc * ntiles * d.Lc + tl, d.Lc, ntiles);
     const float x2 = sum_parts<2>(xC_part + bhc * xctiles * d.Lc + tl, d.Lc, xctiles);
     // row sums: partials of the source tiles k <= t / 64 (rtiles == 1: complete)
@@ -804,8 +822,8 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(
   }
   // ddc_last of this chunk (sum of the state-passing partials)
   ddc = block_sum(ddc, wtot);
-  if (!has_init && c == 0) ddc = 0.f;
-  float sqr = 0.f, sxb = 0.f, sxc = 0.f;
+  if (!has_init && c == 0) ddc = 0;
+  Acc sqr = 0, sxb = 0, sxc = 0;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     if (tb + j == d.Lc - 1) xc[j] += ddc;
@@ -813,18 +831,18 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(
     sxb += xb[j];
     sxc += xc[j];
   }
-  float ex[3], tt[3];
-  block_excl_scan3({sqr, sxb, sxc}, wtot, ex, tt);
-  const float eq = ex[0], eb = ex[1], ec = ex[2], tc = tt[2];
+  Acc ex[3], tt[3];
+  block_excl_scan3<Acc>({sqr, sxb, sxc}, wtot, ex, tt);
+  const Acc eq = ex[0], eb = ex[1], ec = ex[2], tc = tt[2];
   const float a = A[h];
   const float bias = delta_bias ? delta_bias[h] : 0.0f;
-  float rq = eq, rb = eb, rc = ec;
-  float dA_loc = 0.f, db_loc = 0.f;
+  Acc rq = eq, rb = eb, rc = ec;
+  Acc dA_loc = 0, db_loc = 0;
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int t = tb + j;
     if (t < d.Lc) {
-      const float dA_intra = rq, dA_B = rb, dA_C = tc - rc;  // exclusive, exclusive, suffix
+      const Acc dA_intra = rq, dA_B = rb, dA_C = tc - rc;  // exclusive, exclusive, suffix
       rq += qr[j];
       rb += xb[j];
       rc += xc[j];
@@ -832,10 +850,10 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(
         const long off = (static_cast<long>(b) * d.L + static_cast<long>(c) * d.Lc + t) * d.H + h;
         float g = 0.f;
         if (t < lim) {
-          const float da = dA_intra + dA_B + dA_C;
+          const Acc da = dA_intra + dA_B + dA_C;
           const float z = zv[j] + bias;
           const float sp = softplus ? softplus20(z) : z;
-          g = da * a + ddtd[j];
+          g = static_cast<float>(da * a + ddtd[j]);
           if (sp < lo || sp > hi) g = 0.f;
           if (softplus && z <= 20.0f) g *= sigmoidf_acc(z);
           dA_loc += da * dtv[j];
@@ -847,19 +865,20 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(
   }
   block_sum2(dA_loc, db_loc, wtot);
   if (threadIdx.x == 0) {
-    dA_part[(static_cast<long>(b) * d.nc + c) * d.H + h] = dA_loc;
-    db_part[(static_cast<long>(b) * d.nc + c) * d.H + h] = db_loc;
+    dA_part[(static_cast<long>(b) * d.nc + c) * d.H + h] = static_cast<float>(dA_loc);
+    db_part[(static_cast<long>(b) * d.nc + c) * d.H + h] = static_cast<float>(db_loc);
   }
 }
 
+template <typename Acc>
 __global__ __launch_bounds__(256) void param_grad_reduce_kernel(const float* __restrict__ dA_part,
                                                                 const float* __restrict__ db_part,
                                                                 float* __restrict__ dA,
                                                                 float* __restrict__ dbias,
                                                                 int rows, int H) {
-  __shared__ float wtot[4];
+  __shared__ Acc wtot[4];
   const int h = blockIdx.x;
-  float s1 = 0.f, s2 = 0.f;
+  Acc s1 = 0, s2 = 0;
   for (int r = threadIdx.x; r < rows; r += 256) {
     s1 += dA_part[static_cast<long>(r) * H + h];
     s2 += db_part[static_cast<long>(r) * H + h];
@@ -867,8 +886,8 @@ __global__ __launch_bounds__(256) void param_grad_reduce_kernel(const float* __r
   s1 = block_sum(s1, wtot);
   s2 = block_sum(s2, wtot);
   if (threadIdx.x == 0) {
-    dA[h] = s1;
-    if (dbias) dbias[h] = s2;
+    dA[h] = static_cast<float>(s1);
+    if (dbias) dbias[h] = static_cast<float>(s2);
   }
 }
 
@@ -931,12 +950,18 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
   int rc;
 
   const bool fused = sizeof(T) == 2 && w.fused && ssd_bwd_fused_ok(d, u, Bm, Cm, dy);
+  const bool f32 = w.f32 && aligned16(u) && aligned16(Bm) && aligned16(Cm) && aligned16(dy) &&
+                   aligned16(states) && aligned16(du_) && aligned16(dB_) && aligned16(dC_) &&
+                   aligned16(dt) && aligned16(dc) && aligned16(ws);
   bf16* dyp = reinterpret_cast<bf16*>(ws + w.dyp);
   bf16* dSp = reinterpret_cast<bf16*>(ws + w.dSp);
   bf16* dcbp = reinterpret_cast<bf16*>(ws + w.dcbp);
   // 1. dH_intra -> dS buffer (the fused path also writes dy as hi + lo planes)
   if (fused) {
     if ((rc = launch_dstate_planes(dy, C_, dt, dc, length, dS, dyp, d, s))) return rc;
+  } else if (f32) {
+    if ((rc = launch_f32_outer(dy, static_cast<const float*>(C_), dt, dc, length, dS, d, 1, s)))
+      return rc;
   } else {
     if ((rc = launch_chunk_outer<MT, float, T, 1>(dy, C_, dt, dc, length, dS, d, s))) return rc;
   }
@@ -957,6 +982,19 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
       return rc;
     ptiles = ntiles = qtiles = 1;
     xctiles = d.N / 64;   // x_C: one partial per 64 n (ssd_bwd_tgt block)
+    rtiles = d.Lc / 64;
+  } else if (f32) {
+    // 3-5 in fp32 on 64-row tiles (ssd_f32.hip)
+    const SsdF32Ws fw{reinterpret_cast<float*>(ws + w.f32_cb), reinterpret_cast<float*>(ws + w.f32_dCB),
+                      reinterpret_cast<float*>(ws + w.f32_part), rsum, qpart, ddt_part, xB_part,
+                      xC_part};
+    if ((rc = launch_f32_bwd(reinterpret_cast<const float*>(u_), reinterpret_cast<const float*>(B_),
+                             reinterpret_cast<const float*>(C_), dy, dt, dc, states, dS, length,
+                             static_cast<float*>(du_), static_cast<float*>(dB_),
+                             static_cast<float*>(dC_), fw, d, s)))
+      return rc;
+    ptiles = d.P == 32 ? 1 : d.P / 64;
+    ntiles = xctiles = 1;
     rtiles = d.Lc / 64;
   } else {
   // 3. du, ddt_direct
@@ -1002,13 +1040,13 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s,
                        static_cast<const T*>(delta_raw_), A, bias, length, dt, ddt_part, xB_part,
                        xC_part, rsum, qpart, ddc_part, static_cast<T*>(ddelta_), dA_part, db_part,
-                       d, ptiles, ntiles, xctiles, qtiles, rtiles, w.per_bh, has_init, sp, lo, hi);
+                       d, ptiles, ntiles, xctiles, qtiles, rtiles, w.per_bh, has_init, sp, lo, hi, f32 ? 1 : 0);
     SA_CHECK_LAUNCH("chunk_cumsum_bwd");
   }
   // 7. dA, dbias
   {
     ProfScope prof_("param_grad_reduce", s);
-    hipLaunchKernelGGL(param_grad_reduce_kernel, dim3(d.H), dim3(256), 0, s, dA_part, db_part, dA,
+    hipLaunchKernelGGL((param_grad_reduce_kernel<typename CumsumAcc<T>::type>), dim3(d.H), dim3(256), 0, s, dA_part, db_part, dA,
                        dbias, static_cast<int>(bnc), d.H);
     SA_CHECK_LAUNCH("param_grad_reduce");
   }

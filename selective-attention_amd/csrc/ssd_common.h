@@ -22,6 +22,12 @@ __device__ __forceinline__ int chunk_limit(int len, int c, int Lc) {
   return min(Lc, len - c * Lc);
 }
 
+// Running sums of the chunk cumsum kernels: fp64 for fp32 activations, where
+// the roundings of an fp32 sum (dc reaches 1e2 within a chunk) would be the
+// largest error of every decay; fp32 beside bf16 activations' own rounding.
+template <typename T> struct CumsumAcc { typedef double type; };
+template <> struct CumsumAcc<bf16> { typedef float type; };
+
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
 // ---------------------------------------------------------------------------
@@ -122,6 +128,25 @@ int launch_ssd_bwd_fused(const void* u, const void* B, const void* C, const bf16
                          float* ddt_part, float* xB_part, float* xC_part, float* qpart,
                          float* rpart, const SsdDims& d, bool dt_nonneg,
                          hipStream_t s);
+
+// fp32 scan on 64-row tiles (ssd_f32.hip): the shapes it takes, and the shares
+// of a group's heads its dCB and dB / dC launches are split into (each share's
+// sums have their own workspace).  Every tensor pointer 16-byte aligned.
+struct SsdF32Ws {
+  float *cb, *dCB, *part;   // C B^T and dCB (per share) [b][nc][G][Lc][Lc]; dB, dC per share
+  float *rpart, *qpart, *ddt_part, *xB, *xC;
+};
+bool ssd_f32_shape_ok(const SsdDims& d);
+int ssd_f32_dcb_shares(const SsdDims& d);
+int ssd_f32_dbdc_shares(const SsdDims& d);
+int launch_f32_outer(const float* a, const float* x, const float* dt, const float* dc,
+                     const int64_t* length, float* out, const SsdDims& d, int mode, hipStream_t s);
+int launch_f32_scan(const float* u, const float* B, const float* C, const float* dt, const float* dc,
+                    const float* states, float* y, const SsdDims& d, hipStream_t s);
+int launch_f32_bwd(const float* u, const float* B, const float* C, const float* dy, const float* dt,
+                   const float* dc, const float* states, const float* dS, const int64_t* length,
+                   float* du, float* dB, float* dC, const SsdF32Ws& w, const SsdDims& d,
+                   hipStream_t s);
 
 // dH_intra (chunk_outer MODE 1, bf16 dy) that also writes dy as the hi + lo
 // planes of the fused backward

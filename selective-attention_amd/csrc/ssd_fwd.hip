@@ -35,18 +35,19 @@ __global__ __launch_bounds__(256) void chunk_cumsum_kernel(
     const float* __restrict__ delta_bias, const int64_t* __restrict__ length,
     float* __restrict__ dt_out, float* __restrict__ dc_out, SsdDims d, int softplus, float dmin,
     float dmax) {
-  __shared__ float wave_tot[4];
+  typedef typename CumsumAcc<T>::type Acc;
+  __shared__ Acc wave_tot[4];
   const int h = blockIdx.x % d.H;
   const int c = (blockIdx.x / d.H) % d.nc;
   const int b = blockIdx.x / (d.H * d.nc);
   const int len = seq_limit(length, b, d.L);
   const int lim = chunk_limit(len, c, d.Lc);
-  const float a = A[h];
+  const Acc a = A[h];
   const float bias = delta_bias ? delta_bias[h] : 0.0f;
   const int per = (d.Lc + 255) / 256;  // positions per thread (<= 4)
   const int t0 = threadIdx.x * per;
   float v[4];
-  float run = 0.0f;
+  Acc run = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     v[j] = 0.0f;
@@ -57,17 +58,17 @@ __global__ __launch_bounds__(256) void chunk_cumsum_kernel(
       v[j] = make_dt(z, softplus != 0, dmin, dmax);
     }
   }
-  float part[4];
+  Acc part[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    run += v[j] * a;
+    run += static_cast<Acc>(v[j]) * a;
     part[j] = run;
   }
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  float incl = wave_incl_scan(run, lane);
+  Acc incl = wave_incl_scan(run, lane);
   if (lane == 63) wave_tot[wid] = incl;
   __syncthreads();
-  float base = incl - run;
+  Acc base = incl - run;
   for (int w = 0; w < wid; ++w) base += wave_tot[w];
   const long row = ((static_cast<long>(b) * d.H + h) * d.nc + c) * d.Lc;
 #pragma unroll
@@ -75,7 +76,7 @@ __global__ __launch_bounds__(256) void chunk_cumsum_kernel(
     const int tau = t0 + j;
     if (j < per && tau < d.Lc) {
       dt_out[row + tau] = v[j];
-      dc_out[row + tau] = base + part[j];
+      dc_out[row + tau] = static_cast<float>(base + part[j]);
     }
   }
 }
@@ -1427,6 +1428,18 @@ int ssd_fwd_impl(const void* u, const float* A, const void* B, const void* C,
   SA_CHECK_ARG(!go || fast, "sa_ssd_fwd_gated: the fused epilogue needs the bf16 fast path "
                "(state_dim a multiple of 32, <= 256; head_dim a multiple of 8; 16-byte aligned)");
   if ((rc = launch_chunk_cumsum<T>(delta_raw, A, bias, length, dt, dc, d, sp, lo, hi, s))) return rc;
+  if constexpr (sizeof(T) == 4) {
+    // models' sizes in fp32: the 64-row tile kernels (ssd_f32.hip); other sizes
+    // and operands off a 16-byte boundary go on to the general kernels
+    if (ssd_f32_shape_ok(d) && aligned16(u) && aligned16(B) && aligned16(C) && aligned16(states) &&
+        aligned16(y)) {
+      const float *uf = static_cast<const float*>(u), *bf = static_cast<const float*>(B),
+                  *cf = static_cast<const float*>(C);
+      if ((rc = launch_f32_outer(uf, bf, dt, dc, length, states, d, 0, s))) return rc;
+      if ((rc = launch_state_passing_fwd(states, h_init, h_last, dc, d, s))) return rc;
+      return launch_f32_scan(uf, bf, cf, dt, dc, states, y, d, s);
+    }
+  }
   if (sizeof(T) == 2 && chunk_state_pass_ok(d, u, B, h_init, states, h_last)) {
     if ((rc = launch_chunk_state_pass(u, B, dt, dc, h_init, states, h_last, d, s))) return rc;
   } else {
