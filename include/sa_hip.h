@@ -172,6 +172,18 @@ int sa_attn_varlen_fwd(int dtype, int mode, const void* q, const void* k, const 
                        float softmax_scale, void* o, void* stream);
 
 /*
+ * SelectiveMHA's prefill attention over batch rows (modules/selective_attention.py:
+ * 27-144, mode "seq"): mode 0 of sa_attn_varlen_fwd with each row's first
+ * lengths[row] tokens as a sequence (lengths (batch,) int64 or NULL: all of
+ * seq_len); the other rows of o are zeros.
+ *   q, k, v, o: (batch, seq_len, num_heads, head_dim) bf16, head_dim in {64,128}
+ *   log_gate: (batch, num_heads, seq_len) f32 key bias, not applied on j = i
+ */
+int sa_mha_prefill_fwd(int dtype, const void* q, const void* k, const void* v,
+                       const float* log_gate, const int64_t* lengths, int batch, int seq_len,
+                       int num_heads, int head_dim, float softmax_scale, void* o, void* stream);
+
+/*
  * RMSNorm of `rows` rows of `dim` elements (modules/rms_norm.py:33-44):
  * out = x * rsqrt(mean(x^2) + eps) * (1 + weight[row % groups]), fp32
  * arithmetic, out in x's dtype (f32 or bf16); weight (groups, dim) f32.

@@ -18,14 +18,13 @@
 // operand is a single 16-byte read: from LDS for prefill (V transposed on
 // staging) and straight from HBM for decode, whose V pages are stored
 // transposed, (num_pages, Hkv, D, page_size).
+#include "attn_tile.h"
 #include "common.h"
 #include "prof.h"
 #include "tile.h"
 #include "decode.h"
 
 namespace sa {
-
-constexpr float kNegInf = -__builtin_huge_valf();
 
 // Online-softmax update for one block of keys.  s[kt][i]: log2-domain scores
 // of keys 16kt + 4g + i for query column (lane & 15); masked entries are
@@ -79,25 +78,6 @@ struct SparseSmem {
   static constexpr int stage = 2 * tile + 128;      // bf16: K, V, the 64 fp32 key biases
 };
 
-// chunk permutations of row r (16-byte chunks; D = 128: 16 per row, D = 64:
-// 8).  The K tile is read as MFMA A fragments (16 rows key_of_row(kt, 0..15),
-// one chunk per 16-lane group), the V tile by ds_read_b64_tr_b16 (rows
-// 8g + 0..3 and + 4, one chunk pair per group), so each gets its own
-// permutation; both were chosen with the LDS bank-conflict counter
-// (SQ_LDS_BANK_CONFLICT = 0 for these read sets on gfx950).  The V
-// permutation never uses bit 2 of r, so rows r and r + 4 (the two halves of
-// one transpose read) share it.
-template <int D>
-__device__ __forceinline__ int k_swz(int r) {
-  if constexpr (D == 128) return (r & 3) | (((r >> 3) & 3) << 2);
-  else return (((r >> 1) & 1) << 2) | (((r >> 3) & 1) << 1) | ((r >> 4) & 1);
-}
-template <int D>
-__device__ __forceinline__ int v_swz(int r) {
-  if constexpr (D == 128) return ((r & 3) << 2) | (((r >> 3) & 1) << 1) | ((r >> 4) & 1);
-  else return (((r >> 1) & 1) << 2) | (((r >> 3) & 1) << 1) | ((r >> 4) & 1);
-}
-
 // p[i] for a wave-uniform i through the constant address space: a scalar
 // load, counted by lgkmcnt rather than the vector memory counter
 __device__ __forceinline__ int32_t load_uniform(const int32_t* p, int i) {
@@ -105,62 +85,10 @@ __device__ __forceinline__ int32_t load_uniform(const int32_t* p, int i) {
   return ((cint*)p)[__builtin_amdgcn_readfirstlane(i)];
 }
 
-// Online softmax with a lazy reference.  s[kt][i] holds log2-domain scores of
-// this lane's keys for query column lane & 15 (-inf where masked).  The
-// running reference m of a column (log2 domain, shared by its
-// four lane groups) is raised, and O and the partial sums rescaled, only when
-// some score exceeds it by more than 2^8: the common block needs no cross-lane
-// reduction at all, and probabilities stay <= 256.  l is this lane's partial
-// row sum (its own keys); the four lane groups' parts are added at the end.
-// The scores may come unscaled: the log2-domain score is s * sc (sc > 0), and
-// the scale is folded into the exponent's argument.
-template <int KT, int DT>
-__device__ __forceinline__ void softmax_lazy(v4f (&s)[KT], v4f (&o)[DT], float& m, float& l,
-                                             float sc = 1.0f) {
-  float mx = kNegInf;
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][i]);
-  mx *= sc;
-  if (__ballot(mx > m + 8.0f)) {
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (mx > m + 8.0f) {   // the column's new reference
-      if (m != kNegInf) {   // (while m = -inf, every p so far was 0: l and o are 0)
-        const float alpha = fast_exp2(m - mx);
-        l *= alpha;
-#pragma unroll
-        for (int t = 0; t < DT; ++t) o[t] *= alpha;
-      }
-      m = mx;
-    }
-  }
-  // masked scores are -inf; a column without any admissible key yet keeps
-  // m = -inf and only -inf scores, so a zero reference gives p = 0 there
-  const float mref = m == kNegInf ? 0.0f : m;
-  float sum = 0.0f;
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float p = fast_exp2(fmaf(s[kt][i], sc, -mref));
-      s[kt][i] = p;
-      sum += p;
-    }
-  l += sum;
-}
-
-// MODE (which keys a query sees, and which key is exempt from the bias):
-//   kCausalSelf  keys j <= i of the query's own sequence; j = i exempt
-//   kFullSelf    every key of the query's own sequence;  j = i exempt
-//   kCross       every key of the sequence's key range cu_k[s]..cu_k[s+1]
-//                (k, v, key_bias indexed by key token); key 0 exempt
 // SEL (how the key blocks are chosen, fixed per launch):
 //   kSelDense    every key block the mode admits (no table)
 //   kSelShort    a block_idx row of at most 64 slots, held one slot per lane
 //   kSelLong     a longer row, read slot by slot with scalar loads
-constexpr int kCausalSelf = 0, kFullSelf = 1, kCross = 2;
 constexpr int kSelDense = 0, kSelShort = 1, kSelLong = 2;
 
 // Workgroups per CU the register budget is set for: at D = 64 a workgroup
@@ -1170,11 +1098,15 @@ extern "C" int sa_attn_varlen_fwd(int dtype, int mode, const void* q, const void
   if (num_seqs == 0 || total_q == 0) return 0;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const float scale = softmax_scale > 0.f ? softmax_scale : 1.0f / sqrtf(static_cast<float>(head_dim));
+  const int32_t* cu_k = mode == sa::kCross ? cu_seqlens_k : cu_seqlens_q;
+  const int Tk = mode == sa::kCross ? total_k : total_q;
+  // launches that fill the chip with 128-query blocks: attention_dense.hip
+  if (sa::dense_attn_ok(num_heads, total_q))
+    return sa::launch_dense_varlen(mode, head_dim, q, k, v, cu_seqlens_q, cu_k, num_seqs, key_bias, o,
+                                   total_q, Tk, num_heads, scale * sa::kLog2e, s);
   // upper bound on the query blocks (sum over sequences of ceil(len / 64));
   // blocks past the real count find no sequence and exit
   const int n_qblk = total_q / 64 + num_seqs;
-  const int32_t* cu_k = mode == sa::kCross ? cu_seqlens_k : cu_seqlens_q;
-  const int Tk = mode == sa::kCross ? total_k : total_q;
   const int rc = sa::launch_attn(mode, head_dim, q, k, v, cu_seqlens_q, cu_k, num_seqs, nullptr,
                                  n_qblk, 0, n_qblk, 1, key_bias, o, total_q, Tk, num_heads,
                                  scale * sa::kLog2e, s);

@@ -42,6 +42,7 @@ SIGNATURES: dict[str, list] = {
     "sa_sparse_attn_fwd": [_i, _vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _vp, _i, _i, _i, _f,
                            _vp, _vp],
     "sa_attn_varlen_fwd": [_i, _i, _vp, _vp, _vp, _vp, _vp, _i, _vp, _i, _i, _i, _i, _f, _vp, _vp],
+    "sa_mha_prefill_fwd": [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _f, _vp, _vp],
     "sa_rms_norm_fwd": [_i, _vp, _vp, _i64, _i, _i, _f, _vp, _vp],
     "sa_rope_bf16": [_i, _vp, _vp, _vp, _vp, _i64, _i, _i, _vp, _vp, _i, _vp],
     "sa_paged_kv_build": [_vp, _vp, _i64, _i64, _i64, _vp, _i64, _i64, _i64, _vp, _vp, _i, _i, _i,

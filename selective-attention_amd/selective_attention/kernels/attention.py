@@ -101,6 +101,28 @@ def attn_varlen(q, k, v, cu_seqlens_q, mode="causal", cu_seqlens_k=None, key_bia
     return o
 
 
+def mha_prefill(q, k, v, log_gate, lengths=None):
+    """
+    SelectiveMHA's prefill attention over batch rows (sa_mha_prefill_fwd).
+
+    Args:
+        q, k, v: (batch, seq_len, num_heads, head_dim) bfloat16, contiguous
+        log_gate: (batch, num_heads, seq_len) float32 key bias, not applied to
+            a query's own key
+        lengths: (batch,) int64 or None; rows at or past a length come out 0
+
+    Returns:
+        o: (batch, seq_len, num_heads, head_dim) bfloat16
+    """
+    require_device(q, k, v, log_gate, lengths)
+    b, L, H, D = q.shape
+    o = torch.empty_like(q)
+    _lib.call("sa_mha_prefill_fwd", _lib.DTYPE_BF16, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v),
+              _lib.ptr(log_gate), _lib.ptr(lengths), b, L, H, D, -1.0, _lib.ptr(o),
+              _lib.stream_of(q))
+    return o
+
+
 def paged_decode_attn(q, k_pages, v_pages, page_table, seq_lens, softmax_scale=None,
                       key_bias=None):
     """

@@ -7,10 +7,8 @@ per-head compacted cache (inference/selective_attn_cache.py,
 _reset_cache :11-25) for decode.  Here the same attention runs on the new
 ops:
 
-* selective_mha_prefill: each batch row is one sequence for the dense
-  causal mode of attn_varlen (the block-sparse kernel over every causal
-  block).  The gate
-  enters as key_bias = log_gate (the diagonal is exempt, as in mode "seq").
+* selective_mha_prefill: each batch row is one sequence of the dense causal
+  attention kernel.  The gate enters as key_bias = log_gate (the diagonal is exempt, as in mode "seq").
   A key the reference drops from its compressed cache (gate zeroed or below
   the threshold, or past the length) carries key_bias = -inf, which removes
   it from the softmax exactly as compression does, while the query's own key
@@ -35,9 +33,11 @@ from __future__ import annotations
 import torch
 
 from ..kernels.attention import (TRAIN_HEAD_DIMS, gated_attn_train_backward,
-                                 gated_attn_train_forward, score_moments, score_std_backward)
+                                 gated_attn_train_forward, mha_prefill, score_moments,
+                                 score_std_backward)
 from ..kernels.lm_ops import paged_kv_append, paged_kv_build
-from .attention import attn_varlen, paged_decode_attn
+from ..utils import check_shape
+from .attention import paged_decode_attn
 
 
 def _valid_pairs(Lk: int, q_lengths, k_lengths, causal: bool, i0: int, i1: int, device):
@@ -191,38 +191,24 @@ def selective_mha_prefill(q_rot: torch.Tensor, k_rot: torch.Tensor, v: torch.Ten
         (batch_size, seq_len, num_heads, head_dim) memory (the layout the
         module's output projection reads); rows past a length are 0.
 
-    Each batch row is one sequence (cu_seqlens = 0, L, 2L, ...; with
-    lengths, its valid rows and its padding rows are two sequences), so
-    nothing is packed or copied: a query t < length only reaches keys j <= t
-    of its row.  block_size is kept for the signature (the kernel's blocks
-    are 64 keys).
+    Each batch row is one sequence, read in place: nothing is packed or copied,
+    and a query t < length only reaches keys j <= t of its row.  block_size is
+    kept for the signature (the kernel's blocks are 64 keys).
     """
     b, H, L, D = q_rot.shape
     dev = q_rot.device
-    T = b * L
-    if T == 0:
+    if b * L == 0:
         return torch.zeros(b, L, H, D, dtype=torch.bfloat16, device=dev).transpose(1, 2)
 
-    def rows(x):   # (b, H, L, D) -> (b * L, H, D) rows, in place when possible
-        return x.transpose(1, 2).to(torch.bfloat16).contiguous().view(T, H, D)
+    def rows(x):   # (b, H, L, D) -> (b, L, H, D) rows, in place when possible
+        return x.transpose(1, 2).to(torch.bfloat16).contiguous()
 
-    qp, kp, vp = rows(q_rot), rows(k_rot), rows(v)
-    bias = log_gate.to(torch.float32).transpose(0, 1).reshape(H, T)
-    starts = torch.arange(b + 1, dtype=torch.int32, device=dev) * L
-    if lengths is None:
-        cu = starts
-    else:
-        # sequences [i L, i L + len_i) and, between them, the padding rows as
-        # sequences of their own (attended among themselves, then zeroed)
-        lens = lengths.to(dev, torch.int64).clamp(0, L)
-        cu = torch.empty(2 * b + 1, dtype=torch.int32, device=dev)
-        cu[0::2] = starts
-        cu[1::2] = starts[:-1] + lens.to(torch.int32)
-    o = attn_varlen(qp, kp, vp, cu, "causal", key_bias=bias).view(b, L, H, D)
-    if lengths is not None:
-        pad = torch.arange(L, device=dev)[None, :] >= lens[:, None]
-        o.masked_fill_(pad[:, :, None, None], 0.0)
-    return o.transpose(1, 2)
+    check_shape(k_rot, (b, H, L, D), name="k_rot")
+    check_shape(v, (b, H, L, D), name="v")
+    check_shape(log_gate, (b, H, L), name="log_gate")
+    lens = None if lengths is None else lengths.to(dev, torch.int64).expand(b).contiguous()
+    bias = log_gate.to(torch.float32).contiguous()
+    return mha_prefill(rows(q_rot), rows(k_rot), rows(v), bias, lens).transpose(1, 2)
 
 
 class PagedSelectiveAttnCache:

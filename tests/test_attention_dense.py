@@ -1,0 +1,91 @@
+"""Dense prefill attention on 128-query blocks (attention_dense.hip): the three
+modes of attn_varlen at sizes past its dispatch line, and SelectiveMHA's prefill
+over batch rows with 64- and 128-query blocks, against the attention formula in
+fp64 (computed per head on the GPU).  bf16 outputs: the stated rtol / atol 2e-2."""
+import pytest
+import torch
+
+from selective_attention.ops import attn_varlen, selective_mha_prefill
+from tests.helpers import assert_parity
+
+
+def attend(q, k, v, bias, mode):
+    """fp64 (Lq, D) attention of one head; key j of `bias` is not applied on the
+    query's own key ("cross": on key 0)."""
+    s = q.double() @ k.double().T * q.shape[-1] ** -0.5
+    if bias is not None:
+        b = bias.double()[None, :].expand(s.shape).clone()
+        if mode == "cross":
+            b[:, :1] = 0.0
+        else:
+            b.fill_diagonal_(0.0)
+        s = s + b
+    if mode == "causal":
+        s = s.masked_fill(torch.ones_like(s, dtype=torch.bool).triu(1), float("-inf"))
+    return torch.softmax(s, -1) @ v.double() if k.shape[0] else torch.zeros_like(q, dtype=torch.float64)
+
+
+def cu_of(lens):
+    return torch.tensor([0] + lens).cumsum(0).to(torch.int32).cuda()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("mode", ["causal", "full", "cross"])
+@pytest.mark.parametrize("biased", [False, True])
+def test_packed_modes(mode, D, biased):
+    H, lens = 4, [16000, 1, 127, 128, 129, 65, 0, 63, 200]
+    klens = [300, 1, 0, 64, 65, 31, 5, 33, 129] if mode == "cross" else lens
+    g = torch.Generator(device="cuda").manual_seed(D)
+    r = lambda n: torch.randn(n, H, D, generator=g, device="cuda").bfloat16()
+    q, k, v = r(sum(lens)), r(sum(klens)), r(sum(klens))
+    bias = None
+    if biased:
+        bias = 2.0 * torch.randn(H, sum(klens), generator=g, device="cuda")
+        bias = bias.masked_fill(torch.rand(bias.shape, generator=g, device="cuda") < 0.1, float("-inf"))
+    cu, cuk = cu_of(lens), cu_of(klens)
+    o = attn_varlen(q, k, v, cu, mode, cuk if mode == "cross" else None, bias)
+    a = e = 0
+    for n, m in zip(lens, klens):
+        for h in range(H if n < 1000 else 1):
+            # the long sequence: its first, middle and last query blocks
+            for i in ([0] if n < 1000 else [0, 7936, n - 130]):
+                j = min(n, i + 300)
+                hi = j if mode == "causal" else m
+                qs = torch.zeros(hi, D, device="cuda", dtype=torch.bfloat16)
+                if mode == "cross":
+                    want = attend(q[a + i:a + j, h], k[e:e + m, h], v[e:e + m, h],
+                                  None if bias is None else bias[h, e:e + m], mode)
+                else:
+                    qs[:min(hi, n)] = q[a:a + min(hi, n), h]
+                    want = attend(qs, k[e:e + hi, h], v[e:e + hi, h],
+                                  None if bias is None else bias[h, e:e + hi], mode)[i:j]
+                assert_parity(o[a + i:a + j, h], want.cpu(), torch.bfloat16, f"{mode} n={n} h={h} i={i}")
+        a, e = a + n, e + m
+    assert torch.equal(o, attn_varlen(q, k, v, cu, mode, cuk if mode == "cross" else None, bias))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,H,L,D,lens", [
+    (1, 2, 1, 64, None), (2, 2, 64, 64, [64, 63]), (3, 2, 130, 128, [130, 0, 129]),
+    (2, 3, 200, 64, [1, 128]), (2, 16, 2100, 64, [2100, 1999]), (4, 32, 515, 128, [515, 130, 257, 64]),
+])
+def test_rows(b, H, L, D, lens):
+    """The last two take 128-query blocks, the others 64."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q, k, v = (torch.randn(b, L, H, D, generator=g, device="cuda").bfloat16().transpose(1, 2)
+               for _ in range(3))
+    lg = torch.log(torch.sigmoid(torch.randn(b, H, L, generator=g, device="cuda") + 1))
+    lg = lg.masked_fill(torch.rand(b, H, L, generator=g, device="cuda") < 0.2, float("-inf"))
+    lt = None if lens is None else torch.tensor(lens).cuda()
+    o = selective_mha_prefill(q, k, v, lg, lt)
+    assert o.shape == (b, H, L, D) and o.transpose(1, 2).is_contiguous()
+    for i in range(b):
+        n = L if lens is None else lens[i]
+        assert not o[i, :, n:].any()
+        for h in range(0, H, max(1, H // 4)):
+            if n:
+                want = attend(q[i, h, :n], k[i, h, :n], v[i, h, :n], lg[i, h, :n], "causal")
+                assert_parity(o[i, h, :n], want.cpu(), torch.bfloat16, f"row {i} head {h}")
+    # any other layout is copied: the same bits
+    assert torch.equal(o, selective_mha_prefill(q.contiguous(), k, v.contiguous(), lg, lt))
