@@ -10,14 +10,21 @@
 // traffic, barriers and per-tile overhead per score, and no merge.  The key
 // bias enters as the MFMA's initial accumulator (bias / softmax_scale, one value
 // per key row of the transposed score tile), which costs no instruction per
-// score; the scale is folded into the exponent's argument as before.  The
-// kernel is bound by VALU issue (per score an FMA, an exponential, an add and
-// half a conversion), the matrix cores and the tile DMA run beside it.
+// score; the scale is folded into the exponent's argument as before.  Wave 0
+// turns a tile's biases into raw score units on their way to its stage, once.
+// What is left per score is an FMA, an exponential (half rate), an add and
+// half a conversion: VALU busy 47 % of the cycles and the matrix cores 37 %,
+// 13 % both; the rest is waits on LDS, barriers and, for launches of one to
+// two resident rounds, the last round.
 //
 // JT = 1 (64 queries) takes SelectiveMHA launches that would leave the chip
 // short of 128-query blocks.  Small packed launches keep the block-sparse
 // kernel's dense form.
-// Measured: FIGURES
+// Measured, block-sparse kernel -> here: causal rows b 4, H 16, L 8192 (ragged),
+// D 64: 545 -> 403 us (the whole op 597 -> 407); bidirectional, 4 sequences of
+// 1500 to 4096, H 16, D 64, biased: 261 -> 214 us.  The same with a maximum per
+// block instead of the sum test, the biases scaled by every wave and 168
+// instead of 128 VGPRs: 234, 224 and 226 us.
 #include "attn_tile.h"
 #include "prof.h"
 
@@ -36,7 +43,7 @@ struct DenseArgs {
   const float* key_bias;       // packed: (H, Tk); rows: (rows, H, L)
   bf16* o;
   int nseq, grid_q, T, Tk, H, L;
-  float scale_log2, inv_scale;
+  float scale_log2, inv_scale;   // softmax_scale log2(e), 1 / softmax_scale
 };
 
 // D = 64: 33 KB of LDS and a 128-VGPR budget (no spills), four blocks per CU;
@@ -147,9 +154,6 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void dense_attn_kernel(DenseA
     const uint32_t kt = st + lds_wave, vt = kt + 2 * kKeys * D;
     const bf16* kb0 = kbase + static_cast<long>(k0) * rs;
     const bf16* vb0 = vbase + static_cast<long>(k0) * rs;
-    if constexpr (BIAS) {
-      if (w == 0) dma_lds4(bias, 4u * min(k0 + lane, nks - 1), st + 4 * kKeys * D);
-    }
     if (nk == kKeys) {
 #pragma unroll
       for (int i = 0; i < IPW; ++i) {
@@ -167,15 +171,26 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void dense_attn_kernel(DenseA
     }
   };
 
-  float m[JT], l[JT];
+  SoftmaxCol col[JT];
   v4f acc[JT][DT];
 #pragma unroll
   for (int jt = 0; jt < JT; ++jt) {
-    m[jt] = kNegInf;
-    l[jt] = 0.f;
+    col[jt] = SoftmaxCol{-1.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < DT; ++t) acc[jt][t] = v4f{0.f, 0.f, 0.f, 0.f};
   }
+  // the next tile's biases, one per lane of wave 0, on their way to its stage in raw score units
+  float bnext = 0.f;
+  auto load_bias = [&](int kb) __attribute__((always_inline)) {
+    if constexpr (BIAS) {
+      if (w == 0) bnext = bias[min(kb * kKeys + lane, nks - 1)];
+    }
+  };
+  auto store_bias = [&](bf16* st) __attribute__((always_inline)) {
+    if constexpr (BIAS) {
+      if (w == 0) reinterpret_cast<float*>(st + 2 * kKeys * D)[lane] = bnext * a.inv_scale;
+    }
+  };
   // per-lane pieces of the swizzled LDS addresses (rows 32 apart share them)
   int krow_off[2], kswz[2];
 #pragma unroll
@@ -187,12 +202,16 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void dense_attn_kernel(DenseA
   const int vr = 8 * g + (c >> 2), vswz = v_swz<D>(vr);
   const int vhalf = 4 * (c & 1), vchunk = (c & 3) >> 1;
 
-  auto step = [&](int e, const bf16* Ks, uint32_t nxt) __attribute__((always_inline)) {
+  auto step = [&](int e, const bf16* Ks, bf16* nst, uint32_t nxt) __attribute__((always_inline)) {
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_waitcnt(vm_wait<0>());
     __builtin_amdgcn_s_barrier();   // tile e has landed; every wave is done with tile e - 1
     asm volatile("" ::: "memory");
-    if (e + 1 < nt) issue(e + 1, nxt);
+    if (e + 1 < nt) {
+      store_bias(nst);   // (loaded a step ago)
+      issue(e + 1, nxt);
+      if (e + 2 < nt) load_bias(e + 2);
+    }
     if (e < wt) {
       const bf16* Vs = Ks + kKeys * D;
       const int k0 = e * kKeys;
@@ -209,8 +228,8 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void dense_attn_kernel(DenseA
         v4f b0 = v4f{0.f, 0.f, 0.f, 0.f}, b1 = b0;   // biases of keys 8g .. 8g + 7, in raw score units
         if constexpr (BIAS) {
           const float* bs = reinterpret_cast<const float*>(Vs + kKeys * D) + 32 * hh + 8 * g;
-          b0 = *reinterpret_cast<const v4f*>(bs) * a.inv_scale;
-          b1 = *reinterpret_cast<const v4f*>(bs + 4) * a.inv_scale;
+          b0 = *reinterpret_cast<const v4f*>(bs);
+          b1 = *reinterpret_cast<const v4f*>(bs + 4);
         }
         v8bf kfr[2][KS];
 #pragma unroll
@@ -269,8 +288,7 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void dense_attn_kernel(DenseA
         v8bf pb[JT];
 #pragma unroll
         for (int jt = 0; jt < JT; ++jt) {
-          softmax_lazy<2, DT>(sc[jt], acc[jt], m[jt], l[jt], a.scale_log2);
-          pb[jt] = pack_p(sc[jt][0], sc[jt][1]);
+          pb[jt] = softmax_col<DT>(sc[jt], acc[jt], col[jt], a.scale_log2);
         }
 #pragma unroll
         for (int t = 0; t < DT; ++t)
@@ -284,11 +302,16 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void dense_attn_kernel(DenseA
   // the query fragments have arrived before the loop: nothing the compiler
   // tracks is in flight inside it
   __builtin_amdgcn_s_waitcnt(vm_wait<0>());
-  if (nt > 0) issue(0, lds_st0);
+  if (nt > 0) {
+    load_bias(0);
+    store_bias(stage0);
+    issue(0, lds_st0);
+    if (nt > 1) load_bias(1);
+  }
   for (int e = 0; e < nt; e += 2) {
-    step(e, stage0, lds_st1);
+    step(e, stage0, stage1, lds_st1);
     if (e + 1 >= nt) break;
-    step(e + 1, stage1, lds_st0);
+    step(e + 1, stage1, stage0, lds_st0);
   }
   __builtin_amdgcn_s_barrier();   // every wave is done with the tiles
   asm volatile("" ::: "memory");
@@ -300,7 +323,7 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void dense_attn_kernel(DenseA
   bf16* ot = stage0 + w * QW * D;
 #pragma unroll
   for (int jt = 0; jt < JT; ++jt) {
-    float lt = l[jt];
+    float lt = col[jt].l;
     lt += __shfl_xor(lt, 16, 64);
     lt += __shfl_xor(lt, 32, 64);
     const float inv = lt > 0.0f ? 1.0f / lt : 0.0f;

@@ -34,50 +34,57 @@ __device__ __forceinline__ int v_swz(int r) {
   else return (((r >> 1) & 1) << 2) | (((r >> 3) & 1) << 1) | ((r >> 4) & 1);
 }
 
-// Online softmax with a lazy reference.  s[kt][i] holds log2-domain scores of
-// this lane's keys for query column lane & 15 (-inf where masked).  The
-// running reference m of a column (log2 domain, shared by its
-// four lane groups) is raised, and O and the partial sums rescaled, only when
-// some score exceeds it by more than 2^8: the common block needs no cross-lane
-// reduction at all, and probabilities stay <= 256.  l is this lane's partial
-// row sum (its own keys); the four lane groups' parts are added at the end.
-// The scores may come unscaled: the log2-domain score is s * sc (sc > 0), and
-// the scale is folded into the exponent's argument.
-template <int KT, int DT>
-__device__ __forceinline__ void softmax_lazy(v4f (&s)[KT], v4f (&o)[DT], float& m, float& l,
-                                             float sc = 1.0f) {
-  float mx = kNegInf;
+// Online softmax of one query column with a lazy reference (log2 domain): p =
+// 2^(score - reference), the reference raised, and O and the lane's partial
+// row sum rescaled, only when needed.  A p above 2^8 shows in the sum of the
+// lane's eight p, which the row sum needs anyway: no maximum is taken in the
+// common block.  (The sum passes 2^8 without a single p above it at times;
+// the reference is then raised early, to the same effect.)
+struct SoftmaxCol {
+  float limit;   // sums above this raise the reference: 2^8, or -1 while there is none
+  float neg;     // minus the reference; 0 while there is none
+  float l;       // the lane's sum of p
+};
+__device__ __forceinline__ float exp_sum(const v4f (&s)[2], v4f (&p)[2], float sc, float neg) {
 #pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
+  for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][i]);
-  mx *= sc;
-  if (__ballot(mx > m + 8.0f)) {
+    for (int i = 0; i < 4; ++i) p[u][i] = fast_exp2(fmaf(s[u][i], sc, neg));
+  return ((p[0][0] + p[0][1]) + (p[0][2] + p[0][3])) + ((p[1][0] + p[1][1]) + (p[1][2] + p[1][3]));
+}
+template <int DT>
+__device__ __forceinline__ v8bf softmax_col(const v4f (&s)[2], v4f (&o)[DT], SoftmaxCol& c, float sc) {
+  v4f p[2];
+  float sum = exp_sum(s, p, sc, c.neg);
+  if (__ballot(sum > c.limit)) {
+    float mx = kNegInf;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[u][i]);
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    if (mx > m + 8.0f) {   // the column's new reference
-      if (m != kNegInf) {   // (while m = -inf, every p so far was 0: l and o are 0)
-        const float alpha = fast_exp2(m - mx);
-        l *= alpha;
+    const float ref = mx * sc;
+    // a column's four lane groups share the reference, so they decide alike
+    const bool up = c.limit < 0.f ? mx > kNegInf : ref > -c.neg;
+    if (up) {
+      if (c.limit > 0.f) {
+        const float alpha = fast_exp2(-c.neg - ref);
+        c.l *= alpha;
 #pragma unroll
         for (int t = 0; t < DT; ++t) o[t] *= alpha;
       }
-      m = mx;
+      c.neg = -ref;
+      c.limit = 256.0f;
+    }
+    sum = exp_sum(s, p, sc, c.neg);
+    if (c.limit < 0.f) {   // masked keys only so far
+      sum = 0.f;
+      p[0] = p[1] = v4f{0.f, 0.f, 0.f, 0.f};
     }
   }
-  // masked scores are -inf; a column without any admissible key yet keeps
-  // m = -inf and only -inf scores, so a zero reference gives p = 0 there
-  const float mref = m == kNegInf ? 0.0f : m;
-  float sum = 0.0f;
-#pragma unroll
-  for (int kt = 0; kt < KT; ++kt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float p = fast_exp2(fmaf(s[kt][i], sc, -mref));
-      s[kt][i] = p;
-      sum += p;
-    }
-  l += sum;
+  c.l += sum;
+  return pack_p(p[0], p[1]);
 }
 
 // dense attention on 128-query blocks (attention_dense.hip).  Packed sequences
