@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256) void chunk_cumsum_kernel(
     if (j < per && tau < lim) {
       const long t = static_cast<long>(c) * d.Lc + tau;
       const float z = load_f32(delta_raw + (static_cast<long>(b) * d.L + t) * d.H + h) + bias;
-      v[j] = make_dt(z, softplus != 0, dmin, dmax);
+      v[j] = chunk_dt<T>(z, softplus != 0, dmin, dmax);
     }
   }
   Acc part[4];
