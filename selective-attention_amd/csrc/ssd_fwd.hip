@@ -1114,11 +1114,14 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_fwd_bf16_kernel(
   if constexpr (!kEarlyH) load_h(0);
 
   // ---- state contribution exp(dc_tau) * H_in . C^T, one head per stage ----
-  // Without the gate epilogue, the y rows of head k leave through LDS as soon
-  // as its state part is added, so that their stores overlap the next head's
-  // stage: lane pieces in at 16-byte chunk c ^ (row % 16) of [64 rows][64 p]
-  // fp32, then whole 256-byte rows out, 16 bytes per lane (stored from the
-  // fragments, one instruction wrote 64 bytes of each of 16 rows).  The
+  // The y rows of head k leave through LDS as soon as its state part is added,
+  // so that their stores overlap the next head's stage: lane pieces in at
+  // 16-byte chunk c ^ (row % 16) of [64 rows][64 p] fp32, then whole rows out,
+  // 16 bytes per lane (stored from the fragments, one instruction wrote 64
+  // bytes of each of 16 rows).  With the gate epilogue the rows meet their u
+  // and gate there, loaded 16 bytes per lane a stage ahead (from the fragment
+  // layout these reads and both stores were 8-byte pieces, issued at the end:
+  // b 8, L 4096, H 16, N 64, one group: 126 -> 92 us, the same bits).  The
   // staging is the B tile's space when that holds 16 KB, else the U region
   // past the H_in tile; either is disjoint from H_in.
   constexpr int kHsBytes = static_cast<int>(sizeof(bf16)) * 64 * TB::kLd;
@@ -1134,6 +1137,20 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_fwd_bf16_kernel(
     if (k >= nh) break;
     const bool more = k + 1 < nh;
     if (more) load_h(k + 1);
+    // GATED: the head's u and gate rows and D, on their way during the state stage
+    uint4 gu[2], gg[2];
+    float4 gd[2];
+    if constexpr (GATED) {
+      const int col = min(p0 + 8 * (tid & 7), d.P - 8);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = min(t0 + ((tid + 256 * i) >> 3), qlim - 1);
+        const long at = (tok0 + r) * u_rs + static_cast<long>(h0 + k) * d.P + col;
+        gu[i] = *reinterpret_cast<const uint4*>(u + at);
+        gg[i] = *reinterpret_cast<const uint4*>(go.gate + at);
+        gd[i] = *reinterpret_cast<const float4*>(go.D + (h0 + k) * d.P + col + 4 * i);
+      }
+    }
     const float e = fast_exp2(dct[k]);
     {
       v4f st[4];
@@ -1152,13 +1169,13 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_fwd_bf16_kernel(
 #pragma unroll
       for (int t = 0; t < 4; ++t) acc[k][t] += st[t] * e;
     }
-    if constexpr (!GATED) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t)
-        *reinterpret_cast<float4*>(ys + rl * 64 + 4 * ((4 * t + lg) ^ (rl & 15))) =
-            make_float4(acc[k][t][0], acc[k][t][1], acc[k][t][2], acc[k][t][3]);
-      __syncthreads();   // head k's rows staged; every wave is done with its H_in tile
-      if (more) commit_h();
+    for (int t = 0; t < 4; ++t)
+      *reinterpret_cast<float4*>(ys + rl * 64 + 4 * ((4 * t + lg) ^ (rl & 15))) =
+          make_float4(acc[k][t][0], acc[k][t][1], acc[k][t][2], acc[k][t][3]);
+    __syncthreads();   // head k's rows staged; every wave is done with its H_in tile
+    if (more) commit_h();
+    if constexpr (!GATED) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int e2 = tid + 256 * i, r = e2 >> 4, ch = e2 & 15;
@@ -1166,41 +1183,34 @@ __global__ __launch_bounds__(256, 2) void chunk_scan_fwd_bf16_kernel(
           *reinterpret_cast<float4*>(y + (tok0 + t0 + r) * u_rs + static_cast<long>(h0 + k) * d.P + p0 + 4 * ch) =
               *reinterpret_cast<const float4*>(ys + r * 64 + 4 * (ch ^ (r & 15)));
       }
-      if (more) __syncthreads();   // the next H_in tile is in; the staging is free
-    } else if (more) {
-      __syncthreads();
-      commit_h();
-      __syncthreads();
-    }
-  }
-  if constexpr (GATED) {
-    if (tau < qlim) {
+    } else {
       // SSM epilogue: yd = y + D u, out = yd silu(gate) (bf16; y itself is not stored)
+      const float Dv[8] = {gd[0].x, gd[0].y, gd[0].z, gd[0].w, gd[1].x, gd[1].y, gd[1].z, gd[1].w};
 #pragma unroll
-      for (int k = 0; k < HC; ++k) {
-        if (k >= nh) break;
-        const long row = (tok0 + tau) * u_rs + static_cast<long>(h0 + k) * d.P;
+      for (int i = 0; i < 2; ++i) {
+        const int e2 = tid + 256 * i, r = e2 >> 3, ch = e2 & 7;
+        if (t0 + r < qlim && p0 + 8 * ch < d.P) {
+          const float4 y0 = *reinterpret_cast<const float4*>(ys + r * 64 + 4 * ((2 * ch) ^ (r & 15)));
+          const float4 y1 = *reinterpret_cast<const float4*>(ys + r * 64 + 4 * ((2 * ch + 1) ^ (r & 15)));
+          const float yv[8] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
+          const uint32_t uw[4] = {gu[i].x, gu[i].y, gu[i].z, gu[i].w};
+          const uint32_t gw[4] = {gg[i].x, gg[i].y, gg[i].z, gg[i].w};
+          uint32_t ow[4], dw[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const int p = p0 + 16 * t + 4 * lg;
-          if (p >= d.P) continue;
-          const uint2 uq = *reinterpret_cast<const uint2*>(u + row + p);
-          const uint2 gq = *reinterpret_cast<const uint2*>(go.gate + row + p);
-          const float4 dq = *reinterpret_cast<const float4*>(go.D + (h0 + k) * d.P + p);
-          const float uv[4] = {bf16lo_to_f32(uq.x), bf16hi_to_f32(uq.x), bf16lo_to_f32(uq.y), bf16hi_to_f32(uq.y)};
-          const float gv[4] = {bf16lo_to_f32(gq.x), bf16hi_to_f32(gq.x), bf16lo_to_f32(gq.y), bf16hi_to_f32(gq.y)};
-          const float Dv[4] = {dq.x, dq.y, dq.z, dq.w};
-          float yd[4], o[4];
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            yd[i] = acc[k][t][i] + Dv[i] * uv[i];
-            o[i] = yd[i] * gv[i] * fast_sigmoid(gv[i]);
+          for (int q = 0; q < 4; ++q) {
+            const float a0 = yv[2 * q] + Dv[2 * q] * bf16lo_to_f32(uw[q]);
+            const float a1 = yv[2 * q + 1] + Dv[2 * q + 1] * bf16hi_to_f32(uw[q]);
+            const float g0 = bf16lo_to_f32(gw[q]), g1 = bf16hi_to_f32(gw[q]);
+            dw[q] = pack_bf16x2(a0, a1);
+            ow[q] = pack_bf16x2(a0 * g0 * fast_sigmoid(g0), a1 * g1 * fast_sigmoid(g1));
           }
-          *reinterpret_cast<uint2*>(go.out + row + p) = uint2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-          *reinterpret_cast<uint2*>(go.yd + row + p) = uint2{pack_bf16x2(yd[0], yd[1]), pack_bf16x2(yd[2], yd[3])};
+          const long at = (tok0 + t0 + r) * u_rs + static_cast<long>(h0 + k) * d.P + p0 + 8 * ch;
+          *reinterpret_cast<uint4*>(go.out + at) = uint4{ow[0], ow[1], ow[2], ow[3]};
+          *reinterpret_cast<uint4*>(go.yd + at) = uint4{dw[0], dw[1], dw[2], dw[3]};
         }
       }
     }
+    if (more) __syncthreads();   // the next H_in tile is in; the staging is free
   }
 }
 
