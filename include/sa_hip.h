@@ -130,6 +130,18 @@ int sa_ssd_bwd(int dtype, const void* u, const float* A, const void* B, const vo
                void* ddelta_raw, float* ddelta_bias, float* dh_init, void* workspace,
                size_t workspace_bytes, void* stream);
 
+/* sa_ssd_bwd with du + du_add in place of du: du_add (or NULL) a tensor of the
+ * shape and dtype of du (the skip path's gradient), added after du is rounded
+ * to that dtype. */
+int sa_ssd_bwd_add(int dtype, const void* u, const float* A, const void* B, const void* C,
+                   const void* delta_raw, const float* delta_bias, const int64_t* length,
+                   const float* dy, const float* dh_last, const float* dt, const float* dc,
+                   const float* states, int batch, int seqlen, int num_heads, int head_dim,
+                   int num_groups, int state_dim, int chunk_size, int use_softplus,
+                   float delta_min, float delta_max, int has_h_init, const void* du_add, void* du,
+                   float* dA, void* dB, void* dC, void* ddelta_raw, float* ddelta_bias,
+                   float* dh_init, void* workspace, size_t workspace_bytes, void* stream);
+
 /*
  * Varlen block-sparse causal self-attention (prefill), bfloat16.  No
  * counterpart kernel in the reference: semantics of SelectiveMHA's gated

@@ -891,6 +891,18 @@ __global__ __launch_bounds__(256) void param_grad_reduce_kernel(const float* __r
   }
 }
 
+// du += add, element by element (each thread four, 256 apart)
+template <typename T>
+__global__ __launch_bounds__(256) void du_add_kernel(const T* __restrict__ add, long n,
+                                                     T* __restrict__ du) {
+  const long i0 = static_cast<long>(blockIdx.x) * 1024 + threadIdx.x;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const long i = i0 + 256 * j;
+    if (i < n) st(du + i, load_f32(du + i) + load_f32(add + i));
+  }
+}
+
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -924,8 +936,8 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
                  const void* delta_raw_, const float* bias, const int64_t* length,
                  const float* dy, const float* dh_last, const float* dt, const float* dc,
                  const float* states, const SsdDims& d, int sp, float lo, float hi, int has_init,
-                 void* du_, float* dA, void* dB_, void* dC_, void* ddelta_, float* dbias,
-                 float* dh_init, unsigned char* ws, hipStream_t s) {
+                 const void* du_add, void* du_, float* dA, void* dB_, void* dC_, void* ddelta_,
+                 float* dbias, float* dh_init, unsigned char* ws, hipStream_t s) {
   const T* u = static_cast<const T*>(u_);
   const T* Bm = static_cast<const T*>(B_);
   const T* Cm = static_cast<const T*>(C_);
@@ -976,9 +988,9 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
   int ptiles = w.ptiles, ntiles = w.ntiles, xctiles = w.ntiles, qtiles = w.ttiles, rtiles = 1;
   if (fused) {
     // 3-5 fused: du, dB, dC, decay sums
-    if ((rc = launch_ssd_bwd_fused(u, Bm, Cm, dyp, dt, dc, states, dSp, length, du_, dB_, dC_,
-                                   dcbp, ddt_part, xB_part, xC_part, qpart, rsum, d,
-                                   lo >= 0.f, s)))
+    if ((rc = launch_ssd_bwd_fused(u, Bm, Cm, dyp, dt, dc, states, dSp, length,
+                                   aligned16(du_add) ? du_add : nullptr, du_, dB_, dC_, dcbp,
+                                   ddt_part, xB_part, xC_part, qpart, rsum, d, lo >= 0.f, s)))
       return rc;
     ptiles = ntiles = qtiles = 1;
     xctiles = d.N / 64;   // x_C: one partial per 64 n (ssd_bwd_tgt block)
@@ -1028,6 +1040,14 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
     SA_CHECK_LAUNCH("chunk_dbdc_bwd");
   }
   }
+  // du += du_add where the kernels above did not add it as they stored du
+  if (du_add && !(fused && aligned16(du_add))) {
+    const long n = static_cast<long>(d.b) * d.L * d.H * d.P;
+    ProfScope prof_("du_add", s);
+    hipLaunchKernelGGL(du_add_kernel<T>, dim3((n + 1023) / 1024), dim3(256), 0, s,
+                       static_cast<const T*>(du_add), n, static_cast<T*>(du_));
+    SA_CHECK_LAUNCH("du_add");
+  }
   // 6. decay-gradient assembly, d delta_raw, dA/dbias partials
   {
     const long blocks = bnc * d.H;
@@ -1065,14 +1085,16 @@ extern "C" size_t sa_ssd_bwd_workspace_size(int dtype, int batch, int seqlen, in
   return sa::bwd_layout(d, dtype == sa::kBF16 ? 2 : 4).total;
 }
 
-extern "C" int sa_ssd_bwd(int dtype, const void* u, const float* A, const void* B, const void* C,
-                          const void* delta_raw, const float* delta_bias, const int64_t* length,
-                          const float* dy, const float* dh_last, const float* dt, const float* dc,
-                          const float* states, int batch, int seqlen, int num_heads, int head_dim,
-                          int num_groups, int state_dim, int chunk_size, int use_softplus,
-                          float delta_min, float delta_max, int has_h_init, void* du, float* dA,
-                          void* dB, void* dC, void* ddelta_raw, float* ddelta_bias,
-                          float* dh_init, void* workspace, size_t workspace_bytes, void* stream) {
+extern "C" int sa_ssd_bwd_add(int dtype, const void* u, const float* A, const void* B,
+                              const void* C, const void* delta_raw, const float* delta_bias,
+                              const int64_t* length, const float* dy, const float* dh_last,
+                              const float* dt, const float* dc, const float* states, int batch,
+                              int seqlen, int num_heads, int head_dim, int num_groups,
+                              int state_dim, int chunk_size, int use_softplus, float delta_min,
+                              float delta_max, int has_h_init, const void* du_add, void* du,
+                              float* dA, void* dB, void* dC, void* ddelta_raw, float* ddelta_bias,
+                              float* dh_init, void* workspace, size_t workspace_bytes,
+                              void* stream) {
   sa::SsdDims d;
   int rc = sa::make_dims(batch, seqlen, num_heads, head_dim, num_groups, state_dim, chunk_size, &d,
                          "sa_ssd_bwd");
@@ -1092,10 +1114,24 @@ extern "C" int sa_ssd_bwd(int dtype, const void* u, const float* A, const void* 
   if (dtype == sa::kF32)
     return sa::ssd_bwd_impl<float, float>(u, A, B, C, delta_raw, delta_bias, length, dy, dh_last,
                                           dt, dc, states, d, use_softplus, delta_min, delta_max,
-                                          has_h_init, du, dA, dB, dC, ddelta_raw, ddelta_bias,
-                                          dh_init, ws, s);
+                                          has_h_init, du_add, du, dA, dB, dC, ddelta_raw,
+                                          ddelta_bias, dh_init, ws, s);
   return sa::ssd_bwd_impl<sa::bf16, sa::bf16>(u, A, B, C, delta_raw, delta_bias, length, dy,
                                               dh_last, dt, dc, states, d, use_softplus, delta_min,
-                                              delta_max, has_h_init, du, dA, dB, dC, ddelta_raw,
-                                              ddelta_bias, dh_init, ws, s);
+                                              delta_max, has_h_init, du_add, du, dA, dB, dC,
+                                              ddelta_raw, ddelta_bias, dh_init, ws, s);
+}
+
+extern "C" int sa_ssd_bwd(int dtype, const void* u, const float* A, const void* B, const void* C,
+                          const void* delta_raw, const float* delta_bias, const int64_t* length,
+                          const float* dy, const float* dh_last, const float* dt, const float* dc,
+                          const float* states, int batch, int seqlen, int num_heads, int head_dim,
+                          int num_groups, int state_dim, int chunk_size, int use_softplus,
+                          float delta_min, float delta_max, int has_h_init, void* du, float* dA,
+                          void* dB, void* dC, void* ddelta_raw, float* ddelta_bias,
+                          float* dh_init, void* workspace, size_t workspace_bytes, void* stream) {
+  return sa_ssd_bwd_add(dtype, u, A, B, C, delta_raw, delta_bias, length, dy, dh_last, dt, dc, states,
+                        batch, seqlen, num_heads, head_dim, num_groups, state_dim, chunk_size,
+                        use_softplus, delta_min, delta_max, has_h_init, nullptr, du, dA, dB, dC,
+                        ddelta_raw, ddelta_bias, dh_init, workspace, workspace_bytes, stream);
 }

@@ -133,6 +133,24 @@ __device__ __forceinline__ void write_rows(const bf16* t, bf16* g, int grs, int 
   }
 }
 
+// the same for a 64 x 64 tile plus `add` (this thread's 16 bytes of each row
+// it writes), summed in fp32 and rounded
+__device__ __forceinline__ uint32_t add_bf16x2(uint32_t a, uint32_t b) {
+  return pack_bf16x2(bf16lo_to_f32(a) + bf16lo_to_f32(b), bf16hi_to_f32(a) + bf16hi_to_f32(b));
+}
+__device__ __forceinline__ void write_rows_add(const bf16* t, const uint4 (&add)[2], bf16* g, int grs,
+                                               int rows_valid, int tid) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int e = tid + 256 * i, r = e / 8, c = e % 8;
+    const uint4 v = *reinterpret_cast<const uint4*>(t + r * 64 + 8 * (c ^ (r & 7)));
+    if (r < rows_valid)
+      *reinterpret_cast<uint4*>(g + static_cast<unsigned>(r * grs + 8 * c)) =
+          uint4{add_bf16x2(v.x, add[i].x), add_bf16x2(v.y, add[i].y), add_bf16x2(v.z, add[i].z),
+                add_bf16x2(v.w, add[i].w)};
+  }
+}
+
 // fragment of 8 consecutive bf16 of one swizzled row
 template <int RC, int (*F)(int)>
 __device__ __forceinline__ v8bf row_frag(const bf16* t, int row, int col) {
@@ -250,6 +268,13 @@ __device__ __forceinline__ int opaque(int v) {
 // pass adds its share to it (each lane reads back only what it wrote).
 // Passes other than the last hold their heads' u rows in registers; every
 // pass holds the source row's B.
+//
+// ADD: du_add's rows (the skip path's gradient) are read a barrier ahead of
+// the du rows and added as these are stored, du rounded first, as du + du_add
+// of the two tensors would be.  A separate add reads and writes du once more:
+// the training step of an 8 x 4096-token, 16-head block 775 -> 758 us.  Its
+// own instance, as the pointer and the branch alone cost the scan without it
+// 1 % (1151 -> 1163 us at 8 x 4096 tokens, 32 heads).
 // ---------------------------------------------------------------------------
 template <int NK>
 struct SrcSmem {
@@ -262,12 +287,13 @@ enum SrcMode { kSrcOnly = 0, kSrcFirst = 1, kSrcMiddle = 2, kSrcLast = 3 };
 // pass plans: one pass (at most HS heads), two passes, more than two
 enum SrcPlan { kPlanOne = 0, kPlanTwo = 1, kPlanMany = 2 };
 
-template <int NK, int HS, int PLAN>
+template <int NK, int HS, int PLAN, bool ADD>
 __global__ __launch_bounds__(256, 2) void ssd_bwd_src_kernel(
     const bf16* __restrict__ u, const bf16* __restrict__ Bm, const bf16* __restrict__ Cm,
     const bf16* __restrict__ dyp, const float* __restrict__ dt, const float* __restrict__ dc,
-    const bf16* __restrict__ dSp, const int64_t* __restrict__ length, bf16* __restrict__ du,
-    bf16* __restrict__ dB, bf16* __restrict__ dcbp, float* __restrict__ ddt_part,
+    const bf16* __restrict__ dSp, const int64_t* __restrict__ length,
+    const bf16* __restrict__ du_add, bf16* __restrict__ du, bf16* __restrict__ dB,
+    bf16* __restrict__ dcbp, float* __restrict__ ddt_part,
     float* __restrict__ xB_part, float* __restrict__ qpart, float* __restrict__ rpart,
     SsdDims d, int mono) {
   using SM = SrcSmem<NK>;
@@ -326,6 +352,7 @@ __global__ __launch_bounds__(256, 2) void ssd_bwd_src_kernel(
   const float* dcc = dc + bhc0 * d.Lc;
   const float* dtc = dt + bhc0 * d.Lc;
   bf16* duc = du + tok0 * u_rs + h0 * 64;
+  const bf16* addc = ADD ? du_add + tok0 * u_rs + h0 * 64 : nullptr;
   bf16* dBc = dB + tok0 * act_rs + static_cast<long>(g) * N;
   float* ddtc = ddt_part + bhc0 * d.Lc;
   float* xBc = xB_part + bhc0 * d.Lc;
@@ -336,8 +363,11 @@ __global__ __launch_bounds__(256, 2) void ssd_bwd_src_kernel(
   if (s0 >= lim) {   // the strip is past the length: zero outputs and partials
     for (int e = tid; e < 64 * hpg * 8; e += 256) {
       const int row = e / (hpg * 8), col8 = e % (hpg * 8);
-      if (s0 + row < qlim)
-        *reinterpret_cast<uint4*>(duc + static_cast<unsigned>((s0 + row) * u_rs + 8 * col8)) = uint4{0u, 0u, 0u, 0u};
+      if (s0 + row < qlim) {
+        const unsigned o = static_cast<unsigned>((s0 + row) * u_rs + 8 * col8);
+        *reinterpret_cast<uint4*>(duc + o) =
+            ADD ? *reinterpret_cast<const uint4*>(addc + o) : uint4{0u, 0u, 0u, 0u};
+      }
     }
     for (int e = tid; e < 64 * (N / 8); e += 256) {
       const int row = e / (N / 8), col8 = e % (N / 8);
@@ -836,10 +866,26 @@ __global__ __launch_bounds__(256, 2) void ssd_bwd_src_kernel(
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) stage_out8<RCB>(stg1, sl, 16 * nt + 4 * lg, pack4_bf16(dBT[nt]));
     }
+    // the rows to add to du, on their way across the barrier
+    [[maybe_unused]] uint4 add[HS][2];
+    if constexpr (ADD) {
+#pragma unroll
+      for (int h = 0; h < HS; ++h)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int e = tid + 256 * i, r = min(s0 + (e >> 3), qlim - 1);
+          add[h][i] = *reinterpret_cast<const uint4*>(
+              addc + min(KB + h, hpg - 1) * 64 + static_cast<unsigned>(r * u_rs + 8 * (e & 7)));
+        }
+    }
     __syncthreads();
 #pragma unroll
-    for (int h = 0; h < HS; ++h)
-      if (KB + h < hpg) write_rows<8>(stg0 + h * 4096, duc + (KB + h) * 64 + s0 * u_rs, u_rs, qlim - s0, tid);
+    for (int h = 0; h < HS; ++h) {
+      if (KB + h >= hpg) continue;
+      bf16* rows = duc + (KB + h) * 64 + s0 * u_rs;
+      if constexpr (ADD) write_rows_add(stg0 + h * 4096, add[h], rows, u_rs, qlim - s0, tid);
+      else write_rows<8>(stg0 + h * 4096, rows, u_rs, qlim - s0, tid);
+    }
     if constexpr (last) write_rows<RCB>(stg1, dBc + s0 * act_rs, act_rs, qlim - s0, tid);
     // the next pass' first DMA goes into these buffers
     if constexpr (!last) __syncthreads();
@@ -1122,11 +1168,13 @@ __global__ __launch_bounds__(256, 3) void ssd_bwd_tgt_kernel(
 // The host pass leaves the stubs of ssd_bwd_src_kernel undefined when it only
 // meets them through a launch (its device lambdas are not substituted there);
 // explicit instantiation makes it emit them.
-#define SA_SRC_INST(NK, HS, PLAN)                                                                \
-  template __global__ void ssd_bwd_src_kernel<NK, HS, PLAN>(                                     \
+#define SA_SRC_INST_ADD(NK, HS, PLAN, ADD)                                                       \
+  template __global__ void ssd_bwd_src_kernel<NK, HS, PLAN, ADD>(                                \
       const bf16*, const bf16*, const bf16*, const bf16*, const float*, const float*,            \
-      const bf16*, const int64_t*, bf16*, bf16*, bf16*, float*, float*, float*, float*,          \
-      SsdDims, int);
+      const bf16*, const int64_t*, const bf16*, bf16*, bf16*, bf16*, float*, float*, float*,     \
+      float*, SsdDims, int);
+#define SA_SRC_INST(NK, HS, PLAN)                                                                \
+  SA_SRC_INST_ADD(NK, HS, PLAN, false) SA_SRC_INST_ADD(NK, HS, PLAN, true)
 SA_SRC_INST(4, 1, kPlanOne)
 SA_SRC_INST(4, 2, kPlanOne)
 SA_SRC_INST(4, 2, kPlanTwo)
@@ -1136,6 +1184,7 @@ SA_SRC_INST(2, 2, kPlanOne)
 SA_SRC_INST(2, 2, kPlanTwo)
 SA_SRC_INST(2, 2, kPlanMany)
 #undef SA_SRC_INST
+#undef SA_SRC_INST_ADD
 
 template <typename K>
 int raise_smem(K kernel, size_t bytes, const char* who) {
@@ -1147,27 +1196,32 @@ int raise_smem(K kernel, size_t bytes, const char* who) {
   return 0;
 }
 
+template <int NK, bool ADD>
+auto src_kernel(int hpg) {
+  return hpg == 1   ? ssd_bwd_src_kernel<NK, 1, kPlanOne, ADD>
+         : hpg <= 2 ? ssd_bwd_src_kernel<NK, 2, kPlanOne, ADD>
+         : hpg <= 4 ? ssd_bwd_src_kernel<NK, 2, kPlanTwo, ADD>
+                    : ssd_bwd_src_kernel<NK, 2, kPlanMany, ADD>;
+}
+
 template <int NK>
 int launch_fused_nk(const void* u, const void* B, const void* C, const bf16* dyp,
                     const float* dt, const float* dc, const float* states, const bf16* dSp,
-                    const int64_t* length, void* du, void* dB, void* dC, bf16* dcbp,
-                    float* ddt_part, float* xB_part, float* xC_part, float* qpart, float* rpart,
+                    const int64_t* length, const void* du_add, void* du, void* dB, void* dC,
+                    bf16* dcbp, float* ddt_part, float* xB_part, float* xC_part, float* qpart, float* rpart,
                     const SsdDims& d, bool dt_nonneg, hipStream_t s) {
   const long blocks = static_cast<long>(d.b) * d.nc * d.G * (d.Lc / 64);
   {
     // one launch walks every head of the group (in passes of two heads
     // inside each block)
     ProfScope prof_("ssd_bwd_src", s);
-    const int hpg = d.H / d.G;
-    auto kernel = hpg == 1   ? ssd_bwd_src_kernel<NK, 1, kPlanOne>
-                  : hpg <= 2 ? ssd_bwd_src_kernel<NK, 2, kPlanOne>
-                  : hpg <= 4 ? ssd_bwd_src_kernel<NK, 2, kPlanTwo>
-                             : ssd_bwd_src_kernel<NK, 2, kPlanMany>;
+    auto kernel = du_add ? src_kernel<NK, true>(d.H / d.G) : src_kernel<NK, false>(d.H / d.G);
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s,
                        static_cast<const bf16*>(u), static_cast<const bf16*>(B),
                        static_cast<const bf16*>(C), dyp, dt, dc, dSp, length,
-                       static_cast<bf16*>(du), static_cast<bf16*>(dB), dcbp, ddt_part, xB_part,
-                       qpart, rpart, d, dt_nonneg ? 1 : 0);
+                       static_cast<const bf16*>(du_add), static_cast<bf16*>(du),
+                       static_cast<bf16*>(dB), dcbp, ddt_part, xB_part, qpart, rpart, d,
+                       dt_nonneg ? 1 : 0);
     SA_CHECK_LAUNCH("ssd_bwd_src");
   }
   {
@@ -1184,13 +1238,13 @@ int launch_fused_nk(const void* u, const void* B, const void* C, const bf16* dyp
 
 int launch_ssd_bwd_fused(const void* u, const void* B, const void* C, const bf16* dyp,
                          const float* dt, const float* dc, const float* states, const bf16* dSp,
-                         const int64_t* length, void* du, void* dB, void* dC, bf16* dcbp,
-                         float* ddt_part, float* xB_part, float* xC_part, float* qpart,
+                         const int64_t* length, const void* du_add, void* du, void* dB, void* dC,
+                         bf16* dcbp, float* ddt_part, float* xB_part, float* xC_part, float* qpart,
                          float* rpart, const SsdDims& d, bool dt_nonneg, hipStream_t s) {
   if (d.N == 64)
-    return launch_fused_nk<2>(u, B, C, dyp, dt, dc, states, dSp, length, du, dB, dC, dcbp,
+    return launch_fused_nk<2>(u, B, C, dyp, dt, dc, states, dSp, length, du_add, du, dB, dC, dcbp,
                               ddt_part, xB_part, xC_part, qpart, rpart, d, dt_nonneg, s);
-  return launch_fused_nk<4>(u, B, C, dyp, dt, dc, states, dSp, length, du, dB, dC, dcbp,
+  return launch_fused_nk<4>(u, B, C, dyp, dt, dc, states, dSp, length, du_add, du, dB, dC, dcbp,
                             ddt_part, xB_part, xC_part, qpart, rpart, d, dt_nonneg, s);
 }
 

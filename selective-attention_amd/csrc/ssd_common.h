@@ -128,14 +128,15 @@ int launch_chunk_outer(const void* a, const void* b, const float* dt, const floa
 // ssd_bwd_fused.hip.  dyp: dy as bf16 hi + lo planes [b][nc][G][Lc/64][H/G]
 // [2][64][64]; dSp: dS as hi + lo planes [b][nc][H][2][64][N]; dcbp: dCB^T
 // planes [b][nc][G][Lc/64][Lc/64][2][64][64].  dt_nonneg: every dt is >= 0
-// (delta_min >= 0), so each head's dc is monotone within a chunk
+// (delta_min >= 0), so each head's dc is monotone within a chunk.  du_add (or
+// null): a tensor like du, 16-byte aligned, added to it where it is stored
 bool ssd_bwd_fused_shape_ok(const SsdDims& d);
 bool ssd_bwd_fused_ok(const SsdDims& d, const void* u, const void* B, const void* C,
                       const void* dy);
 int launch_ssd_bwd_fused(const void* u, const void* B, const void* C, const bf16* dyp,
                          const float* dt, const float* dc, const float* states, const bf16* dSp,
-                         const int64_t* length, void* du, void* dB, void* dC, bf16* dcbp,
-                         float* ddt_part, float* xB_part, float* xC_part, float* qpart,
+                         const int64_t* length, const void* du_add, void* du, void* dB, void* dC,
+                         bf16* dcbp, float* ddt_part, float* xB_part, float* xC_part, float* qpart,
                          float* rpart, const SsdDims& d, bool dt_nonneg,
                          hipStream_t s);
 

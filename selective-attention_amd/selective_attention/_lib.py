@@ -68,6 +68,9 @@ SIGNATURES: dict[str, list] = {
     "sa_ssd_bwd": [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                    _i, _i, _i, _i, _i, _i, _i, _i, _f, _f, _i,
                    _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
+    "sa_ssd_bwd_add": [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                       _i, _i, _i, _i, _i, _i, _i, _i, _f, _f, _i, _vp,
+                       _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
     "sa_ssm_conv_fwd": [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp],
     "sa_ssm_conv_bwd_workspace_size": [_i, _i, _i, _i],
     "sa_ssm_conv_bwd": [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp,

@@ -147,13 +147,14 @@ def gated_supported(dtype: torch.dtype, head_dim: int, state_dim: int) -> bool:
 
 def ssd_scan_backward(u, A, B, C, delta_raw, delta_bias, h_init, y_grad, h_last_grad, length,
                       chunk_size, use_delta_softplus=True, delta_limit=(0.0, float("inf")),
-                      is_causal=True, saved=None):
+                      is_causal=True, saved=None, du_add=None):
     """
     Args: as ssd_scan_forward, plus
         y_grad: (batch_size, seq_len, num_heads, head_dim) or None
         h_last_grad: (batch_size, num_heads, head_dim, state_dim) or None
         saved: (dt, dc, states) returned by ssd_scan_forward(return_saved=True);
                recomputed when None
+        du_add: tensor like u or None, added to the gradient of u
 
     Returns:
         u_grad, A_grad, B_grad, C_grad, delta_raw_grad, delta_bias_grad, h_init_grad
@@ -188,6 +189,8 @@ def ssd_scan_backward(u, A, B, C, delta_raw, delta_bias, h_init, y_grad, h_last_
     dA = torch.empty((H,), dtype=f32, device=dev)
     dbias = None if delta_bias is None else torch.empty((H,), dtype=f32, device=dev)
     dh0 = None if h_init is None else torch.empty((b, H, P, N), dtype=f32, device=dev)
+    if du_add is not None:
+        du_add = as_dtype(du_add, u.dtype).contiguous()
     if L == 0:
         du.zero_(); dB.zero_(); dC.zero_(); ddr.zero_(); dA.zero_()
         if dbias is not None:
@@ -202,12 +205,12 @@ def ssd_scan_backward(u, A, B, C, delta_raw, delta_bias, h_init, y_grad, h_last_
         ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev)
         lo, hi = limits(delta_limit)
         _lib.call(
-            "sa_ssd_bwd", code, _lib.ptr(u), _lib.ptr(A32), _lib.ptr(B), _lib.ptr(C),
+            "sa_ssd_bwd_add", code, _lib.ptr(u), _lib.ptr(A32), _lib.ptr(B), _lib.ptr(C),
             _lib.ptr(delta_raw), _lib.ptr(bias32), _lib.ptr(length), _lib.ptr(dy),
             _lib.ptr(dh_last), _lib.ptr(dt), _lib.ptr(dc), _lib.ptr(states),
             b, L, H, P, G, N, int(chunk_size), 1 if use_delta_softplus else 0, lo, hi,
             0 if h_init is None else 1,
-            _lib.ptr(du), _lib.ptr(dA), _lib.ptr(dB), _lib.ptr(dC), _lib.ptr(ddr),
+            _lib.ptr(du_add), _lib.ptr(du), _lib.ptr(dA), _lib.ptr(dB), _lib.ptr(dC), _lib.ptr(ddr),
             _lib.ptr(dbias), _lib.ptr(dh0), _lib.ptr(ws), nbytes, _lib.stream_of(u))
     return (as_dtype(du, dtypes["u"]), as_dtype(dA, dtypes["A"]), as_dtype(dB, dtypes["B"]),
             as_dtype(dC, dtypes["C"]), as_dtype(ddr, dtypes["delta_raw"]),

@@ -191,8 +191,7 @@ class SSDScanGatedFn(torch.autograd.Function):
             u.reshape(*u.shape[:2], -1), D, gate.reshape(*u.shape[:2], -1), y_is_yd=ctx.fused)
         grads = ssd_scan_backward(u, A, B, C, delta_raw, delta_bias, h_init, dy.view(u.shape),
                                   h_last_grad, length, chunk_size, sp, limit, True,
-                                  saved=(dt, dc, states))
+                                  saved=(dt, dc, states), du_add=d_skip.view(u.shape))
         du, dA, dB, dC, ddr, dbias, dh0 = grads
-        du = du + d_skip.view(u.shape)
         return (du, dA, dB, dC, ddr, dbias, dh0, None, None, None, None,
                 dD.to(D.dtype), dgate.view(u.shape).to(gate.dtype))
