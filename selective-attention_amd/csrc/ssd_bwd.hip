@@ -754,12 +754,12 @@ __device__ __forceinline__ F block_sum(F v, F* wtot) {
 // first M loads are issued together (clamped to a valid k) before any is
 // used; a loop that adds each load before the next is issued waits a memory
 // round trip per term
-template <int M>
-__device__ __forceinline__ float sum_parts(const float* base, long stride, int n) {   // n >= 1
+template <int M, typename F = float>
+__device__ __forceinline__ F sum_parts(const float* base, long stride, int n) {   // n >= 1
   float v[M];
 #pragma unroll
   for (int k = 0; k < M; ++k) v[k] = base[static_cast<long>(min(k, n - 1)) * stride];
-  float s = 0.f;
+  F s = 0;
 #pragma unroll
   for (int k = 0; k < M; ++k) s += k < n ? v[k] : 0.f;
   for (int k = M; k < n; ++k) s += base[static_cast<long>(k) * stride];
@@ -795,30 +795,30 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(
   for (int k = threadIdx.x; k < per_bh; k += 256) ddc += ddc_part[bhc * per_bh + k];
   // loads from clamped (valid) positions, unconditionally, so that they are
   // all in flight together; positions past Lc, qlim or lim are masked after
-  float qr[PER], xb[PER], zv[PER], dtv[PER], ddtd[PER];
-  Acc xc[PER];
+  float zv[PER], dtv[PER];
+  Acc qr[PER], xb[PER], xc[PER], ddtd[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int t = tb + j;
     const int tl = min(t, d.Lc - 1), tq = min(t, qlim - 1);
     // column sums: partials of the row tiles k >= t / 64 (qlower), or of every one
     const int q0 = qlower ? tl / 64 : 0;
-    const float q = sum_parts<4>(qpart + (bhc * ttiles + q0) * d.Lc + tl, d.Lc, ttiles - q0);
-    const float x1 = sum_parts<2>(xB_part + bhc * ntiles * d.Lc + tl, d.Lc, ntiles);
-    const float x2 = sum_parts<2>(xC_part + bhc * xctiles * d.Lc + tl, d.Lc, xctiles);
+    const Acc q = sum_parts<4, Acc>(qpart + (bhc * ttiles + q0) * d.Lc + tl, d.Lc, ttiles - q0);
+    const Acc x1 = sum_parts<2, Acc>(xB_part + bhc * ntiles * d.Lc + tl, d.Lc, ntiles);
+    const Acc x2 = sum_parts<2, Acc>(xC_part + bhc * xctiles * d.Lc + tl, d.Lc, xctiles);
     // row sums: partials of the source tiles k <= t / 64 (rtiles == 1: complete)
-    const float r = sum_parts<4>(rsum + bhc * rtiles * d.Lc + tl, d.Lc, min(rtiles, tl / 64 + 1));
+    const Acc r = sum_parts<4, Acc>(rsum + bhc * rtiles * d.Lc + tl, d.Lc, min(rtiles, tl / 64 + 1));
     const long off = (static_cast<long>(b) * d.L + static_cast<long>(c) * d.Lc + tq) * d.H + h;
     const float z = load_f32(delta_raw + off);
     const float dtt = dt[crow + tl];
-    const float dd = sum_parts<2>(ddt_part + bhc * ptiles * d.Lc + tl, d.Lc, ptiles);
+    const Acc dd = sum_parts<2, Acc>(ddt_part + bhc * ptiles * d.Lc + tl, d.Lc, ptiles);
     const bool tv = t < d.Lc, tin = tv && t < lim;
-    qr[j] = tv ? q - r : 0.f;
-    xb[j] = tv && t < lim - 1 ? x1 : 0.f;
-    xc[j] = tin ? x2 : 0.f;
+    qr[j] = tv ? q - r : Acc(0);
+    xb[j] = tv && t < lim - 1 ? x1 : Acc(0);
+    xc[j] = tin ? x2 : Acc(0);
     zv[j] = tin ? z : 0.f;
     dtv[j] = tin ? dtt : 0.f;
-    ddtd[j] = tin ? dd : 0.f;
+    ddtd[j] = tin ? dd : Acc(0);
   }
   // ddc_last of this chunk (sum of the state-passing partials)
   ddc = block_sum(ddc, wtot);
@@ -848,18 +848,18 @@ __global__ __launch_bounds__(256) void chunk_cumsum_bwd_kernel(
       rc += xc[j];
       if (t < qlim) {
         const long off = (static_cast<long>(b) * d.L + static_cast<long>(c) * d.Lc + t) * d.H + h;
-        float g = 0.f;
+        Acc g = 0;
         if (t < lim) {
           const Acc da = dA_intra + dA_B + dA_C;
           const float z = zv[j] + bias;
           const float sp = softplus ? softplus20(z) : z;
-          g = static_cast<float>(da * a + ddtd[j]);
-          if (sp < lo || sp > hi) g = 0.f;
+          g = da * a + ddtd[j];
+          if (sp < lo || sp > hi) g = 0;
           if (softplus && z <= 20.0f) g *= sigmoidf_acc(z);
           dA_loc += da * dtv[j];
           db_loc += g;
         }
-        ddelta_raw[off] = from_f32<T>(g);
+        ddelta_raw[off] = from_f32<T>(static_cast<float>(g));
       }
     }
   }
