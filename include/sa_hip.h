@@ -130,17 +130,24 @@ int sa_ssd_bwd(int dtype, const void* u, const float* A, const void* B, const vo
                void* ddelta_raw, float* ddelta_bias, float* dh_init, void* workspace,
                size_t workspace_bytes, void* stream);
 
-/* sa_ssd_bwd with du + du_add in place of du: du_add (or NULL) a tensor of the
- * shape and dtype of du (the skip path's gradient), added after du is rounded
- * to that dtype. */
-int sa_ssd_bwd_add(int dtype, const void* u, const float* A, const void* B, const void* C,
-                   const void* delta_raw, const float* delta_bias, const int64_t* length,
-                   const float* dy, const float* dh_last, const float* dt, const float* dc,
-                   const float* states, int batch, int seqlen, int num_heads, int head_dim,
-                   int num_groups, int state_dim, int chunk_size, int use_softplus,
-                   float delta_min, float delta_max, int has_h_init, const void* du_add, void* du,
-                   float* dA, void* dB, void* dC, void* ddelta_raw, float* ddelta_bias,
-                   float* dh_init, void* workspace, size_t workspace_bytes, void* stream);
+/* Backward of sa_ssd_fwd_gated, bfloat16: dout, yd (as that call saved it),
+ * gate and u (batch, seqlen, num_heads, 64), D (num_heads * 64) float32; dy =
+ * dout silu(gate) is formed inside.  Adds the skip gradient D dy to du and
+ * writes dD and dgate; the other arguments are sa_ssd_bwd's.  head_dim 64,
+ * state_dim 64 or 128, chunk_size a multiple of 64, operands 16-byte aligned;
+ * the workspace size is 0 for shapes and dtypes outside these. */
+size_t sa_ssd_bwd_gated_workspace_size(int dtype, int batch, int seqlen, int num_heads,
+                                       int head_dim, int num_groups, int state_dim,
+                                       int chunk_size);
+int sa_ssd_bwd_gated(const void* u, const float* A, const void* B, const void* C,
+                     const void* delta_raw, const float* delta_bias, const int64_t* length,
+                     const void* dout, const void* yd, const float* D, const void* gate,
+                     const float* dh_last, const float* dt, const float* dc, const float* states,
+                     int batch, int seqlen, int num_heads, int head_dim, int num_groups,
+                     int state_dim, int chunk_size, int use_softplus, float delta_min,
+                     float delta_max, int has_h_init, void* du, float* dA, void* dB, void* dC,
+                     void* ddelta_raw, float* ddelta_bias, float* dh_init, float* dD, void* dgate,
+                     void* workspace, size_t workspace_bytes, void* stream);
 
 /*
  * Varlen block-sparse causal self-attention (prefill), bfloat16.  No

@@ -891,18 +891,6 @@ __global__ __launch_bounds__(256) void param_grad_reduce_kernel(const float* __r
   }
 }
 
-// du += add, element by element (each thread four, 256 apart)
-template <typename T>
-__global__ __launch_bounds__(256) void du_add_kernel(const T* __restrict__ add, long n,
-                                                     T* __restrict__ du) {
-  const long i0 = static_cast<long>(blockIdx.x) * 1024 + threadIdx.x;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const long i = i0 + 256 * j;
-    if (i < n) st(du + i, load_f32(du + i) + load_f32(add + i));
-  }
-}
-
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -936,8 +924,8 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
                  const void* delta_raw_, const float* bias, const int64_t* length,
                  const float* dy, const float* dh_last, const float* dt, const float* dc,
                  const float* states, const SsdDims& d, int sp, float lo, float hi, int has_init,
-                 const void* du_add, void* du_, float* dA, void* dB_, void* dC_, void* ddelta_,
-                 float* dbias, float* dh_init, unsigned char* ws, hipStream_t s) {
+                 const GateBwd* gb, void* du_, float* dA, void* dB_, void* dC_, void* ddelta_, float* dbias,
+                 float* dh_init, unsigned char* ws, hipStream_t s) {
   const T* u = static_cast<const T*>(u_);
   const T* Bm = static_cast<const T*>(B_);
   const T* Cm = static_cast<const T*>(C_);
@@ -968,8 +956,11 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
   bf16* dyp = reinterpret_cast<bf16*>(ws + w.dyp);
   bf16* dSp = reinterpret_cast<bf16*>(ws + w.dSp);
   bf16* dcbp = reinterpret_cast<bf16*>(ws + w.dcbp);
+  SA_CHECK_ARG(!gb || fused, "sa_ssd_bwd_gated: needs 16-byte aligned operands");
   // 1. dH_intra -> dS buffer (the fused path also writes dy as hi + lo planes)
-  if (fused) {
+  if (gb) {
+    if ((rc = launch_dstate_gate(*gb, C_, dt, dc, length, dS, dyp, d, s))) return rc;
+  } else if (fused) {
     if ((rc = launch_dstate_planes(dy, C_, dt, dc, length, dS, dyp, d, s))) return rc;
   } else if (f32) {
     if ((rc = launch_f32_outer(dy, static_cast<const float*>(C_), dt, dc, length, dS, d, 1, s)))
@@ -989,8 +980,8 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
   if (fused) {
     // 3-5 fused: du, dB, dC, decay sums
     if ((rc = launch_ssd_bwd_fused(u, Bm, Cm, dyp, dt, dc, states, dSp, length,
-                                   aligned16(du_add) ? du_add : nullptr, du_, dB_, dC_, dcbp,
-                                   ddt_part, xB_part, xC_part, qpart, rsum, d, lo >= 0.f, s)))
+                                   gb ? gb->D : nullptr, du_, dB_, dC_, dcbp, ddt_part, xB_part, xC_part, qpart, rsum, d,
+                                   lo >= 0.f, s)))
       return rc;
     ptiles = ntiles = qtiles = 1;
     xctiles = d.N / 64;   // x_C: one partial per 64 n (ssd_bwd_tgt block)
@@ -1040,14 +1031,6 @@ int ssd_bwd_impl(const void* u_, const float* A, const void* B_, const void* C_,
     SA_CHECK_LAUNCH("chunk_dbdc_bwd");
   }
   }
-  // du += du_add where the kernels above did not add it as they stored du
-  if (du_add && !(fused && aligned16(du_add))) {
-    const long n = static_cast<long>(d.b) * d.L * d.H * d.P;
-    ProfScope prof_("du_add", s);
-    hipLaunchKernelGGL(du_add_kernel<T>, dim3((n + 1023) / 1024), dim3(256), 0, s,
-                       static_cast<const T*>(du_add), n, static_cast<T*>(du_));
-    SA_CHECK_LAUNCH("du_add");
-  }
   // 6. decay-gradient assembly, d delta_raw, dA/dbias partials
   {
     const long blocks = bnc * d.H;
@@ -1085,16 +1068,14 @@ extern "C" size_t sa_ssd_bwd_workspace_size(int dtype, int batch, int seqlen, in
   return sa::bwd_layout(d, dtype == sa::kBF16 ? 2 : 4).total;
 }
 
-extern "C" int sa_ssd_bwd_add(int dtype, const void* u, const float* A, const void* B,
-                              const void* C, const void* delta_raw, const float* delta_bias,
-                              const int64_t* length, const float* dy, const float* dh_last,
-                              const float* dt, const float* dc, const float* states, int batch,
-                              int seqlen, int num_heads, int head_dim, int num_groups,
-                              int state_dim, int chunk_size, int use_softplus, float delta_min,
-                              float delta_max, int has_h_init, const void* du_add, void* du,
-                              float* dA, void* dB, void* dC, void* ddelta_raw, float* ddelta_bias,
-                              float* dh_init, void* workspace, size_t workspace_bytes,
-                              void* stream) {
+extern "C" int sa_ssd_bwd(int dtype, const void* u, const float* A, const void* B, const void* C,
+                          const void* delta_raw, const float* delta_bias, const int64_t* length,
+                          const float* dy, const float* dh_last, const float* dt, const float* dc,
+                          const float* states, int batch, int seqlen, int num_heads, int head_dim,
+                          int num_groups, int state_dim, int chunk_size, int use_softplus,
+                          float delta_min, float delta_max, int has_h_init, void* du, float* dA,
+                          void* dB, void* dC, void* ddelta_raw, float* ddelta_bias,
+                          float* dh_init, void* workspace, size_t workspace_bytes, void* stream) {
   sa::SsdDims d;
   int rc = sa::make_dims(batch, seqlen, num_heads, head_dim, num_groups, state_dim, chunk_size, &d,
                          "sa_ssd_bwd");
@@ -1114,24 +1095,63 @@ extern "C" int sa_ssd_bwd_add(int dtype, const void* u, const float* A, const vo
   if (dtype == sa::kF32)
     return sa::ssd_bwd_impl<float, float>(u, A, B, C, delta_raw, delta_bias, length, dy, dh_last,
                                           dt, dc, states, d, use_softplus, delta_min, delta_max,
-                                          has_h_init, du_add, du, dA, dB, dC, ddelta_raw,
-                                          ddelta_bias, dh_init, ws, s);
+                                          has_h_init, nullptr, du, dA, dB, dC, ddelta_raw, ddelta_bias,
+                                          dh_init, ws, s);
   return sa::ssd_bwd_impl<sa::bf16, sa::bf16>(u, A, B, C, delta_raw, delta_bias, length, dy,
                                               dh_last, dt, dc, states, d, use_softplus, delta_min,
-                                              delta_max, has_h_init, du_add, du, dA, dB, dC,
-                                              ddelta_raw, ddelta_bias, dh_init, ws, s);
+                                              delta_max, has_h_init, nullptr, du, dA, dB, dC, ddelta_raw,
+                                              ddelta_bias, dh_init, ws, s);
 }
 
-extern "C" int sa_ssd_bwd(int dtype, const void* u, const float* A, const void* B, const void* C,
-                          const void* delta_raw, const float* delta_bias, const int64_t* length,
-                          const float* dy, const float* dh_last, const float* dt, const float* dc,
-                          const float* states, int batch, int seqlen, int num_heads, int head_dim,
-                          int num_groups, int state_dim, int chunk_size, int use_softplus,
-                          float delta_min, float delta_max, int has_h_init, void* du, float* dA,
-                          void* dB, void* dC, void* ddelta_raw, float* ddelta_bias,
-                          float* dh_init, void* workspace, size_t workspace_bytes, void* stream) {
-  return sa_ssd_bwd_add(dtype, u, A, B, C, delta_raw, delta_bias, length, dy, dh_last, dt, dc, states,
-                        batch, seqlen, num_heads, head_dim, num_groups, state_dim, chunk_size,
-                        use_softplus, delta_min, delta_max, has_h_init, nullptr, du, dA, dB, dC,
-                        ddelta_raw, ddelta_bias, dh_init, workspace, workspace_bytes, stream);
+extern "C" size_t sa_ssd_bwd_gated_workspace_size(int dtype, int batch, int seqlen, int num_heads,
+                                                  int head_dim, int num_groups, int state_dim,
+                                                  int chunk_size) {
+  sa::SsdDims d;
+  if (sa::make_dims(batch, seqlen, num_heads, head_dim, num_groups, state_dim, chunk_size, &d,
+                    "sa_ssd_bwd_gated_workspace_size"))
+    return 0;
+  if (dtype != sa::kBF16 || !sa::ssd_bwd_fused_shape_ok(d)) return 0;
+  return sa::bwd_layout(d, 2).total + static_cast<size_t>(d.b) * d.nc * d.H * 64 * 4;
+}
+
+extern "C" int sa_ssd_bwd_gated(const void* u, const float* A, const void* B, const void* C,
+                                const void* delta_raw, const float* delta_bias,
+                                const int64_t* length, const void* dout, const void* yd,
+                                const float* D, const void* gate, const float* dh_last,
+                                const float* dt, const float* dc, const float* states, int batch,
+                                int seqlen, int num_heads, int head_dim, int num_groups,
+                                int state_dim, int chunk_size, int use_softplus, float delta_min,
+                                float delta_max, int has_h_init, void* du, float* dA, void* dB,
+                                void* dC, void* ddelta_raw, float* ddelta_bias, float* dh_init,
+                                float* dD, void* dgate, void* workspace, size_t workspace_bytes,
+                                void* stream) {
+  using sa::bf16;
+  sa::SsdDims d;
+  int rc = sa::make_dims(batch, seqlen, num_heads, head_dim, num_groups, state_dim, chunk_size, &d,
+                         "sa_ssd_bwd_gated");
+  if (rc) return rc;
+  SA_CHECK_ARG(sa::ssd_bwd_fused_shape_ok(d),
+               "sa_ssd_bwd_gated: head_dim 64, state_dim 64 or 128 and chunk_size %% 64 == 0 "
+               "required (got %d, %d, %d)", head_dim, state_dim, chunk_size);
+  SA_CHECK_ARG(u && A && B && C && delta_raw && dout && yd && D && gate && dt && dc && states &&
+                   du && dA && dB && dC && ddelta_raw && dD && dgate && workspace,
+               "sa_ssd_bwd_gated: null tensor pointer");
+  SA_CHECK_ARG(sa::aligned16(u) && sa::aligned16(B) && sa::aligned16(C) && sa::aligned16(dout) &&
+                   sa::aligned16(yd) && sa::aligned16(D) && sa::aligned16(gate) &&
+                   sa::aligned16(du) && sa::aligned16(dgate),
+               "sa_ssd_bwd_gated: needs 16-byte aligned operands");
+  const size_t need = sa_ssd_bwd_gated_workspace_size(sa::kBF16, batch, seqlen, num_heads, head_dim,
+                                                      num_groups, state_dim, chunk_size);
+  SA_CHECK_ARG(workspace_bytes >= need, "sa_ssd_bwd_gated: workspace %zu B < required %zu B",
+               workspace_bytes, need);
+  if (d.b == 0 || d.L == 0) return 0;
+  unsigned char* ws = static_cast<unsigned char*>(workspace);
+  const sa::GateBwd gb{static_cast<const bf16*>(dout), static_cast<const bf16*>(yd),
+                       static_cast<const bf16*>(u), static_cast<const bf16*>(gate), D,
+                       static_cast<bf16*>(du), static_cast<bf16*>(dgate),
+                       reinterpret_cast<float*>(ws + sa::bwd_layout(d, 2).total), dD};
+  return sa::ssd_bwd_impl<bf16, bf16>(u, A, B, C, delta_raw, delta_bias, length, nullptr, dh_last,
+                                      dt, dc, states, d, use_softplus, delta_min, delta_max,
+                                      has_h_init, &gb, du, dA, dB, dC, ddelta_raw, ddelta_bias,
+                                      dh_init, ws, static_cast<hipStream_t>(stream));
 }

@@ -133,21 +133,23 @@ __device__ __forceinline__ void write_rows(const bf16* t, bf16* g, int grs, int 
   }
 }
 
-// the same for a 64 x 64 tile plus `add` (this thread's 16 bytes of each row
-// it writes), summed in fp32 and rounded
-__device__ __forceinline__ uint32_t add_bf16x2(uint32_t a, uint32_t b) {
-  return pack_bf16x2(bf16lo_to_f32(a) + bf16lo_to_f32(b), bf16hi_to_f32(a) + bf16hi_to_f32(b));
+// the same for a 64 x 64 tile plus D dy (Dv: D of this thread's 8 columns;
+// hi, lo: dy's planes at the 16 bytes of each row it writes)
+__device__ __forceinline__ uint32_t add_skip(uint32_t v, uint32_t hi, uint32_t lo, float d0, float d1) {
+  return pack_bf16x2(bf16lo_to_f32(v) + d0 * (bf16lo_to_f32(hi) + bf16lo_to_f32(lo)),
+                     bf16hi_to_f32(v) + d1 * (bf16hi_to_f32(hi) + bf16hi_to_f32(lo)));
 }
-__device__ __forceinline__ void write_rows_add(const bf16* t, const uint4 (&add)[2], bf16* g, int grs,
-                                               int rows_valid, int tid) {
+__device__ __forceinline__ void write_rows_skip(const bf16* t, const float* Dv, const uint4 (&hi)[2],
+                                                const uint4 (&lo)[2], bf16* g, int grs,
+                                                int rows_valid, int tid) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int e = tid + 256 * i, r = e / 8, c = e % 8;
     const uint4 v = *reinterpret_cast<const uint4*>(t + r * 64 + 8 * (c ^ (r & 7)));
     if (r < rows_valid)
       *reinterpret_cast<uint4*>(g + static_cast<unsigned>(r * grs + 8 * c)) =
-          uint4{add_bf16x2(v.x, add[i].x), add_bf16x2(v.y, add[i].y), add_bf16x2(v.z, add[i].z),
-                add_bf16x2(v.w, add[i].w)};
+          uint4{add_skip(v.x, hi[i].x, lo[i].x, Dv[0], Dv[1]), add_skip(v.y, hi[i].y, lo[i].y, Dv[2], Dv[3]),
+                add_skip(v.z, hi[i].z, lo[i].z, Dv[4], Dv[5]), add_skip(v.w, hi[i].w, lo[i].w, Dv[6], Dv[7])};
   }
 }
 
@@ -269,12 +271,13 @@ __device__ __forceinline__ int opaque(int v) {
 // Passes other than the last hold their heads' u rows in registers; every
 // pass holds the source row's B.
 //
-// ADD: du_add's rows (the skip path's gradient) are read a barrier ahead of
-// the du rows and added as these are stored, du rounded first, as du + du_add
-// of the two tensors would be.  A separate add reads and writes du once more:
-// the training step of an 8 x 4096-token, 16-head block 775 -> 758 us.  Its
-// own instance, as the pointer and the branch alone cost the scan without it
-// 1 % (1151 -> 1163 us at 8 x 4096 tokens, 32 heads).
+// SKIP (the gated block): du gets D dy added as its rows are stored, from dy's
+// planes of the strip, so that neither D dy nor a second pass over du goes to
+// memory; rows past the length are the dstate kernel's.  Reading the planes
+// costs 31 us of 276 (8 x 4096 tokens, 16 heads), a separate add of a stored
+// D dy took 32 and its store 13.  Loading them before du is staged instead
+// gained nothing (672 us for the whole block both ways).  An instance of its
+// own: a pointer and a branch alone cost the scan without the term 1 %.
 // ---------------------------------------------------------------------------
 template <int NK>
 struct SrcSmem {
@@ -287,12 +290,12 @@ enum SrcMode { kSrcOnly = 0, kSrcFirst = 1, kSrcMiddle = 2, kSrcLast = 3 };
 // pass plans: one pass (at most HS heads), two passes, more than two
 enum SrcPlan { kPlanOne = 0, kPlanTwo = 1, kPlanMany = 2 };
 
-template <int NK, int HS, int PLAN, bool ADD>
+template <int NK, int HS, int PLAN, bool SKIP>
 __global__ __launch_bounds__(256, 2) void ssd_bwd_src_kernel(
     const bf16* __restrict__ u, const bf16* __restrict__ Bm, const bf16* __restrict__ Cm,
     const bf16* __restrict__ dyp, const float* __restrict__ dt, const float* __restrict__ dc,
     const bf16* __restrict__ dSp, const int64_t* __restrict__ length,
-    const bf16* __restrict__ du_add, bf16* __restrict__ du, bf16* __restrict__ dB,
+    const float* __restrict__ skip_D, bf16* __restrict__ du, bf16* __restrict__ dB,
     bf16* __restrict__ dcbp, float* __restrict__ ddt_part,
     float* __restrict__ xB_part, float* __restrict__ qpart, float* __restrict__ rpart,
     SsdDims d, int mono) {
@@ -352,7 +355,6 @@ __global__ __launch_bounds__(256, 2) void ssd_bwd_src_kernel(
   const float* dcc = dc + bhc0 * d.Lc;
   const float* dtc = dt + bhc0 * d.Lc;
   bf16* duc = du + tok0 * u_rs + h0 * 64;
-  const bf16* addc = ADD ? du_add + tok0 * u_rs + h0 * 64 : nullptr;
   bf16* dBc = dB + tok0 * act_rs + static_cast<long>(g) * N;
   float* ddtc = ddt_part + bhc0 * d.Lc;
   float* xBc = xB_part + bhc0 * d.Lc;
@@ -363,11 +365,8 @@ __global__ __launch_bounds__(256, 2) void ssd_bwd_src_kernel(
   if (s0 >= lim) {   // the strip is past the length: zero outputs and partials
     for (int e = tid; e < 64 * hpg * 8; e += 256) {
       const int row = e / (hpg * 8), col8 = e % (hpg * 8);
-      if (s0 + row < qlim) {
-        const unsigned o = static_cast<unsigned>((s0 + row) * u_rs + 8 * col8);
-        *reinterpret_cast<uint4*>(duc + o) =
-            ADD ? *reinterpret_cast<const uint4*>(addc + o) : uint4{0u, 0u, 0u, 0u};
-      }
+      if (!SKIP && s0 + row < qlim)
+        *reinterpret_cast<uint4*>(duc + static_cast<unsigned>((s0 + row) * u_rs + 8 * col8)) = uint4{0u, 0u, 0u, 0u};
     }
     for (int e = tid; e < 64 * (N / 8); e += 256) {
       const int row = e / (N / 8), col8 = e % (N / 8);
@@ -866,25 +865,34 @@ __global__ __launch_bounds__(256, 2) void ssd_bwd_src_kernel(
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) stage_out8<RCB>(stg1, sl, 16 * nt + 4 * lg, pack4_bf16(dBT[nt]));
     }
-    // the rows to add to du, on their way across the barrier
-    [[maybe_unused]] uint4 add[HS][2];
-    if constexpr (ADD) {
+    // dy's planes of the strip for the skip term, on their way across the barrier
+    [[maybe_unused]] uint4 yh[HS][2], yl[HS][2];
+    if constexpr (SKIP) {
 #pragma unroll
-      for (int h = 0; h < HS; ++h)
+      for (int h = 0; h < HS; ++h) {
+        const bf16* pl = dyp + ((bcg * stiles + S) * hpg + min(KB + h, hpg - 1)) * 8192L + 8 * tid;
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-          const int e = tid + 256 * i, r = min(s0 + (e >> 3), qlim - 1);
-          add[h][i] = *reinterpret_cast<const uint4*>(
-              addc + min(KB + h, hpg - 1) * 64 + static_cast<unsigned>(r * u_rs + 8 * (e & 7)));
+          yh[h][i] = *reinterpret_cast<const uint4*>(pl + 2048 * i);
+          yl[h][i] = *reinterpret_cast<const uint4*>(pl + 4096 + 2048 * i);
         }
+      }
     }
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < HS; ++h) {
       if (KB + h >= hpg) continue;
       bf16* rows = duc + (KB + h) * 64 + s0 * u_rs;
-      if constexpr (ADD) write_rows_add(stg0 + h * 4096, add[h], rows, u_rs, qlim - s0, tid);
-      else write_rows<8>(stg0 + h * 4096, rows, u_rs, qlim - s0, tid);
+      if constexpr (SKIP) {
+        float Dv[8];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          *reinterpret_cast<float4*>(Dv + 4 * i) =
+              *reinterpret_cast<const float4*>(skip_D + (h0 + KB + h) * 64 + 8 * (tid & 7) + 4 * i);
+        write_rows_skip(stg0 + h * 4096, Dv, yh[h], yl[h], rows, u_rs, lim - s0, tid);
+      } else {
+        write_rows<8>(stg0 + h * 4096, rows, u_rs, qlim - s0, tid);
+      }
     }
     if constexpr (last) write_rows<RCB>(stg1, dBc + s0 * act_rs, act_rs, qlim - s0, tid);
     // the next pass' first DMA goes into these buffers
@@ -1168,13 +1176,13 @@ __global__ __launch_bounds__(256, 3) void ssd_bwd_tgt_kernel(
 // The host pass leaves the stubs of ssd_bwd_src_kernel undefined when it only
 // meets them through a launch (its device lambdas are not substituted there);
 // explicit instantiation makes it emit them.
-#define SA_SRC_INST_ADD(NK, HS, PLAN, ADD)                                                       \
-  template __global__ void ssd_bwd_src_kernel<NK, HS, PLAN, ADD>(                                \
+#define SA_SRC_INST_SKIP(NK, HS, PLAN, SKIP)                                                     \
+  template __global__ void ssd_bwd_src_kernel<NK, HS, PLAN, SKIP>(                               \
       const bf16*, const bf16*, const bf16*, const bf16*, const float*, const float*,            \
-      const bf16*, const int64_t*, const bf16*, bf16*, bf16*, bf16*, float*, float*, float*,     \
+      const bf16*, const int64_t*, const float*, bf16*, bf16*, bf16*, float*, float*, float*,    \
       float*, SsdDims, int);
 #define SA_SRC_INST(NK, HS, PLAN)                                                                \
-  SA_SRC_INST_ADD(NK, HS, PLAN, false) SA_SRC_INST_ADD(NK, HS, PLAN, true)
+  SA_SRC_INST_SKIP(NK, HS, PLAN, false) SA_SRC_INST_SKIP(NK, HS, PLAN, true)
 SA_SRC_INST(4, 1, kPlanOne)
 SA_SRC_INST(4, 2, kPlanOne)
 SA_SRC_INST(4, 2, kPlanTwo)
@@ -1184,7 +1192,7 @@ SA_SRC_INST(2, 2, kPlanOne)
 SA_SRC_INST(2, 2, kPlanTwo)
 SA_SRC_INST(2, 2, kPlanMany)
 #undef SA_SRC_INST
-#undef SA_SRC_INST_ADD
+#undef SA_SRC_INST_SKIP
 
 template <typename K>
 int raise_smem(K kernel, size_t bytes, const char* who) {
@@ -1196,18 +1204,18 @@ int raise_smem(K kernel, size_t bytes, const char* who) {
   return 0;
 }
 
-template <int NK, bool ADD>
+template <int NK, bool SKIP>
 auto src_kernel(int hpg) {
-  return hpg == 1   ? ssd_bwd_src_kernel<NK, 1, kPlanOne, ADD>
-         : hpg <= 2 ? ssd_bwd_src_kernel<NK, 2, kPlanOne, ADD>
-         : hpg <= 4 ? ssd_bwd_src_kernel<NK, 2, kPlanTwo, ADD>
-                    : ssd_bwd_src_kernel<NK, 2, kPlanMany, ADD>;
+  return hpg == 1   ? ssd_bwd_src_kernel<NK, 1, kPlanOne, SKIP>
+         : hpg <= 2 ? ssd_bwd_src_kernel<NK, 2, kPlanOne, SKIP>
+         : hpg <= 4 ? ssd_bwd_src_kernel<NK, 2, kPlanTwo, SKIP>
+                    : ssd_bwd_src_kernel<NK, 2, kPlanMany, SKIP>;
 }
 
 template <int NK>
 int launch_fused_nk(const void* u, const void* B, const void* C, const bf16* dyp,
                     const float* dt, const float* dc, const float* states, const bf16* dSp,
-                    const int64_t* length, const void* du_add, void* du, void* dB, void* dC,
+                    const int64_t* length, const float* skip_D, void* du, void* dB, void* dC,
                     bf16* dcbp, float* ddt_part, float* xB_part, float* xC_part, float* qpart, float* rpart,
                     const SsdDims& d, bool dt_nonneg, hipStream_t s) {
   const long blocks = static_cast<long>(d.b) * d.nc * d.G * (d.Lc / 64);
@@ -1215,13 +1223,12 @@ int launch_fused_nk(const void* u, const void* B, const void* C, const bf16* dyp
     // one launch walks every head of the group (in passes of two heads
     // inside each block)
     ProfScope prof_("ssd_bwd_src", s);
-    auto kernel = du_add ? src_kernel<NK, true>(d.H / d.G) : src_kernel<NK, false>(d.H / d.G);
+    auto kernel = skip_D ? src_kernel<NK, true>(d.H / d.G) : src_kernel<NK, false>(d.H / d.G);
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(256), 0, s,
                        static_cast<const bf16*>(u), static_cast<const bf16*>(B),
-                       static_cast<const bf16*>(C), dyp, dt, dc, dSp, length,
-                       static_cast<const bf16*>(du_add), static_cast<bf16*>(du),
-                       static_cast<bf16*>(dB), dcbp, ddt_part, xB_part, qpart, rpart, d,
-                       dt_nonneg ? 1 : 0);
+                       static_cast<const bf16*>(C), dyp, dt, dc, dSp, length, skip_D,
+                       static_cast<bf16*>(du), static_cast<bf16*>(dB), dcbp, ddt_part, xB_part,
+                       qpart, rpart, d, dt_nonneg ? 1 : 0);
     SA_CHECK_LAUNCH("ssd_bwd_src");
   }
   {
@@ -1238,13 +1245,13 @@ int launch_fused_nk(const void* u, const void* B, const void* C, const bf16* dyp
 
 int launch_ssd_bwd_fused(const void* u, const void* B, const void* C, const bf16* dyp,
                          const float* dt, const float* dc, const float* states, const bf16* dSp,
-                         const int64_t* length, const void* du_add, void* du, void* dB, void* dC,
+                         const int64_t* length, const float* skip_D, void* du, void* dB, void* dC,
                          bf16* dcbp, float* ddt_part, float* xB_part, float* xC_part, float* qpart,
                          float* rpart, const SsdDims& d, bool dt_nonneg, hipStream_t s) {
   if (d.N == 64)
-    return launch_fused_nk<2>(u, B, C, dyp, dt, dc, states, dSp, length, du_add, du, dB, dC, dcbp,
+    return launch_fused_nk<2>(u, B, C, dyp, dt, dc, states, dSp, length, skip_D, du, dB, dC, dcbp,
                               ddt_part, xB_part, xC_part, qpart, rpart, d, dt_nonneg, s);
-  return launch_fused_nk<4>(u, B, C, dyp, dt, dc, states, dSp, length, du_add, du, dB, dC, dcbp,
+  return launch_fused_nk<4>(u, B, C, dyp, dt, dc, states, dSp, length, skip_D, du, dB, dC, dcbp,
                             ddt_part, xB_part, xC_part, qpart, rpart, d, dt_nonneg, s);
 }
 

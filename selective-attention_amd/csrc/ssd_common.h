@@ -117,6 +117,15 @@ inline int make_dims(int b, int L, int H, int P, int G, int N, int Lc, SsdDims* 
   return 0;
 }
 
+// the gated block's backward (out = (y + D u) silu(gate)): yd = y + D u as the
+// forward saved it, u, gate and dout (b, L, H, 64) bf16, D (H * 64)
+struct GateBwd {
+  const bf16 *dout, *yd, *u, *gate;
+  const float* D;
+  bf16 *du, *dgate;     // du: only the rows at t >= length (the scan adds nothing there)
+  float *dD_part, *dD;  // dD_part [b * nc][H * 64]
+};
+
 // launchers shared between the forward and backward translation units
 template <typename T>
 int launch_chunk_cumsum(const void* delta_raw, const float* A, const float* bias,
@@ -133,14 +142,15 @@ int launch_chunk_outer(const void* a, const void* b, const float* dt, const floa
 // ssd_bwd_fused.hip.  dyp: dy as bf16 hi + lo planes [b][nc][G][Lc/64][H/G]
 // [2][64][64]; dSp: dS as hi + lo planes [b][nc][H][2][64][N]; dcbp: dCB^T
 // planes [b][nc][G][Lc/64][Lc/64][2][64][64].  dt_nonneg: every dt is >= 0
-// (delta_min >= 0), so each head's dc is monotone within a chunk.  du_add (or
-// null): a tensor like du, 16-byte aligned, added to it where it is stored
+// (delta_min >= 0), so each head's dc is monotone within a chunk.  skip_D (or
+// null): the gated block's D; du gets D dy added at t < length and is left
+// unwritten from there on
 bool ssd_bwd_fused_shape_ok(const SsdDims& d);
 bool ssd_bwd_fused_ok(const SsdDims& d, const void* u, const void* B, const void* C,
                       const void* dy);
 int launch_ssd_bwd_fused(const void* u, const void* B, const void* C, const bf16* dyp,
                          const float* dt, const float* dc, const float* states, const bf16* dSp,
-                         const int64_t* length, const void* du_add, void* du, void* dB, void* dC,
+                         const int64_t* length, const float* skip_D, void* du, void* dB, void* dC,
                          bf16* dcbp, float* ddt_part, float* xB_part, float* xC_part, float* qpart,
                          float* rpart, const SsdDims& d, bool dt_nonneg,
                          hipStream_t s);
@@ -169,5 +179,12 @@ int launch_f32_bwd(const float* u, const float* B, const float* C, const float* 
 int launch_dstate_planes(const float* dy, const void* C, const float* dt, const float* dc,
                          const int64_t* length, float* out, bf16* dyp, const SsdDims& d,
                          hipStream_t s);
+// the same with dy = dout silu(gate) formed in the kernel, which also writes
+// dgate, the dD partials and the skip rows of du past the length
+int launch_dstate_gate(const GateBwd& gb, const void* C, const float* dt, const float* dc,
+                       const int64_t* length, float* out, bf16* dyp, const SsdDims& d,
+                       hipStream_t s);
+// out[e] = sum_p part[p][n] (ssm_io.hip)
+int launch_reduce_partials(const float* part, int np, long n, float* out, hipStream_t s);
 
 }  // namespace sa

@@ -177,6 +177,16 @@ __device__ __forceinline__ void split_scaled(uint32_t v, float sc, uint32_t& hi,
 //           dyp set (P = 64) it also writes dy (zero at t >= length) as the
 //           hi + lo bf16 planes the fused backward reads, [b][nc][G][Lc/64]
 //           [H/G][2][64][64]
+//   MODE 2: MODE 1 with dyp, for the gated block (P = 64): dy = dout
+//           silu(gate) is formed as the tile is committed, and what else the
+//           gate's backward gives is written from the same registers: dgate,
+//           dD's partial sums (one row of them per chunk) and, past the
+//           length, du = D dy (the scan's backward adds that term elsewhere).
+//           It is bound by memory: 4 bf16 reads, dgate and the planes, 470 MB
+//           at 8 x 4096 tokens, 16 heads: 96 us (4.9 TB/s) for the 186 us of
+//           a gate backward that writes fp32 dy and D dy and of MODE 1, which
+//           reads dy back; the block's forward and backward 761 -> 667 us,
+//           373 -> 337 us at the smallest sizes (two launches fewer).
 // One block per (b, chunk, head, 64-wide p tile), 4 waves; wave w computes
 // D^T[n][p] for its N/4 columns n and the 64 p.  Both operands come from
 // row-major t tiles in LDS through transpose reads: A = X^T (X = B or C) and
@@ -186,12 +196,14 @@ __device__ __forceinline__ void split_scaled(uint32_t v, float sc, uint32_t& hi,
 // previous tile's MFMAs and committed to a single LDS stage (35 KB at
 // N = 128), so three or four blocks share a CU: more resident blocks hide
 // the loads better than a second stage did (chunk states 88 -> 72-78 us).
+// MODE 2 at N = 128 holds 32 registers more of loads: two blocks a CU, where
+// three would spill 86 registers.
 // ---------------------------------------------------------------------------
 template <int NK, int MODE>
-__global__ __launch_bounds__(256, 3) void chunk_outer_bf16_kernel(
+__global__ __launch_bounds__(256, MODE == 2 && NK == 4 ? 2 : 3) void chunk_outer_bf16_kernel(
     const void* __restrict__ a_src, const bf16* __restrict__ x_src, const float* __restrict__ dt,
     const float* __restrict__ dc, const int64_t* __restrict__ length, float* __restrict__ out,
-    bf16* __restrict__ dyp, SsdDims d) {
+    bf16* __restrict__ dyp, SsdDims d, GateBwd gb) {
   constexpr int N = 32 * NK;
   using TA = LdsTile<64>;                  // the scaled operand's planes
   using TX = LdsTile<N>;                   // the B or C tile
@@ -223,7 +235,10 @@ __global__ __launch_bounds__(256, 3) void chunk_outer_bf16_kernel(
 #pragma unroll
     for (int pt = 0; pt < 4; ++pt) acc[i][pt] = v4f{0.f, 0.f, 0.f, 0.f};
 
-  if (klim > 0) {
+  float dD[MODE == 2 ? 8 : 1] = {};   // sums of dy u over this thread's rows, 8 columns
+  // MODE 2 walks the rows past the length too: the gate's gradients exist there
+  const int rlim = MODE == 2 ? qlim : klim;
+  if (rlim > 0) {
     const long tok0 = static_cast<long>(b) * d.L + static_cast<long>(c) * d.Lc;
     const int a_rs = d.H * d.P, x_rs = d.G * N;
     const bf16* xc = x_src + tok0 * x_rs + static_cast<long>(g) * N;
@@ -234,6 +249,14 @@ __global__ __launch_bounds__(256, 3) void chunk_outer_bf16_kernel(
     // order), before the current tile's MFMAs.
     int slot_tile = 0;   // tile index held by the prefetch registers
     uint4 pa0[MODE == 0 ? 2 : 1];
+    uint4 pg[MODE == 2 ? 2 : 1][4];   // dout, gate, yd, u
+    float Dv[MODE == 2 ? 8 : 1];
+    if constexpr (MODE == 2) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        *reinterpret_cast<float4*>(Dv + 4 * i) =
+            *reinterpret_cast<const float4*>(gb.D + h * 64 + 8 * (tid & 7) + 4 * i);
+    }
     float4 pa1[MODE == 1 ? 4 : 1];
     float pdc[2], pdt[2];   // dc, dt of the rows (clamped to klim - 1)
     // scale of row t of the held tile from its dc, dt (0 past klim)
@@ -249,6 +272,20 @@ __global__ __launch_bounds__(256, 3) void chunk_outer_bf16_kernel(
     auto load_tile = [&](int tt) __attribute__((always_inline)) {
       const int t0 = 64 * tt, kv = min(64, klim - t0);
       slot_tile = tt;
+      if constexpr (MODE == 2) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int e = tid + 256 * i, t = min(t0 + (e >> 3), qlim - 1);
+          const long o = tok0 * a_rs + h * 64 + static_cast<unsigned>(t * a_rs + 8 * (e & 7));
+          pg[i][0] = *reinterpret_cast<const uint4*>(gb.dout + o);
+          pg[i][1] = *reinterpret_cast<const uint4*>(gb.gate + o);
+          pg[i][2] = *reinterpret_cast<const uint4*>(gb.yd + o);
+          pg[i][3] = *reinterpret_cast<const uint4*>(gb.u + o);
+          pdc[i] = dc[crow + t];
+        }
+        if (kv > 0) px.load(xc + static_cast<long>(t0) * x_rs, x_rs, kv, tid);
+        return;
+      }
       if constexpr (MODE == 0) {
         const bf16* ac = static_cast<const bf16*>(a_src) + tok0 * a_rs + h * d.P + p0;
 #pragma unroll
@@ -272,6 +309,58 @@ __global__ __launch_bounds__(256, 3) void chunk_outer_bf16_kernel(
     auto commit_tile = [&]() __attribute__((always_inline)) {
       bf16* As = sm;
       bf16* Xs = As + NPL * PLA;
+      if constexpr (MODE == 2) {
+        const int hpg = d.H / d.G;
+        const bool live = 64 * slot_tile < klim;
+        const long tileo = ((((static_cast<long>(b) * d.nc + c) * d.G + g) * (d.Lc / 64) + slot_tile) * hpg +
+                            (h - g * hpg)) * (2L * 64 * 64);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const int e = tid + 256 * i, row = e >> 3, t = 64 * slot_tile + row;
+          const bool in = t < klim, q = t < qlim;
+          const float sc = row_scale(t, pdc[i], 0.f);
+          uint32_t hi[4], lo[4], shi[4], slo[4], dg[4], sk[4];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const uint32_t w4[4] = {(&pg[i][0].x)[j], (&pg[i][1].x)[j], (&pg[i][2].x)[j], (&pg[i][3].x)[j]};
+            float dv[2], dgv[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+              const float ov = k ? bf16hi_to_f32(w4[0]) : bf16lo_to_f32(w4[0]);
+              const float gv = k ? bf16hi_to_f32(w4[1]) : bf16lo_to_f32(w4[1]);
+              const float yv = k ? bf16hi_to_f32(w4[2]) : bf16lo_to_f32(w4[2]);
+              const float xv = k ? bf16hi_to_f32(w4[3]) : bf16lo_to_f32(w4[3]);
+              const float sg = fast_sigmoid(gv);
+              const float dyv = ov * gv * sg;                       // dout silu(gate)
+              dgv[k] = ov * yv * sg * (1.0f + gv * (1.0f - sg));
+              if (q) dD[2 * j + k] += dyv * xv;
+              dv[k] = dyv;
+            }
+            dg[j] = pack_bf16x2(dgv[0], dgv[1]);
+            sk[j] = pack_bf16x2(Dv[2 * j] * dv[0], Dv[2 * j + 1] * dv[1]);
+            const float v0 = in ? dv[0] : 0.f, v1 = in ? dv[1] : 0.f;
+            hi[j] = pack_bf16x2(v0, v1);
+            lo[j] = pack_bf16x2(v0 - bf16lo_to_f32(hi[j]), v1 - bf16hi_to_f32(hi[j]));
+            const float s0 = v0 * sc, s1 = v1 * sc;
+            shi[j] = pack_bf16x2(s0, s1);
+            slo[j] = pack_bf16x2(s0 - bf16lo_to_f32(shi[j]), s1 - bf16hi_to_f32(shi[j]));
+          }
+          const int col = 8 * (e & 7);
+          if (live) {
+            const int ao = TA::off(row, col);
+            *reinterpret_cast<uint4*>(As + ao) = uint4{shi[0], shi[1], shi[2], shi[3]};
+            *reinterpret_cast<uint4*>(As + PLA + ao) = uint4{slo[0], slo[1], slo[2], slo[3]};
+            bf16* pl = dyp + tileo + row * 64 + col;
+            *reinterpret_cast<uint4*>(pl) = uint4{hi[0], hi[1], hi[2], hi[3]};
+            *reinterpret_cast<uint4*>(pl + 64 * 64) = uint4{lo[0], lo[1], lo[2], lo[3]};
+          }
+          const long o = tok0 * a_rs + h * 64 + static_cast<unsigned>(t * a_rs + col);
+          if (q) *reinterpret_cast<uint4*>(gb.dgate + o) = uint4{dg[0], dg[1], dg[2], dg[3]};
+          if (q && !in) *reinterpret_cast<uint4*>(gb.du + o) = uint4{sk[0], sk[1], sk[2], sk[3]};
+        }
+        if (live) commit_lds(px, Xs, tid);
+        return;
+      }
       if constexpr (MODE == 0) {
         // w * u is fp32 (dt up to z > 20 makes it large): hi + lo planes keep
         // the chunk states near fp32, which the backward's dC, dA and
@@ -342,7 +431,7 @@ __global__ __launch_bounds__(256, 3) void chunk_outer_bf16_kernel(
       }
     };
 
-    const int ntt = (klim + 63) / 64;
+    const int ntt = (rlim + 63) / 64;
     load_tile(0);
     commit_tile();
     __syncthreads();
@@ -353,6 +442,7 @@ __global__ __launch_bounds__(256, 3) void chunk_outer_bf16_kernel(
       const bf16* Xs = As + NPL * PLA;
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
+        if (MODE == 2 && 64 * tt >= klim) break;
         v8bf bop[4][NPL];
 #pragma unroll
         for (int pt = 0; pt < 4; ++pt)
@@ -371,6 +461,21 @@ __global__ __launch_bounds__(256, 3) void chunk_outer_bf16_kernel(
       __syncthreads();   // every wave is done with the stage
       if (has_next) commit_tile();
       __syncthreads();
+    }
+  }
+  if constexpr (MODE == 2) {   // dD of this chunk: the block's 32 row groups in a fixed order
+    __syncthreads();
+    float* red = reinterpret_cast<float*>(smem_raw);   // [32][64]
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      *reinterpret_cast<float4*>(red + (tid >> 3) * 64 + 8 * (tid & 7) + 4 * i) =
+          make_float4(dD[4 * i], dD[4 * i + 1], dD[4 * i + 2], dD[4 * i + 3]);
+    __syncthreads();
+    if (tid < 64) {
+      float sum = 0.f;
+#pragma unroll 8
+      for (int r = 0; r < 32; ++r) sum += red[r * 64 + tid];
+      gb.dD_part[(static_cast<long>(b) * d.nc + c) * (d.H * 64) + h * 64 + tid] = sum;
     }
   }
   // D^T[n][p]: lane holds n = 16 nt + 4 lg + r of p = 16 pt + li
@@ -1239,7 +1344,7 @@ int launch_chunk_cumsum(const void* delta_raw, const float* A, const float* bias
 template <int NK, int MODE>
 int launch_chunk_outer_bf16_nk(const void* a, const void* x, const float* dt, const float* dc,
                                const int64_t* length, float* out, const SsdDims& d, hipStream_t s,
-                               bf16* dyp = nullptr) {
+                               bf16* dyp = nullptr, const GateBwd& gb = {}) {
   const long blocks = static_cast<long>(d.P / 64) * d.H * d.nc * d.b;
   const size_t smem = sizeof(bf16) * 64 * (2 * LdsTile<64>::kLd + LdsTile<32 * NK>::kLd);
   if (smem > 64 * 1024) {
@@ -1247,9 +1352,9 @@ int launch_chunk_outer_bf16_nk(const void* a, const void* x, const float* dt, co
                                        hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(smem));
     SA_CHECK_ARG(e == hipSuccess, "chunk_outer_bf16: %zu B of LDS refused", smem);
   }
-  ProfScope prof_(MODE == 0 ? "chunk_state_fwd" : "chunk_dstate_bwd", s);
+  ProfScope prof_(MODE == 0 ? "chunk_state_fwd" : MODE == 1 ? "chunk_dstate_bwd" : "chunk_dstate_gate_bwd", s);
   hipLaunchKernelGGL((chunk_outer_bf16_kernel<NK, MODE>), dim3(blocks), dim3(256), smem, s, a,
-                     static_cast<const bf16*>(x), dt, dc, length, out, dyp, d);
+                     static_cast<const bf16*>(x), dt, dc, length, out, dyp, d, gb);
   SA_CHECK_LAUNCH("chunk_outer_bf16");
   return 0;
 }
@@ -1285,6 +1390,16 @@ int launch_dstate_planes(const float* dy, const void* C, const float* dt, const 
                "launch_dstate_planes: P 64, N 64 or 128, chunk %% 64 and aligned operands required");
   if (d.N == 64) return launch_chunk_outer_bf16_nk<2, 1>(dy, C, dt, dc, length, out, d, s, dyp);
   return launch_chunk_outer_bf16_nk<4, 1>(dy, C, dt, dc, length, out, d, s, dyp);
+}
+
+int launch_dstate_gate(const GateBwd& gb, const void* C, const float* dt, const float* dc,
+                       const int64_t* length, float* out, bf16* dyp, const SsdDims& d,
+                       hipStream_t s) {
+  const int rc = d.N == 64 ? launch_chunk_outer_bf16_nk<2, 2>(nullptr, C, dt, dc, length, out, d, s, dyp, gb)
+                           : launch_chunk_outer_bf16_nk<4, 2>(nullptr, C, dt, dc, length, out, d, s, dyp, gb);
+  if (rc) return rc;
+  ProfScope prof_("ssm_gate_dD_reduce", s);
+  return launch_reduce_partials(gb.dD_part, d.b * d.nc, static_cast<long>(d.H) * 64, gb.dD, s);
 }
 
 // compute units of the current device (cached per device; 256 if unknown)

@@ -23,6 +23,7 @@
 // gate forward, which sums nothing, gives a thread one row (see there).
 #include "common.h"
 #include "prof.h"
+#include "ssd_common.h"
 
 namespace sa {
 namespace {
@@ -553,6 +554,13 @@ size_t conv_part_elems(int batch, int L, int Dc, int K) {
 }
 
 }  // namespace
+
+int launch_reduce_partials(const float* part, int np, long n, float* out, hipStream_t s) {
+  hipLaunchKernelGGL(reduce_partials_kernel, dim3(reduce_blocks(n)), dim3(256), 0, s, part, np, n, out);
+  SA_CHECK_LAUNCH("reduce_partials");
+  return 0;
+}
+
 }  // namespace sa
 
 using sa::bf16;

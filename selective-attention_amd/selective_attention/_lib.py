@@ -68,9 +68,10 @@ SIGNATURES: dict[str, list] = {
     "sa_ssd_bwd": [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
                    _i, _i, _i, _i, _i, _i, _i, _i, _f, _f, _i,
                    _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
-    "sa_ssd_bwd_add": [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
-                       _i, _i, _i, _i, _i, _i, _i, _i, _f, _f, _i, _vp,
-                       _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
+    "sa_ssd_bwd_gated_workspace_size": [_i, _i, _i, _i, _i, _i, _i, _i],
+    "sa_ssd_bwd_gated": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp,
+                         _i, _i, _i, _i, _i, _i, _i, _i, _f, _f, _i,
+                         _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp],
     "sa_ssm_conv_fwd": [_i, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp],
     "sa_ssm_conv_bwd_workspace_size": [_i, _i, _i, _i],
     "sa_ssm_conv_bwd": [_i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp, _vp, _vp,
@@ -87,6 +88,7 @@ SIGNATURES: dict[str, list] = {
 }
 
 RESTYPES = {"sa_last_error": ctypes.c_char_p, "sa_profile_enable": None, "sa_ssd_bwd_workspace_size": ctypes.c_size_t,
+            "sa_ssd_bwd_gated_workspace_size": ctypes.c_size_t,
             "sa_paged_decode_workspace_size": ctypes.c_size_t,
             "sa_paged_decode_noalloc_limit": ctypes.c_size_t,
             "sa_ssm_conv_bwd_workspace_size": ctypes.c_size_t,

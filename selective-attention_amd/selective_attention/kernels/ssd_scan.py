@@ -147,14 +147,13 @@ def gated_supported(dtype: torch.dtype, head_dim: int, state_dim: int) -> bool:
 
 def ssd_scan_backward(u, A, B, C, delta_raw, delta_bias, h_init, y_grad, h_last_grad, length,
                       chunk_size, use_delta_softplus=True, delta_limit=(0.0, float("inf")),
-                      is_causal=True, saved=None, du_add=None):
+                      is_causal=True, saved=None):
     """
     Args: as ssd_scan_forward, plus
         y_grad: (batch_size, seq_len, num_heads, head_dim) or None
         h_last_grad: (batch_size, num_heads, head_dim, state_dim) or None
         saved: (dt, dc, states) returned by ssd_scan_forward(return_saved=True);
                recomputed when None
-        du_add: tensor like u or None, added to the gradient of u
 
     Returns:
         u_grad, A_grad, B_grad, C_grad, delta_raw_grad, delta_bias_grad, h_init_grad
@@ -189,8 +188,6 @@ def ssd_scan_backward(u, A, B, C, delta_raw, delta_bias, h_init, y_grad, h_last_
     dA = torch.empty((H,), dtype=f32, device=dev)
     dbias = None if delta_bias is None else torch.empty((H,), dtype=f32, device=dev)
     dh0 = None if h_init is None else torch.empty((b, H, P, N), dtype=f32, device=dev)
-    if du_add is not None:
-        du_add = as_dtype(du_add, u.dtype).contiguous()
     if L == 0:
         du.zero_(); dB.zero_(); dC.zero_(); ddr.zero_(); dA.zero_()
         if dbias is not None:
@@ -205,14 +202,77 @@ def ssd_scan_backward(u, A, B, C, delta_raw, delta_bias, h_init, y_grad, h_last_
         ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev)
         lo, hi = limits(delta_limit)
         _lib.call(
-            "sa_ssd_bwd_add", code, _lib.ptr(u), _lib.ptr(A32), _lib.ptr(B), _lib.ptr(C),
+            "sa_ssd_bwd", code, _lib.ptr(u), _lib.ptr(A32), _lib.ptr(B), _lib.ptr(C),
             _lib.ptr(delta_raw), _lib.ptr(bias32), _lib.ptr(length), _lib.ptr(dy),
             _lib.ptr(dh_last), _lib.ptr(dt), _lib.ptr(dc), _lib.ptr(states),
             b, L, H, P, G, N, int(chunk_size), 1 if use_delta_softplus else 0, lo, hi,
             0 if h_init is None else 1,
-            _lib.ptr(du_add), _lib.ptr(du), _lib.ptr(dA), _lib.ptr(dB), _lib.ptr(dC), _lib.ptr(ddr),
+            _lib.ptr(du), _lib.ptr(dA), _lib.ptr(dB), _lib.ptr(dC), _lib.ptr(ddr),
             _lib.ptr(dbias), _lib.ptr(dh0), _lib.ptr(ws), nbytes, _lib.stream_of(u))
     return (as_dtype(du, dtypes["u"]), as_dtype(dA, dtypes["A"]), as_dtype(dB, dtypes["B"]),
             as_dtype(dC, dtypes["C"]), as_dtype(ddr, dtypes["delta_raw"]),
             None if dbias is None else as_dtype(dbias, dtypes["bias"]),
             None if dh0 is None else as_dtype(dh0, dtypes["h"]))
+
+
+def _addr16(*tensors):
+    return all(t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def ssd_scan_backward_gated(u, A, B, C, delta_raw, delta_bias, h_init, dout, yd, D, gate,
+                            h_last_grad, length, chunk_size, use_delta_softplus=True,
+                            delta_limit=(0.0, float("inf")), saved=None):
+    """Backward of ssd_scan_forward_gated with the gate's backward inside: dy =
+    dout silu(gate) goes straight into the scan's operand planes and D dy into
+    the gradient of u.
+
+    Args: as ssd_scan_backward, plus
+        dout, yd, gate: (batch_size, seq_len, num_heads, head_dim); yd and
+            saved as ssd_scan_forward_gated returned them
+        D: (num_heads * head_dim,)
+
+    Returns:
+        ssd_scan_backward's gradients (the skip path's part in u_grad), then
+        D_grad (float32) and gate_grad (dtype of u); or None for what the
+        kernels do not take (bfloat16, head_dim 64, state_dim 64 or 128,
+        chunk_size a multiple of 64, operands on 16-byte boundaries).
+    """
+    if u.dtype != torch.bfloat16 or u.numel() == 0:
+        return None
+    b, L, H, P = u.shape
+    G, N = B.shape[2], B.shape[3]
+    lib = _lib.load()
+    nbytes = lib.sa_ssd_bwd_gated_workspace_size(_lib.DTYPE_BF16, b, L, H, P, G, N, int(chunk_size))
+    if nbytes == 0:
+        return None
+    dtypes = (A.dtype, B.dtype, C.dtype, delta_raw.dtype)
+    _, u, A32, B, C, delta_raw, bias32, _, length = _prep(
+        u, A, B, C, delta_raw, delta_bias, None, length)
+    dout = as_dtype(dout, u.dtype).contiguous()
+    gate = as_dtype(gate, u.dtype).contiguous()
+    yd = yd.contiguous()
+    D32 = as_dtype(D, torch.float32).contiguous()
+    if not _addr16(u, B, C, dout, yd, gate, D32):
+        return None
+    dt, dc, states = saved
+    dh_last = _f32_aligned(h_last_grad)
+    dev, f32 = u.device, torch.float32
+    du, dB, dC, ddr, dgate = (torch.empty_like(t) for t in (u, B, C, delta_raw, u))
+    dA = torch.empty((H,), dtype=f32, device=dev)
+    dD = torch.empty((H * P,), dtype=f32, device=dev)
+    dbias = None if delta_bias is None else torch.empty((H,), dtype=f32, device=dev)
+    dh0 = None if h_init is None else torch.empty((b, H, P, N), dtype=f32, device=dev)
+    ws = torch.empty((nbytes,), dtype=torch.uint8, device=dev)
+    lo, hi = limits(delta_limit)
+    _lib.call(
+        "sa_ssd_bwd_gated", _lib.ptr(u), _lib.ptr(A32), _lib.ptr(B), _lib.ptr(C),
+        _lib.ptr(delta_raw), _lib.ptr(bias32), _lib.ptr(length), _lib.ptr(dout), _lib.ptr(yd),
+        _lib.ptr(D32), _lib.ptr(gate), _lib.ptr(dh_last), _lib.ptr(dt), _lib.ptr(dc),
+        _lib.ptr(states), b, L, H, P, G, N, int(chunk_size), 1 if use_delta_softplus else 0, lo,
+        hi, 0 if h_init is None else 1, _lib.ptr(du), _lib.ptr(dA), _lib.ptr(dB), _lib.ptr(dC),
+        _lib.ptr(ddr), _lib.ptr(dbias), _lib.ptr(dh0), _lib.ptr(dD), _lib.ptr(dgate),
+        _lib.ptr(ws), nbytes, _lib.stream_of(u))
+    return (du, as_dtype(dA, dtypes[0]), as_dtype(dB, dtypes[1]), as_dtype(dC, dtypes[2]),
+            as_dtype(ddr, dtypes[3]),
+            None if dbias is None else as_dtype(dbias, delta_bias.dtype),
+            None if dh0 is None else as_dtype(dh0, h_init.dtype), dD, dgate)

@@ -137,6 +137,8 @@ class SSDScanGatedFn(torch.autograd.Function):
     is never written; the scan saves yd = y + D u (bf16) for the gate's
     backward instead.  Other inputs run the scan and SSMGateFn's kernel in
     turn.  u is used twice (scan input and D skip); its gradient is the sum.
+    The backward of head_dim 64, state_dim 64 or 128 forms dy inside the
+    scan's backward (ssd_scan_backward_gated).
     """
 
     @staticmethod
@@ -179,19 +181,26 @@ class SSDScanGatedFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, h_last_grad):
-        from ..kernels.ssd_scan import ssd_scan_backward
+        from ..kernels.ssd_scan import ssd_scan_backward, ssd_scan_backward_gated
         u, A, B, C, delta_raw, delta_bias, h_init, length, D, gate, ysave, dt, dc, states = \
             ctx.saved_tensors
         chunk_size, sp, limit = ctx.cfg
         if dout is None:
             dout = torch.zeros_like(u)
-        P = u.shape[-1]
+        if ctx.fused:
+            grads = ssd_scan_backward_gated(u, A, B, C, delta_raw, delta_bias, h_init, dout, ysave,
+                                            D, gate, h_last_grad, length, chunk_size, sp, limit,
+                                            (dt, dc, states))
+            if grads is not None:
+                *grads, dD, dgate = grads
+                return (*grads, None, None, None, None, dD.to(D.dtype), dgate.to(gate.dtype))
         dy, d_skip, dD, dgate = ssm_gate_backward(
             dout.reshape(*u.shape[:2], -1), ysave.reshape(*u.shape[:2], -1),
             u.reshape(*u.shape[:2], -1), D, gate.reshape(*u.shape[:2], -1), y_is_yd=ctx.fused)
         grads = ssd_scan_backward(u, A, B, C, delta_raw, delta_bias, h_init, dy.view(u.shape),
                                   h_last_grad, length, chunk_size, sp, limit, True,
-                                  saved=(dt, dc, states), du_add=d_skip.view(u.shape))
+                                  saved=(dt, dc, states))
         du, dA, dB, dC, ddr, dbias, dh0 = grads
+        du = du + d_skip.view(u.shape)
         return (du, dA, dB, dC, ddr, dbias, dh0, None, None, None, None,
                 dD.to(D.dtype), dgate.view(u.shape).to(gate.dtype))

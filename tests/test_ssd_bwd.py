@@ -6,7 +6,6 @@ import torch
 
 from oracle import ssd as ref
 from selective_attention import workloads
-from selective_attention.kernels.ssd_scan import ssd_scan_backward
 from tests.helpers import assert_parity
 from tests.test_ssd_fwd import large_z, make_inputs, to_dev
 
@@ -313,32 +312,3 @@ def test_ssd_bwd_deterministic():
     b = gpu_grads(x, dy, None, 64)
     for k in a:
         assert torch.equal(a[k], b[k]), f"d{k} differs between runs"
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("dtype,b,L,H,P,N,G,chunk,lens,off", [
-    (torch.bfloat16, 1, 1, 1, 64, 64, 1, 64, None, 0),         # fused, one head per group
-    (torch.bfloat16, 2, 333, 4, 64, 128, 2, 256, [333, 70], 0),  # fused, two heads, a ragged strip
-    (torch.bfloat16, 2, 200, 3, 64, 64, 1, 128, [200, 64], 0),   # fused, an odd head in the last pass
-    (torch.bfloat16, 2, 520, 7, 64, 128, 1, 256, [0, 391], 0),   # fused, more passes; an empty row
-    (torch.bfloat16, 1, 200, 4, 64, 64, 1, 128, [150], 1),       # fused, du_add off a 16-byte boundary
-    (torch.bfloat16, 2, 150, 2, 32, 16, 1, 64, [150, 9], 0),     # general kernels
-    (torch.float32, 2, 150, 2, 64, 64, 1, 64, [150, 9], 0),      # fp32 tiles
-    (torch.float32, 1, 77, 3, 24, 16, 1, 64, None, 1),           # general kernels, fp32
-])
-def test_bwd_du_add(dtype, b, L, H, P, N, G, chunk, lens, off):
-    """du_add is added to the rounded du and rounded again: equal to the sum of
-    the two tensors, past a row's length too; no other gradient changes."""
-    g = torch.Generator().manual_seed(L + H)
-    r = lambda *s: torch.randn(*s, generator=g).cuda()
-    act = lambda *s: r(*s).to(dtype)
-    u, dy = act(b, L, H, P), r(b, L, H, P)
-    A, bias = -torch.exp(r(H)), 0.3 * r(H)
-    B, C, dr = act(b, L, G, N) / 8, act(b, L, G, N) / 8, act(b, L, H) - 3
-    add = act(u.numel() + off)[off:].view(u.shape)
-    length = None if lens is None else torch.tensor(lens).cuda()
-    run = lambda **kw: ssd_scan_backward(u, A, B, C, dr, bias, None, dy, None, length, chunk, **kw)
-    plain, both = run(), run(du_add=add)
-    assert torch.equal(both[0], plain[0] + add)
-    for x, y in zip(plain[1:], both[1:]):
-        assert (x is None and y is None) or torch.equal(x, y)

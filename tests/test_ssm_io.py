@@ -365,3 +365,58 @@ def test_ssd_scan_gated_parity(name, dtype, shape, chunk):
         assert_parity(leaf.grad, exp[k], tol, f"d{k}")
     assert_parity(Dd.grad, dD, dtype, "dD")
     assert_parity(gd.grad, dgate.reshape(b, L, H, P), dtype, "dgate")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,L,H,N,G,chunk,lens,off", [
+    (1, 1, 1, 64, 1, 64, None, 0),            # one row, one head per group
+    (2, 333, 4, 128, 2, 256, [333, 70], 0),   # ragged strips, whole tiles past a length
+    (2, 200, 3, 64, 1, 128, [200, 64], 0),    # an odd head in the last pass; a length on a tile edge
+    (2, 520, 7, 128, 1, 256, [0, 391], 0),    # more than two passes; an empty row
+    (1, 200, 4, 64, 1, 128, [150], 1),        # dout off a 16-byte boundary: the separate kernels
+    (1, 100, 2, 64, 1, 48, None, 0),          # a chunk the gated kernels do not take
+])
+def test_gated_backward_forms_dy_inside(b, L, H, N, G, chunk, lens, off, monkeypatch):
+    """Against the gate's and the scan's backward run in turn: dy and its planes
+    are the same, so every gradient but du and dD is equal.  du adds D dy (dy to
+    2^-17) after one rounding of each term instead of three in all; dD sums
+    dy u in another order."""
+    from selective_attention.kernels import ssd_scan as ks
+    from selective_attention.ops import SSDScanGatedFn
+    g = torch.Generator().manual_seed(L + H)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()
+    act = lambda *s: r(*s).bfloat16()
+    leaf = lambda t: t.requires_grad_(True)
+    u, dr = leaf(act(b, L, H, 64)), leaf(act(b, L, H) - 3)
+    B, C = leaf(act(b, L, G, N) / 8), leaf(act(b, L, G, N) / 8)
+    A, bias, D = leaf(-torch.exp(r(H))), leaf(0.3 * r(H)), leaf(r(H * 64))
+    h0 = leaf(0.2 * r(b, H, 64, N))
+    gate = leaf(act(b, L, H, 64))
+    length = None if lens is None else torch.tensor(lens).cuda()
+    dout, dh = act(u.numel() + off)[off:].view(u.shape), 0.2 * r(b, H, 64, N)
+    leaves = (u, A, B, C, dr, bias, h0, D, gate)
+    taken, gated = [], ks.ssd_scan_backward_gated
+
+    def both(split):
+        def call(*a):
+            taken.append(None if split else gated(*a))
+            return taken[-1]
+        monkeypatch.setattr(ks, "ssd_scan_backward_gated", call)
+        out, h = SSDScanGatedFn.apply(u, A, B, C, dr, bias, h0, length, chunk, True,
+                                      (0.0, float("inf")), D, gate)
+        return torch.autograd.grad((out, h), leaves, (dout, dh))
+    got, exp = both(False), both(True)
+    assert (taken[0] is None) == (off != 0 or chunk % 64 != 0)
+    for i, name in enumerate("u A B C dr bias h0 D gate".split()):
+        x, y = got[i].double(), exp[i].double()
+        if name == "u":
+            gd, od = gate.detach().double(), dout.double()
+            skip = (D.detach().double().view(H, 64) * od * gd * torch.sigmoid(gd)).abs()
+            # two bf16 roundings of the sum, one of the skip term there
+            assert ((x - y).abs() <= 2 ** -7 * (y.abs() + x.abs()) + 2 ** -8 * skip).all()
+        elif name == "D":
+            gd, od = gate.detach().double(), dout.double()
+            size = (od * gd * torch.sigmoid(gd) * u.detach().double()).abs().sum((0, 1)).view(-1)
+            assert ((x - y).abs() <= 64 * 2 ** -24 * size + 1e-12).all()
+        else:
+            assert torch.equal(x, y), name
