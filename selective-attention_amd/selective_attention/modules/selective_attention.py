@@ -40,6 +40,25 @@ def _threshold(thr, num_heads: int, device):
     return torch.as_tensor(thr, device=device).reshape(num_heads)
 
 
+def _later_bool(flag: torch.Tensor):
+    """A function that returns bool(flag).  On a GPU the value is on its way to
+    the host from here on, so that what is launched before the function is
+    called runs meanwhile: it waits for `flag` alone, where bool(flag) there
+    would wait for all of it."""
+    if not flag.is_cuda or torch.cuda.is_current_stream_capturing():
+        value = bool(flag)
+        return lambda: value
+    host = torch.empty((), dtype=torch.bool, pin_memory=True)
+    host.copy_(flag, non_blocking=True)
+    done = torch.cuda.Event()
+    done.record(torch.cuda.current_stream(flag.device))
+
+    def get():
+        done.synchronize()
+        return bool(host)
+    return get
+
+
 class SelectiveMHA(nn.Module):
     def __init__(self, layer_idx: int, dim: int, head_dim: int, log_gate_penalty: float,
                  is_causal: bool = True):
@@ -101,9 +120,7 @@ class SelectiveMHA(nn.Module):
             lens = lengths.to(dev)
             kept &= (torch.arange(L, device=dev)[None, :] < lens[:, None])[:, None, :]
         v = self.v_proj(hidden_states)
-        if not bool(kept.any()):
-            # every key dropped: each query attends only itself (:208-209)
-            return self.out_proj(v * out_gate)
+        any_kept = _later_bool(kept.any())
         q, k = self.rope.rotate_qk(self.q_proj(hidden_states).view(b, L, H, D),
                                    self.k_proj(hidden_states).view(b, L, H, D), None, L)
         q, k = q.transpose(1, 2), k.transpose(1, 2)                   # (b, H, L, D) views
@@ -111,11 +128,15 @@ class SelectiveMHA(nn.Module):
         log_gate = self._log_gate(select_gate, kept)
         if self.is_causal:
             out = selective_mha_prefill(q, k, vh, log_gate, lengths)
+            if not any_kept():
+                return self.out_proj(v * out_gate)
             if cache is not None:
                 cache.build_kv(k, vh, log_gate, lengths)
             out = out.transpose(1, 2).reshape(b, L, self.dim)
         else:
             out = self._bidirectional(q, k, vh, log_gate, lengths)
+            if not any_kept():
+                return self.out_proj(v * out_gate)
         return self.out_proj(out.to(hidden_states.dtype) * out_gate)
 
     def _train_forward(self, hidden_states, lengths):

@@ -317,3 +317,52 @@ def test_drop_evicted_pages_keeps_reserved_pages():
     assert cache.drop_evicted_pages() == 1
     assert cache.lens == [66] and len(cache.rows[0]) == 4
     assert cache.drop_evicted_pages() == 0 and cache.lens == [66]
+
+
+@pytest.mark.gpu
+def test_eager_append_matches_indexed_stores():
+    """append's kernel against the indexed stores (a log_gate of another rank
+    takes them), over page edges, pool growth, unappend, a compaction and a row
+    without tokens: the pages, lengths and attention are equal."""
+    H, D, ps = 3, 64, 64
+    g = torch.Generator().manual_seed(5)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()
+    lens = torch.tensor([129, 64, 0])
+    k, v, lg = r(3, H, 129, D).bfloat16(), r(3, H, 129, D).bfloat16(), r(3, H, 129)
+    lg[0, :, :64] = float("-inf")
+    caches = [PagedSelectiveAttnCache(3, H, D, 40, "cuda", page_size=ps, grow=True) for _ in range(2)]
+    for c in caches:
+        c.build(k, v, lg, lens)
+    held = caches[0].seq_lens()
+    for t in range(70):
+        kt, vt, lt, q = r(3, H, D).bfloat16(), r(3, H, D), r(3, H), r(3, H, D)
+        caches[0].append(kt, vt, lt)
+        caches[1].append(kt, vt, lt[None])
+        if t == 3:
+            for c in caches:
+                c.unappend(rows=[1])
+        if t == 20:
+            assert [c.drop_evicted_pages() for c in caches] == [1, 1]
+        assert caches[0].lens == caches[1].lens == caches[0].seq_lens().tolist()
+        assert caches[0].rows == caches[1].rows
+        assert torch.equal(caches[0].attend(q), caches[1].attend(q))
+    assert held.tolist() == [129, 64, 0]      # a tensor handed out earlier stays as it was
+    for name in ("k_pages", "v_pages", "gate_pages"):
+        assert torch.equal(getattr(caches[0], name), getattr(caches[1], name))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("causal", [True, False])
+def test_prefill_with_every_key_dropped(causal):
+    """A threshold above every gate: each query attends itself alone, so the
+    layer returns out_proj(v * out_gate) bit for bit and fills no cache."""
+    from selective_attention.inference import SelectiveAttnCache
+    from selective_attention.modules.selective_attention import SelectiveMHA
+    torch.manual_seed(0)
+    m = SelectiveMHA(0, 128, 64, 1.5, is_causal=causal).cuda().bfloat16().eval()
+    x = torch.randn(2, 70, 128).bfloat16().cuda()
+    cache = SelectiveAttnCache()
+    with torch.no_grad():
+        got = m(x, attn_gate_threshold=2.0, cache=cache)
+        exp = m.out_proj(m.v_proj(x) * m._gates(x)[1])
+    assert torch.equal(got, exp) and cache.pages is None
