@@ -229,6 +229,15 @@ int sa_add_rms_norm_bf16(const void* x, const void* y, const float* weight, long
 int sa_mha_gates_bf16(const void* g, const float* thr, const float* score_std, float penalty,
                       long rows, int heads, int dim, float* log_gate, void* out_gate, void* stream);
 
+/* The same over a prompt: g (batch * seqlen, heads + dim), log_gate (batch,
+ * heads, seqlen) with -inf at t >= lengths[b] (lengths may be NULL), out_gate
+ * (batch * seqlen, dim); any_kept[0] is set to 1 if any key is kept and left
+ * alone otherwise. */
+int sa_mha_prompt_gates_bf16(const void* g, const float* thr, const float* score_std,
+                             const int64_t* lengths, float penalty, int batch, int seqlen,
+                             int heads, int dim, float* log_gate, void* out_gate,
+                             int32_t* any_kept, void* stream);
+
 /*
  * Per-head statistics of the valid attention scores s_ij = scale * q_i . k_j,
  * for the training forwards of SelectiveMHA and CrossSelectiveMHA:

@@ -50,6 +50,7 @@ SIGNATURES: dict[str, list] = {
     "sa_paged_kv_append": [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp, _vp],
     "sa_add_rms_norm_bf16": [_vp, _vp, _vp, _i64, _i, _f, _vp, _vp, _vp],
     "sa_mha_gates_bf16": [_vp, _vp, _vp, _f, _i64, _i, _i, _vp, _vp, _vp],
+    "sa_mha_prompt_gates_bf16": [_vp, _vp, _vp, _vp, _f, _i, _i, _i, _i, _vp, _vp, _vp, _vp],
     "sa_silu_mul_bf16": [_vp, _vp, _i64, _vp, _vp],
     "sa_score_stats_workspace_size": [_i, _i, _i],
     "sa_score_stats": [_i, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _f, _vp, _sz, _vp, _vp],

@@ -123,6 +123,26 @@ def mha_gates(g: torch.Tensor, threshold: torch.Tensor | None, score_std: torch.
     return lg, og
 
 
+def mha_prompt_gates(g: torch.Tensor, threshold: torch.Tensor | None, score_std: torch.Tensor,
+                     lengths: torch.Tensor | None, penalty: float, heads: int):
+    """g (batch, seq_len, heads + dim) bf16, lengths (batch,) -> (log_gate (batch,
+    heads, seq_len) f32, out_gate (batch, seq_len, dim) bf16, any_kept (1,)
+    int32, 1 if any key is kept)."""
+    require_device(g, threshold, score_std, lengths)
+    g = g.contiguous()
+    b, L, W = g.shape
+    lg = torch.empty(b, heads, L, dtype=torch.float32, device=g.device)
+    og = torch.empty(b, L, W - heads, dtype=torch.bfloat16, device=g.device)
+    flag = torch.zeros(1, dtype=torch.int32, device=g.device)
+    thr = None if threshold is None else threshold.to(torch.float32).contiguous()
+    std = score_std.to(torch.float32).contiguous()
+    lens = None if lengths is None else lengths.to(torch.int64).expand(b).contiguous()
+    _lib.call("sa_mha_prompt_gates_bf16", _lib.ptr(g), _lib.ptr(thr), _lib.ptr(std), _lib.ptr(lens),
+              float(penalty), b, L, heads, W - heads, _lib.ptr(lg), _lib.ptr(og), _lib.ptr(flag),
+              _lib.stream_of(g))
+    return lg, og, flag
+
+
 def silu_mul(a: torch.Tensor, c: torch.Tensor) -> torch.Tensor:
     """bf16(a * bf16(silu(c))) for bf16 tensors of one shape (numel % 8 == 0)."""
     require_device(a, c)

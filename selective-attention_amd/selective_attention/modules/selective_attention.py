@@ -26,7 +26,7 @@ from __future__ import annotations
 import torch
 import torch.nn as nn
 
-from ..kernels.lm_ops import mha_gates
+from ..kernels.lm_ops import mha_gates, mha_prompt_gates
 from ..ops.attention import attn_varlen
 from ..ops.selective_mha import ScoreStdFn, gated_attention_train, selective_mha_prefill
 from .layers import Linear, RoPE, project
@@ -48,7 +48,7 @@ def _later_bool(flag: torch.Tensor):
     if not flag.is_cuda or torch.cuda.is_current_stream_capturing():
         value = bool(flag)
         return lambda: value
-    host = torch.empty((), dtype=torch.bool, pin_memory=True)
+    host = torch.empty(flag.shape, dtype=flag.dtype, pin_memory=True)
     host.copy_(flag, non_blocking=True)
     done = torch.cuda.Event()
     done.record(torch.cuda.current_stream(flag.device))
@@ -57,6 +57,18 @@ def _later_bool(flag: torch.Tensor):
         done.synchronize()
         return bool(host)
     return get
+
+
+def _one_kernel_gates(g, thr, lengths) -> bool:
+    """What mha_prompt_gates takes with the same values: bf16 on the GPU, a
+    threshold that float32 holds exactly, one integer length a row, and no
+    gradient asked of the gates."""
+    return (g.is_cuda and g.dtype == torch.bfloat16 and g.numel() > 0
+            and not (torch.is_grad_enabled() and g.requires_grad)
+            and (thr is None or (thr.dtype in (torch.float32, torch.bfloat16, torch.float16)
+                                 and thr.device == g.device))
+            and (lengths is None or (lengths.dtype in (torch.int32, torch.int64)
+                                     and lengths.shape == (g.shape[0],))))
 
 
 class SelectiveMHA(nn.Module):
@@ -110,22 +122,30 @@ class SelectiveMHA(nn.Module):
         b, L, _ = hidden_states.shape
         dev = hidden_states.device
         H, D = self.num_heads, self.head_dim
-        select_gate, out_gate = self._gates(hidden_states)
-        select_gate = select_gate.transpose(1, 2)                     # (b, H, L)
         thr = _threshold(attn_gate_threshold, H, dev)
-        kept = select_gate > 0.0
-        if thr is not None:
-            kept &= select_gate >= thr[None, :, None]
-        if lengths is not None:
-            lens = lengths.to(dev)
-            kept &= (torch.arange(L, device=dev)[None, :] < lens[:, None])[:, None, :]
+        g = self.gate_proj(hidden_states)
+        if _one_kernel_gates(g, thr, lengths):
+            # sigmoid, split, threshold, lengths and log-gate in one kernel
+            log_gate, out_gate, kept = mha_prompt_gates(
+                g, thr, self.score_std_ema, None if lengths is None else lengths.to(dev),
+                self.log_gate_penalty, H)
+        else:
+            select_gate, out_gate = torch.split(torch.sigmoid(g), [H, self.dim], dim=-1)
+            select_gate = select_gate.transpose(1, 2)                 # (b, H, L)
+            kept = select_gate > 0.0
+            if thr is not None:
+                kept &= select_gate >= thr[None, :, None]
+            if lengths is not None:
+                lens = lengths.to(dev)
+                kept &= (torch.arange(L, device=dev)[None, :] < lens[:, None])[:, None, :]
+            log_gate = self._log_gate(select_gate, kept)
+            kept = kept.any()
         v = self.v_proj(hidden_states)
-        any_kept = _later_bool(kept.any())
+        any_kept = _later_bool(kept)
         q, k = self.rope.rotate_qk(self.q_proj(hidden_states).view(b, L, H, D),
                                    self.k_proj(hidden_states).view(b, L, H, D), None, L)
         q, k = q.transpose(1, 2), k.transpose(1, 2)                   # (b, H, L, D) views
         vh = v.view(b, L, H, D).to(torch.bfloat16).transpose(1, 2)
-        log_gate = self._log_gate(select_gate, kept)
         if self.is_causal:
             out = selective_mha_prefill(q, k, vh, log_gate, lengths)
             if not any_kept():

@@ -272,3 +272,41 @@ def test_rope_keeps_fp32_frequencies_after_bf16_cast():
     ref = RoPE(64)                                       # ... the rotation still uses fp32 ones
     eq, _ = ref(q.float().cpu(), q.float().cpu(), pos.cpu(), "pos")
     assert ulp_bf16_close(yq.cpu(), eq.to(BF16), 1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("b,L,H,dim,thr,lens", [
+    (1, 1, 8, 64, None, None),
+    (2, 16, 16, 128, 0.4, [16, 3]),        # one block a row
+    (3, 37, 8, 512, 0.6, [37, 0, 21]),     # blocks across rows, a ragged last block
+    (2, 50, 6, 384, 0.5, None),            # heads off a multiple of 8: one column a thread
+    (2, 9, 4, 36, None, [5, 9]),
+    (1, 40, 8, 64, 2.0, None),             # nothing kept
+])
+def test_mha_prompt_gates_kernel(b, L, H, dim, thr, lens):
+    """log_gate, out_gate and the flag against torch's sigmoid, compare and log:
+    the gates to a bf16 rounding either way (2^-8), a log-gate to the same of
+    its gate plus fp32 rounding; kept or not by the kernel's own gate value."""
+    from selective_attention.kernels.lm_ops import mha_prompt_gates
+    g = torch.Generator().manual_seed(L)
+    z = (torch.randn(b, L, H + dim, generator=g) * 2).to(BF16)
+    z[0, 0, 0] = float("-inf")                       # gate 0: dropped
+    std = torch.rand(H, generator=g) + 0.5
+    t = None if thr is None else torch.full((H,), thr)
+    ln = None if lens is None else torch.tensor(lens)
+    print(f"mha_prompt_gates {b} {L} {H} {dim}", flush=True)
+    lg, og, flag = (x.cpu() for x in mha_prompt_gates(
+        z.cuda(), None if t is None else t.cuda(), std.cuda(), None if ln is None else ln.cuda(), 2.0, H))
+    s = torch.sigmoid(z.float())
+    torch.testing.assert_close(og.float(), s[..., H:], rtol=2 ** -8, atol=0)
+    sel = s[..., :H].to(BF16).float().transpose(1, 2)
+    kept = sel > 0
+    if t is not None:
+        kept &= sel >= t[None, :, None]
+    if ln is not None:
+        kept &= (torch.arange(L)[None] < ln[:, None])[:, None]
+    exp = torch.where(kept, torch.log(sel) * std[None, :, None] * 2.0, torch.tensor(float("-inf")))
+    near = torch.zeros_like(kept) if t is None else (sel - t[None, :, None]).abs() <= 2 ** -8 * sel
+    assert bool(((lg == exp) | near | ((lg - exp).abs() <= 2 ** -8 * 3 + 2 ** -20 * exp.abs())).all())
+    assert flag.item() == int((lg > float("-inf")).any())
+    assert flag.item() == int(bool(kept.any()))
