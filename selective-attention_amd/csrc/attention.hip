@@ -91,10 +91,17 @@ __device__ __forceinline__ int32_t load_uniform(const int32_t* p, int i) {
 //   kSelLong     a longer row, read slot by slot with scalar loads
 constexpr int kSelDense = 0, kSelShort = 1, kSelLong = 2;
 
-// Workgroups per CU the register budget is set for: at D = 64 (33 KB of LDS)
-// three, which none of the forms spills at; at D = 128 (66 KB) two.
+// Workgroups per CU the register budget is set for: at D = 64 a workgroup
+// holds 33 KB of LDS, so four fit (dense self-attention fits 128 VGPRs; the
+// table walks and the cross mode would spill there and take three); at
+// D = 128 (66 KB) two.
+template <int D, int MODE, int SEL>
+constexpr int attn_blocks_per_cu() {
+  return D == 64 ? (SEL == kSelDense && MODE != kCross ? 4 : 3) : 2;
+}
+
 template <int D, bool BIAS, int MODE, int SEL>
-__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void sparse_attn_fwd_kernel(
+__global__ __launch_bounds__(256, (attn_blocks_per_cu<D, MODE, SEL>())) void sparse_attn_fwd_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
     const int32_t* __restrict__ cu, const int32_t* __restrict__ cu_k, int nseq,
     const int32_t* __restrict__ block_idx, int n_qblk, int max_blocks, int grid_qblk,
@@ -267,8 +274,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void sparse_attn_fwd_kernel(
     }
   };
 
-  SoftmaxCol col[2];
-  col[0] = col[1] = SoftmaxCol{-1.f, 0.f, 0.f};
+  float m[2] = {kNegInf, kNegInf}, l[2] = {0.f, 0.f};
   v4f acc[2][DT];
 #pragma unroll
   for (int jt = 0; jt < 2; ++jt)
@@ -388,10 +394,12 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void sparse_attn_fwd_kernel(
       vfr[t] = __builtin_bit_cast(v8bf, __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7));
     }
     __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int jt = 0; jt < 2; ++jt) softmax_lazy<2, DT>(sc[jt], acc[jt], m[jt], l[jt], scl);
     // O^T += V^T . P^T over the wave's 32 keys
     {
-      const v8bf pb0 = softmax_col<DT>(sc[0], acc[0], col[0], scl);
-      const v8bf pb1 = softmax_col<DT>(sc[1], acc[1], col[1], scl);
+      const v8bf pb0 = pack_p(sc[0][0], sc[0][1]);
+      const v8bf pb1 = pack_p(sc[1][0], sc[1][1]);
 #pragma unroll
       for (int t = 0; t < DT; ++t) {
         acc[0][t] = mfma_bf16(vfr[t], pb0, acc[0][t]);
@@ -419,11 +427,8 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void sparse_attn_fwd_kernel(
   asm volatile("" ::: "memory");
 
   // the row sums so far are per lane (its own keys): add the four lane groups
-  float m[2], l[2];   // the columns' references (-inf: no key) and sums
 #pragma unroll
   for (int jt = 0; jt < 2; ++jt) {
-    m[jt] = col[jt].limit < 0.f ? kNegInf : -col[jt].neg;
-    l[jt] = col[jt].l;
     l[jt] += __shfl_xor(l[jt], 16, 64);
     l[jt] += __shfl_xor(l[jt], 32, 64);
   }

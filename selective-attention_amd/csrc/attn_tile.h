@@ -34,12 +34,65 @@ __device__ __forceinline__ int v_swz(int r) {
   else return (((r >> 1) & 1) << 2) | (((r >> 3) & 1) << 1) | ((r >> 4) & 1);
 }
 
-// Online softmax of one query column with a lazy reference (log2 domain): p =
+// Online softmax of the block-sparse kernel, with a lazy reference.  s[kt][i] holds log2-domain scores of
+// this lane's keys for query column lane & 15 (-inf where masked).  The
+// running reference m of a column (log2 domain, shared by its
+// four lane groups) is raised, and O and the partial sums rescaled, only when
+// some score exceeds it by more than 2^8: the common block needs no cross-lane
+// reduction at all, and probabilities stay <= 256.  l is this lane's partial
+// row sum (its own keys); the four lane groups' parts are added at the end.
+// The scores may come unscaled: the log2-domain score is s * sc (sc > 0), and
+// the scale is folded into the exponent's argument.
+// (softmax_col's sum test computes a row's first block twice; a block-sparse
+// row has 16 blocks at most: rows of 214 to 1284 tokens, H 16, took 350 us
+// with it and take 337 so at D = 128, 198 and 186 at D = 64, against 683 and
+// 687 us at 512 to 8192 tokens, D = 128.)
+template <int KT, int DT>
+__device__ __forceinline__ void softmax_lazy(v4f (&s)[KT], v4f (&o)[DT], float& m, float& l,
+                                             float sc = 1.0f) {
+  float mx = kNegInf;
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[kt][i]);
+  mx *= sc;
+  if (__ballot(mx > m + 8.0f)) {
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    if (mx > m + 8.0f) {   // the column's new reference
+      if (m != kNegInf) {   // (while m = -inf, every p so far was 0: l and o are 0)
+        const float alpha = fast_exp2(m - mx);
+        l *= alpha;
+#pragma unroll
+        for (int t = 0; t < DT; ++t) o[t] *= alpha;
+      }
+      m = mx;
+    }
+  }
+  // masked scores are -inf; a column without any admissible key yet keeps
+  // m = -inf and only -inf scores, so a zero reference gives p = 0 there
+  const float mref = m == kNegInf ? 0.0f : m;
+  float sum = 0.0f;
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float p = fast_exp2(fmaf(s[kt][i], sc, -mref));
+      s[kt][i] = p;
+      sum += p;
+    }
+  l += sum;
+}
+
+// Online softmax of one query column of the dense kernel (rows of many blocks),
+// with a lazy reference (log2 domain): p =
 // 2^(score - reference), the reference raised, and O and the lane's partial
 // row sum rescaled, only when needed.  A p above 2^8 shows in the sum of the
 // lane's eight p, which the row sum needs anyway: no maximum is taken in the
 // common block.  (The sum passes 2^8 without a single p above it at times;
-// the reference is then raised early, to the same effect.)
+// the reference is then raised early, to the same effect.)  A test that sends
+// the first block straight to the maximum costs the others more: 405 -> 435 us
+// (causal rows, b 4, H 16, L 8192).
 struct SoftmaxCol {
   float limit;   // sums above this raise the reference: 2^8, or -1 while there is none
   float neg;     // minus the reference; 0 while there is none
