@@ -2,8 +2,8 @@
 attention ops.
 
 Parameters and interfaces follow the reference.  Prefill runs
-selective_mha_prefill (the block-sparse kernel over every causal block with
-the log-gate as key bias) and fills the paged cache; step appends to the
+its gates (mha_prompt_gates) and selective_mha_prefill (dense causal attention
+over the batch rows with the log-gate as key bias) and fills the paged cache; step appends to the
 paged cache and runs the paged decode kernel.  A key whose gate is zeroed
 (below the threshold, or past a length) enters as key bias -inf: the
 reference's compression of the cache (its compressed branch, :63-83) drops
