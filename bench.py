@@ -341,7 +341,7 @@ def run_selective_mha(args, torch):
     pre_kernels = {n: round(x["avg_us"], 2) for n, x in kt.stats.items()}
     pairs = b * H * L * (L + 1) // 2
     flops = 4 * D * pairs
-    sp_us = pre_kernels.get("sparse_attn_fwd", ms_pre * 1e3)
+    sp_us = pre_kernels.get("dense_attn_fwd", ms_pre * 1e3)
     tf = flops / (sp_us / 1e6) / 1e12
 
     cache = PagedSelectiveAttnCache(b, H, D, max_tokens=L + 64, device=dev)
