@@ -136,8 +136,12 @@ class GatedAttnTrainFn(torch.autograd.Function):
         q, k, v, log_gate, out, stats = ctx.saved_tensors
         if torch.is_grad_enabled():
             need = ctx.needs_input_grad[:4]
-            dense = _gated_attention_dense(q, k, v, log_gate, ctx.causal)
-            wanted = [t for t, n in zip((q, k, v, log_gate), need) if n]
+            # aliases of their own: where one input was made from another, the
+            # derivative with respect to the inputs themselves would hold that
+            # path too, and the outer engine adds it once more
+            ts = [t.view_as(t) for t in (q, k, v, log_gate)]
+            dense = _gated_attention_dense(*ts, ctx.causal)
+            wanted = [t for t, n in zip(ts, need) if n]
             grads = iter(torch.autograd.grad(dense, wanted, dout, create_graph=True))
             return tuple(next(grads) if n else None for n in need) + (None,)
         return gated_attn_train_backward(q, k, v, log_gate, out, stats, dout, ctx.causal) + (None,)

@@ -159,3 +159,42 @@ def test_dense_form_on_the_cpu():
     assert not M._train_kernel_ok(q, k, v, lg)
     check(grads(gated_attention_train, (q, k, v, lg), do),
           grads(lambda *t: M._gated_attention_dense(*t, True), (q, k, v, lg), do, torch.float64))
+
+
+def _dependent(kind):
+    """Calls of gated_attention_train in which one input is made of another."""
+    if kind == "gate of q and k":
+        return lambda fn, q, k, v, lg: fn(q, k, v, lg + (q * k).sum(-1))
+    if kind == "one tensor for q, k and v":
+        return lambda fn, q, k, v, lg: fn(q, q, q, lg)
+    return lambda fn, q, k, v, lg: fn(q, 2.0 * q, v + k, lg)
+
+
+@pytest.mark.parametrize("kind", ["gate of q and k", "one tensor for q, k and v", "k of q"])
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_recorded_backward_of_dependent_inputs(kind, device, monkeypatch):
+    """First and second gradients where the inputs depend on each other, against
+    the dense form: a recorded backward differentiates with respect to the
+    inputs of this call alone.  On the CPU the function runs with the dense form
+    in the place of the kernels."""
+    q, k, v, lg, do = inputs(1, 2, 24, 64, device=device, seed=11)
+    lg = lg.clamp(min=-20.0)
+    fn = gated_attention_train
+    if device == "cpu":
+        def forward(q, k, v, lg, causal):
+            return M._gated_attention_dense(q, k, v, lg, causal), torch.zeros(2, *lg.shape)
+        monkeypatch.setattr(M, "gated_attn_train_forward", forward)
+        fn = lambda *t: M.GatedAttnTrainFn.apply(*t, True)
+
+    def both(fn, dtype):
+        ts = [t.to(dtype).requires_grad_(True) for t in (q, k, v, lg)]
+        out = _dependent(kind)(fn, *ts)
+        first = torch.autograd.grad(out, ts, do.to(dtype), create_graph=True, allow_unused=True)
+        first = [g for g in first if g is not None]
+        second = torch.autograd.grad(sum((g * g).sum() for g in first), ts, allow_unused=True)
+        return first + [g for g in second if g is not None]
+    got = both(fn, torch.float32)
+    want = both(lambda *t: M._gated_attention_dense(*t, True), torch.float64)
+    assert len(got) == len(want)
+    for a, e in zip(got, want):
+        assert float((a.double() - e).norm() / e.norm()) < 1e-4
