@@ -305,6 +305,9 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : 2) void dense_attn_kernel(DenseA
   if (nt > 0) {
     load_bias(0);
     store_bias(stage0);
+    // complete before the first barrier, as a step's own stores are by the wait
+    // that ends it: neither the barrier nor the wait on the DMA covers them
+    __builtin_amdgcn_s_waitcnt(kLgkmWait0);
     issue(0, lds_st0);
     if (nt > 1) load_bias(1);
   }
