@@ -570,8 +570,10 @@ __global__ __launch_bounds__(256) void f32_sum_kernel(const float4* __restrict__
   else dC[i - n4] = a;
 }
 
-// shares of a group's heads that bring `blocks` to about four per CU
+// shares of a group's heads that bring `blocks` to about four per CU (one for
+// an empty scan, which launches nothing)
 int head_shares(long blocks, int hpg) {
+  if (blocks <= 0) return 1;
   long want = (1024 + blocks - 1) / blocks;
   if (want > hpg) want = hpg;
   const int per = (hpg + static_cast<int>(want) - 1) / static_cast<int>(want);

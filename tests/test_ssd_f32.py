@@ -98,3 +98,38 @@ def test_other_sizes_keep_the_general_kernels(P, N, chunk):
     got, want = run_gpu(x, chunk), run_ref(x, chunk)
     for k, v in want.items():
         assert_parity(got[k], v, torch.float32, k)
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("b,L", [(0, 64), (2, 0), (0, 0), (1, 1)])
+@pytest.mark.parametrize("P,N", [(64, 64), (32, 128), (48, 64)])
+def test_workspace_of_empty_sizes(dtype, b, L, P, N):
+    """The workspace queries take an empty batch or sequence on every path (the
+    fp32 path divides a block count of the launch among the heads)."""
+    from selective_attention import _lib
+    lib = _lib.load()
+    nbytes = lib.sa_ssd_bwd_workspace_size(dtype, b, L, 2, P, 1, N, 64)
+    lib.sa_ssd_bwd_gated_workspace_size(dtype, b, L, 2, P, 1, N, 64)
+    assert (nbytes > 0) == (b * L > 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_empty_scans(dtype):
+    """An empty sequence passes the state and its gradient through; an empty
+    batch is refused, forward and backward, with an exception."""
+    from selective_attention.kernels.ssd_scan import ssd_scan_backward
+    x = make(2, 0, 4, 64, 64, 2, None, True, 0)
+    for k in ("u", "B", "C", "dr"):
+        x[k] = x[k].to(dtype)
+    out = run_gpu(x, 64)
+    assert not out["dA"].any() and not out["dbias"].any()
+    assert torch.equal(out["h"].cpu(), x["h0"]) and torch.equal(out["dh0"].cpu(), x["dh"])
+    x = make(0, 70, 4, 64, 64, 2, None, False, 0)
+    t = [x[k].to(dtype if k in ("u", "B", "C", "dr") else torch.float32).cuda()
+         for k in ("u", "A", "B", "C", "dr", "bias")]
+    with pytest.raises(RuntimeError):
+        SSDScanFn.apply(*t, None, None, 64)
+    saved = [torch.empty(s, device="cuda") for s in ((0, 4, 2, 64), (0, 4, 2, 64), (0, 2, 4, 64, 64))]
+    with pytest.raises(RuntimeError):
+        ssd_scan_backward(*t, None, x["dy"].cuda(), None, None, 64, saved=saved)
