@@ -120,9 +120,22 @@ def _gated_attention_dense(q, k, v, log_gate, causal):
     return torch.matmul(torch.softmax(s, dim=-1), v)
 
 
+def _needs_torch_ops(t: torch.Tensor) -> bool:
+    """Whether something has to see torch's own ops on t, which a kernel launch
+    hides or cannot serve: a functorch or legacy batched wrapper (vmap,
+    is_grads_batched), forward-mode AD, a dispatch mode, tracing."""
+    return (torch._C._functorch.is_functorch_wrapped_tensor(t)
+            or torch._C._functorch.is_legacy_batchedtensor(t)
+            or torch._C._are_functorch_transforms_active()
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch.compiler.is_compiling() or torch.jit.is_tracing())
+
+
 class GatedAttnTrainFn(torch.autograd.Function):
     """gated_attention_train on the fp32 MFMA kernels.  A backward that is itself
-    recorded (create_graph) differentiates the dense form instead."""
+    recorded (create_graph), batched over upstream gradients or in forward mode
+    differentiates the dense form instead."""
 
     @staticmethod
     def forward(ctx, q, k, v, log_gate, causal):
@@ -134,15 +147,17 @@ class GatedAttnTrainFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout):
         q, k, v, log_gate, out, stats = ctx.saved_tensors
-        if torch.is_grad_enabled():
+        recorded = torch.is_grad_enabled()
+        if recorded or _needs_torch_ops(dout):
             need = ctx.needs_input_grad[:4]
             # aliases of their own: where one input was made from another, the
             # derivative with respect to the inputs themselves would hold that
             # path too, and the outer engine adds it once more
-            ts = [t.view_as(t) for t in (q, k, v, log_gate)]
-            dense = _gated_attention_dense(*ts, ctx.causal)
+            with torch.enable_grad():
+                ts = [t.view_as(t) for t in (q, k, v, log_gate)]
+                dense = _gated_attention_dense(*ts, ctx.causal)
             wanted = [t for t, n in zip(ts, need) if n]
-            grads = iter(torch.autograd.grad(dense, wanted, dout, create_graph=True))
+            grads = iter(torch.autograd.grad(dense, wanted, dout, create_graph=recorded))
             return tuple(next(grads) if n else None for n in need) + (None,)
         return gated_attn_train_backward(q, k, v, log_gate, out, stats, dout, ctx.causal) + (None,)
 
@@ -159,10 +174,7 @@ def _train_kernel_ok(q, k, v, log_gate) -> bool:
             and q.shape[-1] in TRAIN_HEAD_DIMS and 0 < q.numel()
             and q.shape[0] * q.shape[1] * ((q.shape[2] + 63) // 64) < 2 ** 31
             and not torch.is_autocast_enabled("cuda")
-            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
-            and not torch._C._are_functorch_transforms_active()
-            and torch.autograd.forward_ad._current_level < 0
-            and torch._C._len_torch_dispatch_stack() == 0)
+            and not any(_needs_torch_ops(t) for t in ts))
 
 
 def gated_attention_train(q_rot, k_rot, v, log_gate, causal=True):

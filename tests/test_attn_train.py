@@ -201,3 +201,39 @@ def test_recorded_backward_of_dependent_inputs(kind, device, monkeypatch):
     assert len(got) == len(want)
     for a, e in zip(got, want):
         assert float((a.double() - e).norm() / e.norm()) < 1e-4
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_batched_and_dual_upstream_gradients(device, monkeypatch):
+    """A backward that is vectorised over upstream gradients, or run with a
+    forward-mode tangent on one, sees the dense form's ops."""
+    q, k, v, lg, do = inputs(1, 2, 24, 64, device=device, seed=12)
+    lg = lg.clamp(min=-20.0)
+    fn = gated_attention_train
+    if device == "cpu":
+        def forward(q, k, v, lg, causal):
+            return M._gated_attention_dense(q, k, v, lg, causal), torch.zeros(2, *lg.shape)
+
+        def backward(q, k, v, lg, out, stats, dout, causal):
+            dout.data_ptr()
+            return tuple(torch.zeros_like(t) for t in (q, k, v, lg))
+        monkeypatch.setattr(M, "gated_attn_train_forward", forward)
+        monkeypatch.setattr(M, "gated_attn_train_backward", backward)
+        fn = lambda *t: M.GatedAttnTrainFn.apply(*t, True)
+    G = torch.stack([do, 2.0 * do.flip(2), torch.zeros_like(do)])
+
+    def run(fn, how):
+        ts = [t.detach().requires_grad_(True) for t in (q, k, v, lg)]
+        out = fn(*ts)
+        if how == "is_grads_batched":
+            return torch.autograd.grad(out, ts, G, is_grads_batched=True)
+        if how == "vmap":
+            return torch.vmap(lambda g: torch.autograd.grad(out, ts, g, retain_graph=True))(G)
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(G[0], G[1])
+            pairs = [torch.autograd.forward_ad.unpack_dual(g) for g in torch.autograd.grad(out, ts, dual)]
+            return [t for p in pairs for t in (p.primal, p.tangent)]
+    for how in ("is_grads_batched", "vmap", "dual"):
+        got, want = run(fn, how), run(lambda *t: M._gated_attention_dense(*t, True), how)
+        for a, e in zip(got, want):
+            torch.testing.assert_close(a, e, rtol=1e-4, atol=1e-5)
