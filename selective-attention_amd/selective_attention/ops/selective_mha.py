@@ -77,7 +77,7 @@ class ScoreStdFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, g):
         q, k, stats = ctx.saved_tensors
-        if torch.is_grad_enabled():      # a recorded backward: torch ops by query chunks
+        if torch.is_grad_enabled() or _needs_torch_ops(g):   # torch ops by query chunks
             dq, dk = _score_std_backward_dense(q, k, stats, g, ctx)
         else:
             dq, dk = score_std_backward(q, k, ctx.q_lengths, ctx.k_lengths, ctx.causal, stats, g)

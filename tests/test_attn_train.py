@@ -237,3 +237,29 @@ def test_batched_and_dual_upstream_gradients(device, monkeypatch):
         got, want = run(fn, how), run(lambda *t: M._gated_attention_dense(*t, True), how)
         for a, e in zip(got, want):
             torch.testing.assert_close(a, e, rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+def test_score_std_dual_upstream_gradient(device, monkeypatch):
+    """The std's backward is linear in the upstream gradient: its tangent is the
+    backward of the tangent."""
+    from oracle import attn as ref
+    q, k, *_ = inputs(1, 2, 24, 64, device=device, seed=13)
+    if device == "cpu":
+        def moments(q, k, ql, kl, causal):
+            st = ref.score_stats(q.double(), k.double(), 64 ** -0.5, ql, kl, causal)
+            return st, ref.score_std(st).float()
+        monkeypatch.setattr(M, "score_moments", moments)
+        monkeypatch.setattr(M, "score_std_backward", lambda q, k, *a: (torch.zeros_like(q), torch.zeros_like(k)))
+    ts = [t.requires_grad_(True) for t in (q, k)]
+    std = M.ScoreStdFn.apply(*ts)
+    g, tangent = torch.tensor([1.0, -2.0], device=device), torch.tensor([0.5, 3.0], device=device)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(g, tangent)
+        got = [torch.autograd.forward_ad.unpack_dual(x)
+               for x in torch.autograd.grad(std, ts, dual, retain_graph=True)]
+        got = [(x.primal.clone(), x.tangent.clone()) for x in got]
+    for i, up in enumerate((g, tangent)):
+        want = torch.autograd.grad(std, ts, up, create_graph=True)
+        for x, e in zip(got, want):
+            torch.testing.assert_close(x[i], e.detach(), rtol=1e-5, atol=1e-7)
