@@ -195,7 +195,8 @@ int sa_attn_varlen_fwd(int dtype, int mode, const void* q, const void* k, const 
  * 27-144, mode "seq"): mode 0 of sa_attn_varlen_fwd with each row's first
  * lengths[row] tokens as a sequence (lengths (batch,) int64 or NULL: all of
  * seq_len); the other rows of o are zeros.
- *   q, k, v, o: (batch, seq_len, num_heads, head_dim) bf16, head_dim in {64,128}
+ *   q, k, v, o: (batch, seq_len, num_heads, head_dim) bf16 on 16-byte boundaries,
+ *   head_dim in {64,128}
  *   log_gate: (batch, num_heads, seq_len) f32 key bias, not applied on j = i
  */
 int sa_mha_prefill_fwd(int dtype, const void* q, const void* k, const void* v,

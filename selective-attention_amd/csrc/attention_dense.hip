@@ -411,6 +411,9 @@ extern "C" int sa_mha_prefill_fwd(int dtype, const void* q, const void* k, const
                    static_cast<int64_t>(batch) * seq_len < (1LL << 31),
                "sa_mha_prefill_fwd: bad sizes");
   SA_CHECK_ARG(q && k && v && log_gate && o, "sa_mha_prefill_fwd: null pointer");
+  SA_CHECK_ARG(((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
+                 reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(o)) & 15) == 0,
+               "sa_mha_prefill_fwd: q, k, v and o must be 16-byte aligned");
   if (batch == 0 || seq_len == 0) return 0;
   const float scale = softmax_scale > 0.f ? softmax_scale : 1.0f / sqrtf(static_cast<float>(head_dim));
   sa::DenseArgs a{};

@@ -22,6 +22,13 @@ def _i32(t: torch.Tensor) -> torch.Tensor:
     return t if t.dtype == torch.int32 and t.is_contiguous() else t.to(torch.int32).contiguous()
 
 
+def _rows16(t: torch.Tensor) -> torch.Tensor:
+    """t contiguous on a 16-byte boundary, which the dense kernel's row copies need
+    (a view into a larger buffer may start anywhere)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def sparse_attn_varlen(q, k, v, cu_seqlens, block_idx, block_size=64, softmax_scale=None,
                        key_bias=None):
     """
@@ -89,7 +96,7 @@ def attn_varlen(q, k, v, cu_seqlens_q, mode="causal", cu_seqlens_k=None, key_bia
     for t in (q, k, v):
         if t.dtype != torch.bfloat16:
             raise TypeError("attn_varlen: q, k, v must be bfloat16")
-    q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
+    q, k, v = _rows16(q), _rows16(k), _rows16(v)
     cu_q = _i32(cu_seqlens_q)
     cu_k = None if cu_seqlens_k is None else _i32(cu_seqlens_k)
     bias = None if key_bias is None else key_bias.to(torch.float32).contiguous()
@@ -106,7 +113,7 @@ def mha_prefill(q, k, v, log_gate, lengths=None):
     SelectiveMHA's prefill attention over batch rows (sa_mha_prefill_fwd).
 
     Args:
-        q, k, v: (batch, seq_len, num_heads, head_dim) bfloat16, contiguous
+        q, k, v: (batch, seq_len, num_heads, head_dim) bfloat16
         log_gate: (batch, num_heads, seq_len) float32 key bias, not applied to
             a query's own key
         lengths: (batch,) int64 or None; rows at or past a length come out 0
@@ -116,6 +123,7 @@ def mha_prefill(q, k, v, log_gate, lengths=None):
     """
     require_device(q, k, v, log_gate, lengths)
     b, L, H, D = q.shape
+    q, k, v = _rows16(q), _rows16(k), _rows16(v)
     o = torch.empty_like(q)
     _lib.call("sa_mha_prefill_fwd", _lib.DTYPE_BF16, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v),
               _lib.ptr(log_gate), _lib.ptr(lengths), b, L, H, D, -1.0, _lib.ptr(o),

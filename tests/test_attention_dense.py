@@ -89,3 +89,38 @@ def test_rows(b, H, L, D, lens):
                 assert_parity(o[i, h, :n], want.cpu(), torch.bfloat16, f"row {i} head {h}")
     # any other layout is copied: the same bits
     assert torch.equal(o, selective_mha_prefill(q.contiguous(), k, v.contiguous(), lg, lt))
+
+
+def test_prefill_entry_refuses_misaligned_rows():
+    """The kernel moves rows 16 bytes at a time; an odd pointer is an error, not a
+    launch (the addresses are never read: the checks come first)."""
+    from selective_attention import _lib
+    lib = _lib.load()
+    for bad in range(5):
+        p = [0x1000 * (i + 1) for i in range(5)]   # q, k, v, log_gate, o
+        p[bad] += 2
+        q, k, v, lg, o = p
+        rc = lib.sa_mha_prefill_fwd(_lib.DTYPE_BF16, q, k, v, lg, None, 0, 64, 4, 64, -1.0, o, None)
+        assert (rc != 0) == (bad != 3), bad
+        if rc:
+            assert b"aligned" in lib.sa_last_error()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("off", [1, 4, 8])
+def test_rows_off_a_16_byte_boundary(off):
+    """Contiguous views `off` elements into a buffer: the aligned call's bits."""
+    b, H, L, D = 2, 3, 150, 64
+    g = torch.Generator(device="cuda").manual_seed(off)
+
+    def odd(t):
+        return torch.empty(t.numel() + off, device="cuda", dtype=t.dtype)[off:].view(t.shape).copy_(t)
+    q, k, v = (torch.randn(b, L, H, D, generator=g, device="cuda").bfloat16() for _ in range(3))
+    lg = -torch.rand(b, H, L, generator=g, device="cuda")
+    want = selective_mha_prefill(*(t.transpose(1, 2) for t in (q, k, v)), lg)
+    assert torch.equal(want, selective_mha_prefill(*(odd(t).transpose(1, 2) for t in (q, k, v)), odd(lg)))
+    n, Hn = 4200, 16      # a packed launch of the same kernel
+    q, k, v = (torch.randn(n, Hn, D, generator=g, device="cuda").bfloat16() for _ in range(3))
+    bias = -torch.rand(Hn, n, generator=g, device="cuda")
+    assert torch.equal(attn_varlen(q, k, v, cu_of([n]), "full", None, bias),
+                       attn_varlen(odd(q), odd(k), odd(v), cu_of([n]), "full", None, odd(bias)))
