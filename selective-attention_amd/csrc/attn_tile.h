@@ -130,11 +130,9 @@ __device__ __forceinline__ v8bf softmax_col(const v4f (&s)[2], v4f (&o)[DT], Sof
       c.neg = -ref;
       c.limit = 256.0f;
     }
+    // (a column without a reference has met masked keys, whose p are 0, and
+    // scores that are no numbers, whose p have to stay)
     sum = exp_sum(s, p, sc, c.neg);
-    if (c.limit < 0.f) {   // masked keys only so far
-      sum = 0.f;
-      p[0] = p[1] = v4f{0.f, 0.f, 0.f, 0.f};
-    }
   }
   c.l += sum;
   return pack_p(p[0], p[1]);

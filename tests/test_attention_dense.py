@@ -124,3 +124,51 @@ def test_rows_off_a_16_byte_boundary(off):
     bias = -torch.rand(Hn, n, generator=g, device="cuda")
     assert torch.equal(attn_varlen(q, k, v, cu_of([n]), "full", None, bias),
                        attn_varlen(odd(q), odd(k), odd(v), cu_of([n]), "full", None, odd(bias)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 128])
+def test_nan_and_infinite_rows(D):
+    """A query, key or value that is not a number shows in every row that meets
+    it and in no other: rows of one half tile (0, 5, 31) and of several."""
+    b, H, L = 1, 4, 200
+    g = torch.Generator(device="cuda").manual_seed(D)
+    base = [torch.randn(b, L, H, D, generator=g, device="cuda").bfloat16() for _ in range(3)]
+    lg = -torch.rand(b, H, L, generator=g, device="cuda")
+    run = lambda q, k, v: selective_mha_prefill(*(t.transpose(1, 2) for t in (q, k, v)), lg).transpose(1, 2)
+    clean = run(*base)
+    for row in (0, 5, 31, 32, 130):
+        q = base[0].clone()
+        q[0, row, 1, 3] = float("nan")
+        o = run(q, *base[1:])
+        assert o[0, row, 1].isnan().all()
+        o[0, row, 1] = clean[0, row, 1]
+        torch.testing.assert_close(o, clean, rtol=2e-2, atol=2e-2)
+        for value in (float("nan"), float("inf")):   # (inf - inf in the softmax)
+            k = base[1].clone()
+            k[0, row, 1, 3] = value
+            o = run(base[0], k, base[2])
+            hit = base[0][0, row:, 1, 3] > 0 if value > 0 else torch.ones(L - row, dtype=torch.bool, device="cuda")
+            assert o[0, row:, 1][hit].isnan().all()
+            torch.testing.assert_close(o[0, :row], clean[0, :row], rtol=2e-2, atol=2e-2)
+    # packed: a sequence of one half tile, and a cross range of few keys
+    n, Hn = 4200, 16
+    q, k, v = (torch.randn(n, Hn, D, generator=g, device="cuda").bfloat16() for _ in range(3))
+    q[4100, 2, 0] = float("nan")
+    cu = cu_of([4096, 20, 84])
+    for mode, cuk in (("causal", None), ("full", None), ("cross", cu_of([4096, 20, 84]))):
+        o = attn_varlen(q, k, v, cu, mode, cuk)
+        assert o[4100, 2].isnan().all() and int(o.isnan().any(-1).sum()) == 1, mode
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("low", [torch.finfo(torch.float32).min, -1e30])
+def test_biases_of_the_lowest_value(low):
+    """A mask written as a huge finite bias drops its keys as -inf does."""
+    b, H, L, D = 2, 2, 150, 64
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn(b, L, H, D, generator=g, device="cuda").bfloat16().transpose(1, 2) for _ in range(3))
+    drop = torch.rand(b, H, L, generator=g, device="cuda") < 0.5
+    lg = -torch.rand(b, H, L, generator=g, device="cuda")
+    want = selective_mha_prefill(q, k, v, lg.masked_fill(drop, float("-inf")))
+    assert torch.equal(selective_mha_prefill(q, k, v, lg.masked_fill(drop, low)), want)

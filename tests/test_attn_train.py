@@ -200,7 +200,7 @@ def test_recorded_backward_of_dependent_inputs(kind, device, monkeypatch):
     want = both(lambda *t: M._gated_attention_dense(*t, True), torch.float64)
     assert len(got) == len(want)
     for a, e in zip(got, want):
-        assert float((a.double() - e).norm() / e.norm()) < 1e-4
+        assert float(((a.double() - e).norm() / e.norm()).detach()) < 1e-4
 
 
 @pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
