@@ -109,7 +109,12 @@ template <int DT>
 __device__ __forceinline__ v8bf softmax_col(const v4f (&s)[2], v4f (&o)[DT], SoftmaxCol& c, float sc) {
   v4f p[2];
   float sum = exp_sum(s, p, sc, c.neg);
-  if (__ballot(sum > c.limit)) {
+  const uint64_t vote = __ballot(sum > c.limit);
+  if (vote) {
+    // a column's four lane groups share the reference and decide by their own
+    // sums alone: a row's bits do not depend on the rows beside it
+    const uint32_t half = static_cast<uint32_t>(vote) | static_cast<uint32_t>(vote >> 32);
+    const bool mine = ((half | half >> 16) >> (threadIdx.x & 15)) & 1;
     float mx = kNegInf;
 #pragma unroll
     for (int u = 0; u < 2; ++u)
@@ -118,8 +123,7 @@ __device__ __forceinline__ v8bf softmax_col(const v4f (&s)[2], v4f (&o)[DT], Sof
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
     mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
     const float ref = mx * sc;
-    // a column's four lane groups share the reference, so they decide alike
-    const bool up = c.limit < 0.f ? mx > kNegInf : ref > -c.neg;
+    const bool up = mine && (c.limit < 0.f ? mx > kNegInf : ref > -c.neg);
     if (up) {
       if (c.limit > 0.f) {
         const float alpha = fast_exp2(-c.neg - ref);

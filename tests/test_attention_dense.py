@@ -172,3 +172,20 @@ def test_biases_of_the_lowest_value(low):
     lg = -torch.rand(b, H, L, generator=g, device="cuda")
     want = selective_mha_prefill(q, k, v, lg.masked_fill(drop, float("-inf")))
     assert torch.equal(selective_mha_prefill(q, k, v, lg.masked_fill(drop, low)), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,L,H", [(64, 300, 4), (128, 300, 4), (64, 4200, 16)])
+def test_a_row_does_not_see_its_neighbours(D, L, H):
+    """Other queries of the same tile, whose scores rise far above theirs (or are
+    no numbers), leave a row's bits alone."""
+    g = torch.Generator(device="cuda").manual_seed(L)
+    q, k, v = (torch.randn(1, L, H, D, generator=g, device="cuda").bfloat16() for _ in range(3))
+    lg = -torch.rand(1, H, L, generator=g, device="cuda")
+    run = lambda q: selective_mha_prefill(*(t.transpose(1, 2) for t in (q, k, v)), lg).transpose(1, 2)
+    clean, rows = run(q), torch.arange(3, L, 7, device="cuda")
+    keep = torch.ones(L, dtype=torch.bool, device="cuda").index_fill(0, rows, False)
+    for other in (20.0 * q[:, rows], -20.0 * q[:, rows], float("nan") * q[:, rows]):
+        mixed = q.clone()
+        mixed[:, rows] = other
+        assert torch.equal(run(mixed)[:, keep], clean[:, keep])
