@@ -1100,8 +1100,9 @@ extern "C" int sa_attn_varlen_fwd(int dtype, int mode, const void* q, const void
   const float scale = softmax_scale > 0.f ? softmax_scale : 1.0f / sqrtf(static_cast<float>(head_dim));
   const int32_t* cu_k = mode == sa::kCross ? cu_seqlens_k : cu_seqlens_q;
   const int Tk = mode == sa::kCross ? total_k : total_q;
-  // launches that fill the chip with 128-query blocks: attention_dense.hip
-  if (sa::dense_attn_ok(num_heads, total_q))
+  // launches that fill the chip with 128-query blocks: attention_dense.hip.  It
+  // holds biases as bias / scale, which must not overflow
+  if (sa::dense_attn_ok(num_heads, total_q) && (!key_bias || scale >= 0x1p-20f))
     return sa::launch_dense_varlen(mode, head_dim, q, k, v, cu_seqlens_q, cu_k, num_seqs, key_bias, o,
                                    total_q, Tk, num_heads, scale * sa::kLog2e, s);
   // upper bound on the query blocks (sum over sequences of ceil(len / 64));

@@ -189,3 +189,19 @@ def test_a_row_does_not_see_its_neighbours(D, L, H):
         mixed = q.clone()
         mixed[:, rows] = other
         assert torch.equal(run(mixed)[:, keep], clean[:, keep])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1e-39, 1e-36, 1e-6, 1.0])
+def test_any_softmax_scale(scale):
+    """Down to scales whose reciprocal leaves the range: only the biases count."""
+    H, n, D = 16, 4200, 64
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn(n, H, D, generator=g, device="cuda").bfloat16() for _ in range(3))
+    bias = 300.0 * torch.rand(H, n, generator=g, device="cuda")
+    o = attn_varlen(q, k, v, cu_of([n]), "full", None, bias, scale)
+    for h in (0, 9):
+        s = q[:200, h].double() @ k[:, h].double().T * scale + bias[h].double()
+        i = torch.arange(200, device="cuda")
+        s[i, i] -= bias[h, :200].double()
+        assert_parity(o[:200, h], (torch.softmax(s, -1) @ v[:, h].double()).cpu(), torch.bfloat16, f"head {h}")
