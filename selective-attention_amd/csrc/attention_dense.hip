@@ -365,7 +365,16 @@ int launch_dense(const DenseArgs& a, hipStream_t s) {
 
 }  // namespace
 
-// 128-query blocks: two and more of them for every CU
+// 128-query blocks: two and more of them for every CU.  The tokens are counted,
+// not the sequences: a pack of short ones leaves waves without queries and
+// empty blocks behind, and is still the faster here, since a tile's 64-query
+// blocks (four waves that share its keys) and their merge cost more.  Packs past
+// this line, block-sparse kernel -> here, H 16, D 64, causal with biases: 256
+// sequences of 16 tokens 25.4 -> 21.5 us, 32: 31 -> 25, 64: 42 -> 38, 100: 66 ->
+// 50, 200: 168 -> 106; 1024 of 32: 195 -> 158, of 100: 428 -> 302 us.  Over 4 and
+// 16 heads, both head_dims, all modes, 64 to 1024 sequences of 16 to 1000
+// tokens: 0.93 to 2.1 times as fast, 1.3 in the middle (below 1 at 4 heads and
+// 256 sequences of 80 to 128 tokens alone).
 bool dense_attn_ok(int num_heads, int total_q) {
   return static_cast<long>(num_heads) * (total_q / 128) >= 512;
 }
