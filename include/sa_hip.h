@@ -262,8 +262,10 @@ int sa_score_stats(int dtype, const void* q, const void* k, const int64_t* q_len
                    double* out, void* stream);
 
 /*
- * The same statistics without visiting every pair (Gram matrices of the keys),
- * and the gradient of the per-head std.  `out` (heads, 3) as sa_score_stats;
+ * The same statistics without visiting every pair (Gram matrices of the keys,
+ * in fp64), and the gradient of the per-head std.  The workspace grows with
+ * heads and head_dim: batch heads ceil(len / 256) (head_dim^2 + head_dim) 8
+ * bytes, about the size of k in fp32 at head_dim 128.  `out` (heads, 3) as sa_score_stats;
  * `std` (heads,) fp32 or NULL: sqrt(max(sum^2 / n - (sum / n)^2, 0)).
  * sa_score_std_bwd: for stats = out of sa_score_moments and std_grad (heads,)
  * fp32, dq and dk (shapes and dtype of q and k) of std_grad . std; a head of

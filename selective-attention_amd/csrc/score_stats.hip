@@ -32,11 +32,25 @@
 // dk) over the chunks (score_gram_scan_kernel), and in score_apply_kernel
 // the chunk's own pairs as 64x64 score tiles.  Work per row: 4 D^2 FLOP for
 // the Gram matrix and its product and 160 pairs on average, against L / 2
-// pairs.  All products are fp32 MFMA (bf16 inputs are widened); at b 4, H 8,
-// L 2048, D 64, fp32: statistics 51 us (Gram 12, scan 5, apply 33; the pass
-// over every pair 202), gradient 123 us (the same in torch ops by query chunks
-// of the dense scores 2.7 ms).  sa_score_stats keeps the pass over every pair
-// for callers that size its workspace without the key length and head_dim.
+// pairs.
+// Precision.  q . M q and scale M q - mean kappa cancel where rows share a
+// component, as sum^2 / n - mean^2 does, so everything that stands for a sum over
+// pairs is fp64: the Gram matrices (exact products of fp32 values on
+// v_mfma_f64_16x16x4_f64), their scan, the products with them, and the sums over
+// the scores and over a chunk's tiles.  fp32 is the score of one pair and a
+// gradient's sum over one 64-row tile.  The std's error is that of its rounding
+// (at most 5e-8, also with common parts of 100 standard deviations), the
+// gradients' at most 6e-8 without a common part and below the dense fp32 form's
+// with one (q and k offset by 10: 5e-8 for 3e-7; k by 100, across q: 6e-7 for
+// 1.2e-6).  With fp32 Gram matrices the std was off by 1.5e-5 and a gradient by
+// 5e-5 there, for 17 us and 40 us less:
+// at b 4, H 8, L 2048, D 64, fp32: statistics 69 us (Gram 16, scan 5, apply 43,
+// reduction 5; the pass over every pair 202), gradient 163 us (the same in torch
+// ops by query chunks of the dense scores 2.7 ms).
+// Memory: b H ceil(L / 256) (D^2 + D) doubles of workspace, about the size of k
+// itself in fp32 at D 128 and half of it at D 64 (b 8, H 16, L 32768, D 128:
+// 2.2 GB).  sa_score_stats keeps the pass over every pair for callers that size
+// its workspace without the key length and head_dim.
 #include "common.h"
 #include "fp32_tile.h"
 #include "prof.h"
@@ -183,6 +197,14 @@ __global__ __launch_bounds__(256) void score_stats_reduce_kernel(const double* _
 // moments through Gram matrices
 // ---------------------------------------------------------------------------
 constexpr int kChunk = 256;   // rows of a Gram matrix
+
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef double v4d __attribute__((ext_vector_type(4)));
+// 16x16 += 16x4 . 4x16: lane l supplies A row l % 16 and B column l % 16 at
+// k = l / 16 and holds result rows l / 16 + 4 i (not 4 (l / 16) + i as in fp32)
+__device__ __forceinline__ v4d mfma_f64(double a, double b, const v4d& c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
 enum class Pairs { kBefore, kAfter, kAll };   // keys y <= x, y >= x, every y
 
 __device__ __forceinline__ int row_count(const int64_t* length, int b, int L) {
@@ -194,18 +216,18 @@ __device__ __forceinline__ int row_count(const int64_t* length, int b, int L) {
 template <typename T, int D>
 __global__ __launch_bounds__(256) void score_gram_kernel(const T* __restrict__ y,
                                                          const int64_t* __restrict__ length, int H,
-                                                         int L, int nc, float* __restrict__ gram) {
+                                                         int L, int nc, double* __restrict__ gram) {
   constexpr int NT = D / 16, NP = NT * NT / 4;
   __shared__ __align__(16) float yt[kRows * (D + 4)];
   const int bh = blockIdx.x / nc, c = blockIdx.x % nc;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, li = lane & 15, lg = lane >> 4;
   const int len = row_count(length, bh / H, L);
   const T* yh = y + static_cast<long>(bh) * L * D;
-  float* out = gram + static_cast<long>(blockIdx.x) * (D * D + D);
-  v4f acc[NP];
+  double* out = gram + static_cast<long>(blockIdx.x) * (D * D + D);
+  v4d acc[NP];
 #pragma unroll
-  for (int j = 0; j < NP; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
-  float sum = 0.f;
+  for (int j = 0; j < NP; ++j) acc[j] = v4d{0.0, 0.0, 0.0, 0.0};
+  double sum = 0.0;
   TileRegs<D> yr;
   const int r1 = min(kChunk * (c + 1), len);   // (may lie before the chunk: zeros are written)
   tile_load<D>(yr, yh, D, kChunk * c, r1, tid);
@@ -219,20 +241,21 @@ __global__ __launch_bounds__(256) void score_gram_kernel(const T* __restrict__ y
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float* row = yt + (16 * t + 4 * lg + i) * (D + 4) + li;
-        float a[NT];
+        // tile pair p = w + 4 j, (row tile p / NT, column tile p % NT)
+        if constexpr (NT % 4 == 0) {
+          double a[NT], z[NT / 4];
 #pragma unroll
-        for (int n = 0; n < NT; ++n) a[n] = row[16 * n];
+          for (int n = 0; n < NT; ++n) a[n] = row[16 * n];
 #pragma unroll
-        for (int j = 0; j < NP; ++j) {
-          // tile pair w + 4 j; w is wave-uniform, so the selects are scalar
-          const int p = w + 4 * j;
-          float x = 0.f, z = 0.f;
+          for (int n = 0; n < NT / 4; ++n) z[n] = row[16 * (4 * n + w)];
 #pragma unroll
-          for (int n = 0; n < NT; ++n) {
-            x = p / NT == n ? a[n] : x;
-            z = p % NT == n ? a[n] : z;
+          for (int j = 0; j < NP; ++j) acc[j] = mfma_f64(a[4 * j / NT], z[j % (NT / 4)], acc[j]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < NP; ++j) {
+            const int p = w + 4 * j;
+            acc[j] = mfma_f64(row[16 * (p / NT)], row[16 * (p % NT)], acc[j]);
           }
-          acc[j] = mfma_f32(x, z, acc[j]);
         }
       }
     if (tid < D)
@@ -243,7 +266,7 @@ __global__ __launch_bounds__(256) void score_gram_kernel(const T* __restrict__ y
     const int p = w + 4 * j;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      out[(16 * (p / NT) + 4 * lg + i) * D + 16 * (p % NT) + li] = acc[j][i];
+      out[(16 * (p / NT) + lg + 4 * i) * D + 16 * (p % NT) + li] = acc[j][i];
   }
   if (tid < D) out[D * D + tid] = sum;
 }
@@ -251,14 +274,14 @@ __global__ __launch_bounds__(256) void score_gram_kernel(const T* __restrict__ y
 // over the chunks of one (batch row, head), in place: each slot becomes the sum
 // of the slots before it (kBefore), after it (kAfter); kAll: slot 0 the total
 template <Pairs PAIRS>
-__global__ __launch_bounds__(256) void score_gram_scan_kernel(float* __restrict__ gram, int nc,
+__global__ __launch_bounds__(256) void score_gram_scan_kernel(double* __restrict__ gram, int nc,
                                                               int size) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i >= size) return;
-  float* g = gram + static_cast<long>(blockIdx.y) * nc * size + i;
-  float run = 0.f;
+  double* g = gram + static_cast<long>(blockIdx.y) * nc * size + i;
+  double run = 0.0;
   for (int c0 = 0; c0 < nc; c0 += 8) {
-    float t[8];
+    double t[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int c = min(c0 + u, nc - 1);
@@ -283,7 +306,7 @@ template <typename T, int D, Pairs PAIRS, bool STATS>
 __global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void score_apply_kernel(
     const T* __restrict__ x, const T* __restrict__ y, const int64_t* __restrict__ x_length,
     const int64_t* __restrict__ y_length, int H, int Lx, int Ly, int nc, float scale,
-    const float* __restrict__ gram, const double* __restrict__ stats, const float* __restrict__ g,
+    const double* __restrict__ gram, const double* __restrict__ stats, const float* __restrict__ g,
     double* __restrict__ part, T* __restrict__ dx) {
   constexpr int NT = D / 16;
   __shared__ __align__(16) float yt[kRows * (D + 4)];
@@ -295,53 +318,57 @@ __global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void score_apply_kernel(
   const T* yh = y + static_cast<long>(bh) * Ly * D;
   const int xi = kRows * xb + 16 * w + li;
   const long row = static_cast<long>(bh) * Lx + min(xi, Lx - 1);
-  v4f xf[NT], acc[NT];
+  v4f xf[NT];
+  v4d mx[NT];   // M x, then the row's gradient
   row_frag<D>(xf, x + row * D, lg, xi < xlen);
 #pragma unroll
-  for (int i = 0; i < NT; ++i) acc[i] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int n = 0; n < NT; ++n) mx[n] = v4d{0.0, 0.0, 0.0, 0.0};
 
-  float coef = 0.f, mean = 0.f;
+  double coef = 0.0, mean = 0.0;
   if (!STATS) {
     const double n = fmax(stats[3 * h], 1.0), mu = stats[3 * h + 1] / n;
     const double var = stats[3 * h + 2] / n - mu * mu, sd = sqrt(var < 0.0 ? 0.0 : var);
-    coef = sd > 0.0 ? static_cast<float>(static_cast<double>(g[h]) / (n * sd)) : 0.f;
-    mean = static_cast<float>(mu);
+    coef = sd > 0.0 ? static_cast<double>(g[h]) / (n * sd) : 0.0;
+    mean = mu;
   }
 
   // rows y outside the chunk, through their Gram matrix
   const int c = PAIRS == Pairs::kAll ? 0 : kRows * xb / kChunk;
-  const bool outside = PAIRS == Pairs::kAll || (PAIRS == Pairs::kBefore ? c > 0 : c + 1 < nc);
+  const bool outside =
+      PAIRS == Pairs::kAfter ? c + 1 < nc : PAIRS == Pairs::kAll || c > 0;
   double s1 = 0.0, s2 = 0.0;
   if (outside) {
-    const float* gm = gram + (static_cast<long>(bh) * nc + c) * (D * D + D);
+    const double* gm = gram + (static_cast<long>(bh) * nc + c) * (D * D + D);
+    // row 4 (li % 4) + li / 4 of a 16-row tile as A row li: result element i of
+    // lane group lg is then row 4 lg + i of the tile, as in xf
+    const double* gr = gm + (4 * (li & 3) + (li >> 2)) * D + 4 * lg;
 #pragma unroll
     for (int s = 0; s < NT; ++s) {
-      v4f a[NT];
+      v2d a[NT][2];
 #pragma unroll
       for (int n = 0; n < NT; ++n)
-        a[n] = *reinterpret_cast<const v4f*>(gm + (16 * n + li) * D + 16 * s + 4 * lg);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          a[n][i] = *reinterpret_cast<const v2d*>(gr + 16 * n * D + 16 * s + 2 * i);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int n = 0; n < NT; ++n) acc[n] = mfma_f32(a[n][i], xf[s][i], acc[n]);
+        for (int n = 0; n < NT; ++n) mx[n] = mfma_f64(a[n][i >> 1][i & 1], xf[s][i], mx[n]);
     }
-    float t1 = 0.f, t2 = 0.f;
 #pragma unroll
-    for (int s = 0; s < NT; ++s) {
-      const v4f kap = *reinterpret_cast<const v4f*>(gm + D * D + 16 * s + 4 * lg);
-      if (STATS) {
+    for (int s = 0; s < NT; ++s)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          t1 = fmaf(xf[s][i], kap[i], t1);
-          t2 = fmaf(xf[s][i], acc[s][i], t2);
+      for (int i = 0; i < 4; ++i) {
+        const double kap = gm[D * D + 16 * s + 4 * lg + i], xv = xf[s][i];
+        if (STATS) {
+          s1 = fma(xv, kap, s1);
+          s2 = fma(xv, mx[s][i], s2);
+        } else {
+          mx[s][i] = coef * (scale * mx[s][i] - mean * kap);
         }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[s][i] = coef * (scale * acc[s][i] - mean * kap[i]);
       }
-    }
-    s1 = static_cast<double>(t1) * scale;
-    s2 = static_cast<double>(t2) * scale * scale;
+    s1 *= scale;
+    s2 = s2 * scale * scale;
   }
 
   // the chunk's own pairs: tiles of 64 rows y
@@ -359,35 +386,41 @@ __global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void score_apply_kernel(
       score_tile<D>(s, yt, xf, li, lg);
       // rows past a length are zero on either side and add nothing; the pair
       // order matters in the diagonal tile alone
-      float t1 = 0.f, t2 = 0.f;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int yi = kRows * t0 + 16 * t + 4 * lg + i;
           const bool ok = t0 != xb || (PAIRS == Pairs::kBefore ? yi <= xi : yi >= xi);
-          const float v = s[t][i] * scale;
+          const double v = static_cast<double>(s[t][i]) * scale;
           if (STATS) {
-            t1 += ok ? v : 0.f;
-            t2 += ok ? v * v : 0.f;
+            s1 += ok ? v : 0.0;
+            s2 += ok ? v * v : 0.0;
           } else {
-            s[t][i] = ok ? coef * (v - mean) : 0.f;
+            s[t][i] = ok ? static_cast<float>(coef * (v - mean)) : 0.f;
           }
         }
-      if (STATS) {
-        s1 += t1;
-        s2 += t2;
-      } else {
-        weigh_tile<D>(acc, yt, s, li, lg);
+      if (!STATS) {
+        v4f tile[NT];   // fp32 over a tile, fp64 from there on
+        zero_frag(tile);
+        weigh_tile<D>(tile, yt, s, li, lg);
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) mx[n][i] += tile[n][i];
       }
     }
   }
   if (!STATS) {
     if (xi >= Lx) return;
 #pragma unroll
-    for (int i = 0; i < NT; ++i)
-      store4(dx + row * D + 16 * i + 4 * lg,
-             xi < xlen ? acc[i] * scale : v4f{0.f, 0.f, 0.f, 0.f});
+    for (int n = 0; n < NT; ++n) {
+      v4f v = {0.f, 0.f, 0.f, 0.f};
+      if (xi < xlen)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = static_cast<float>(mx[n][i] * scale);
+      store4(dx + row * D + 16 * n + 4 * lg, v);
+    }
     return;
   }
   double n = xi < xlen && lg == 0 ? (PAIRS == Pairs::kAll ? ylen : min(xi + 1, ylen)) : 0.0;
@@ -410,7 +443,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void score_apply_kernel(
 
 // Gram matrices of y and their scan; nothing to do for causal rows of one chunk
 template <typename T, int D, Pairs PAIRS>
-int launch_gram(const T* y, const int64_t* length, int batch, int H, int L, float* gram,
+int launch_gram(const T* y, const int64_t* length, int batch, int H, int L, double* gram,
                 hipStream_t s) {
   const int nc = (L + kChunk - 1) / kChunk, size = D * D + D;
   if (PAIRS != Pairs::kAll && nc == 1) return 0;
@@ -435,7 +468,7 @@ int launch_gram(const T* y, const int64_t* length, int batch, int H, int L, floa
 
 template <typename T, int D, Pairs PAIRS, bool STATS>
 int launch_apply(const T* x, const T* y, const int64_t* x_length, const int64_t* y_length,
-                 int batch, int H, int Lx, int Ly, float scale, float* gram, const double* stats,
+                 int batch, int H, int Lx, int Ly, float scale, double* gram, const double* stats,
                  const float* g, double* part, T* dx, hipStream_t s) {
   const int rc = launch_gram<T, D, PAIRS>(y, y_length, batch, H, Ly, gram, s);
   if (rc) return rc;
@@ -450,7 +483,7 @@ int launch_apply(const T* x, const T* y, const int64_t* x_length, const int64_t*
 
 template <typename T, int D>
 int launch_moments(const void* q, const void* k, const int64_t* ql, const int64_t* kl, int batch,
-                   int H, int Lq, int Lk, int causal, float scale, double* part, float* gram,
+                   int H, int Lq, int Lk, int causal, float scale, double* part, double* gram,
                    double* out, float* std, hipStream_t s) {
   const T *qt = static_cast<const T*>(q), *kt = static_cast<const T*>(k);
   const int rc =
@@ -469,7 +502,7 @@ int launch_moments(const void* q, const void* k, const int64_t* ql, const int64_
 template <typename T, int D>
 int launch_std_bwd(const void* q, const void* k, const int64_t* ql, const int64_t* kl, int batch,
                    int H, int Lq, int Lk, int causal, float scale, const double* stats,
-                   const float* g, float* gram, void* dq, void* dk, hipStream_t s) {
+                   const float* g, double* gram, void* dq, void* dk, hipStream_t s) {
   const T *qt = static_cast<const T*>(q), *kt = static_cast<const T*>(k);
   T *dqt = static_cast<T*>(dq), *dkt = static_cast<T*>(dk);
   if (causal) {
@@ -594,11 +627,20 @@ extern "C" size_t sa_score_moments_workspace_size(int batch, int heads, int q_le
   if (batch <= 0 || heads <= 0 || q_len <= 0 || k_len <= 0 || head_dim <= 0) return 0;
   const size_t nc = (static_cast<size_t>(max(q_len, k_len)) + sa::kChunk - 1) / sa::kChunk;
   return moments_part(batch, heads, q_len) * sizeof(double) +
-         static_cast<size_t>(batch) * heads * nc * (head_dim * head_dim + head_dim) * sizeof(float);
+         static_cast<size_t>(batch) * heads * nc * (head_dim * head_dim + head_dim) * sizeof(double);
 }
 
-#define SA_MOMENTS_CASE(DD, FN, ...)                        case DD:                                                    return dtype == sa::kBF16 ? sa::FN<sa::bf16, DD>(__VA_ARGS__) : sa::FN<float, DD>(__VA_ARGS__)
-#define SA_MOMENTS_DISPATCH(FN, ...)         switch (head_dim) {                          SA_MOMENTS_CASE(32, FN, __VA_ARGS__);      SA_MOMENTS_CASE(64, FN, __VA_ARGS__);      SA_MOMENTS_CASE(96, FN, __VA_ARGS__);      SA_MOMENTS_CASE(128, FN, __VA_ARGS__);     default: return 1;                       }
+#define SA_MOMENTS_CASE(DD, FN, ...) \
+  case DD:                           \
+    return dtype == sa::kBF16 ? sa::FN<sa::bf16, DD>(__VA_ARGS__) : sa::FN<float, DD>(__VA_ARGS__)
+#define SA_MOMENTS_DISPATCH(FN, ...)       \
+  switch (head_dim) {                      \
+    SA_MOMENTS_CASE(32, FN, __VA_ARGS__);  \
+    SA_MOMENTS_CASE(64, FN, __VA_ARGS__);  \
+    SA_MOMENTS_CASE(96, FN, __VA_ARGS__);  \
+    SA_MOMENTS_CASE(128, FN, __VA_ARGS__); \
+    default: return 1;                     \
+  }
 
 extern "C" int sa_score_moments(int dtype, const void* q, const void* k, const int64_t* q_length,
                                 const int64_t* k_length, int batch, int heads, int q_len, int k_len,
@@ -613,7 +655,7 @@ extern "C" int sa_score_moments(int dtype, const void* q, const void* k, const i
                workspace_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
   double* part = static_cast<double*>(workspace);
-  float* gram = reinterpret_cast<float*>(part + moments_part(batch, heads, q_len));
+  double* gram = part + moments_part(batch, heads, q_len);
   SA_MOMENTS_DISPATCH(launch_moments, q, k, q_length, k_length, batch, heads, q_len, k_len, causal,
                       scale, part, gram, out, std, s)
 }
@@ -633,8 +675,7 @@ extern "C" int sa_score_std_bwd(int dtype, const void* q, const void* k, const i
                "sa_score_std_bwd: 16-byte aligned workspace of %zu B needed, %zu B given", need,
                workspace_bytes);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  float* gram = reinterpret_cast<float*>(static_cast<double*>(workspace) +
-                                         moments_part(batch, heads, q_len));
+  double* gram = static_cast<double*>(workspace) + moments_part(batch, heads, q_len);
   SA_MOMENTS_DISPATCH(launch_std_bwd, q, k, q_length, k_length, batch, heads, q_len, k_len, causal,
                       scale, stats, std_grad, gram, dq, dk, s)
 }

@@ -263,3 +263,42 @@ def test_score_std_dual_upstream_gradient(device, monkeypatch):
         want = torch.autograd.grad(std, ts, up, create_graph=True)
         for x, e in zip(got, want):
             torch.testing.assert_close(x[i], e.detach(), rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("D,L,causal", [(32, 600, True), (64, 2048, True), (96, 700, False),
+                                        (128, 1100, True)])
+@pytest.mark.parametrize("q_off,k_off,orthogonal", [(0, 0, False), (4, 4, False), (10, 10, False),
+                                                    (0, 100, True), (100, 0, True)])
+def test_score_std_with_common_components(q_off, k_off, orthogonal, D, L, causal, dtype):
+    """Vectors with a common part, which cancels in the variance, or meets nothing
+    on the other side: the std and its gradient against fp64 are no further off
+    than by the pass over every pair and the dense gradient, whose sums over the
+    pairs do not cancel before fp64 (or than one rounding to fp32 and the
+    products' own, 4 * 2^-24; bf16 gradients 2^-8)."""
+    from oracle import attn as ref
+    from selective_attention.kernels.attention import score_stats
+    g = torch.Generator().manual_seed(D + L)
+    q, k = (torch.randn(1, 2, L, D, generator=g) for _ in range(2))
+    if orthogonal:      # the other side has nothing along the common vector
+        e = torch.nn.functional.normalize(torch.randn(D, generator=g), dim=0)
+        q, k = (t - (t @ e)[..., None] * e for t in (q, k))
+        q, k = q + q_off * e, k + k_off * e
+    else:
+        q, k = q + q_off * torch.randn(D, generator=g).sign(), k + k_off * torch.randn(D, generator=g).sign()
+    q, k = q.to(dtype).cuda().requires_grad_(True), k.to(dtype).cuda().requires_grad_(True)
+    go = torch.randn(2, generator=g).cuda()
+    q64, k64 = (t.detach().cpu().double().requires_grad_(True) for t in (q, k))
+    std64 = ref.score_std(ref.score_stats(q64, k64, D ** -0.5, None, None, causal))
+    want = [std64] + list(torch.autograd.grad(std64, (q64, k64), go.cpu().double()))
+    std = M.ScoreStdFn.apply(q, k, None, None, causal)
+    got = [std] + list(torch.autograd.grad(std, (q, k), go, retain_graph=True))
+    pairs = ref.score_std(score_stats(q.detach(), k.detach(), None, None, causal)).float()
+    dense = [pairs] + list(torch.autograd.grad(std, (q, k), go, create_graph=True))
+    errs = [[float(((a.detach().cpu().double() - e).norm() / e.norm()).detach()) for a, e in zip(x, want)]
+            for x in (got, dense)]
+    print([f"{x:.1e}" for x in sum(errs, [])], flush=True)
+    for i, (mine, other) in enumerate(zip(*errs)):
+        one = 4 * 2.0 ** -24 if dtype == torch.float32 or i == 0 else 2.0 ** -8
+        assert mine <= max(1.1 * other, one), (("std", "dq", "dk")[i], mine, other)
