@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void score_apply_kernel(
   // rows y outside the chunk, through their Gram matrix
   const int c = PAIRS == Pairs::kAll ? 0 : kRows * xb / kChunk;
   const bool outside =
-      PAIRS == Pairs::kAfter ? c + 1 < nc : PAIRS == Pairs::kAll || c > 0;
+      PAIRS == Pairs::kAfter ? kChunk * (c + 1) < ylen : ylen > 0 && (PAIRS == Pairs::kAll || c > 0);
   double s1 = 0.0, s2 = 0.0;
   if (outside) {
     const double* gm = gram + (static_cast<long>(bh) * nc + c) * (D * D + D);
@@ -367,8 +367,8 @@ __global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void score_apply_kernel(
           mx[s][i] = coef * (scale * mx[s][i] - mean * kap);
         }
       }
-    s1 *= scale;
-    s2 = s2 * scale * scale;
+    s1 = xi < xlen ? s1 * scale : 0.0;   // (a zero row times an infinite sum is no number)
+    s2 = xi < xlen ? s2 * scale * scale : 0.0;
   }
 
   // the chunk's own pairs: tiles of 64 rows y
@@ -384,14 +384,17 @@ __global__ __launch_bounds__(256, D <= 64 ? 3 : 1) void score_apply_kernel(
       if (t0 < last) tile_load<D>(yr, yh, D, kRows * (t0 + 1), ylen, tid);
       v4f s[4];
       score_tile<D>(s, yt, xf, li, lg);
-      // rows past a length are zero on either side and add nothing; the pair
-      // order matters in the diagonal tile alone
+      // the pair order matters in the diagonal tile, lengths in the last ones
+      const bool edge = t0 == xb || kRows * (t0 + 1) > ylen || kRows * (xb + 1) > xlen;
 #pragma unroll
       for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int yi = kRows * t0 + 16 * t + 4 * lg + i;
-          const bool ok = t0 != xb || (PAIRS == Pairs::kBefore ? yi <= xi : yi >= xi);
+          bool ok = true;
+          if (edge)
+            ok = xi < xlen && yi < ylen &&
+                 (t0 != xb || (PAIRS == Pairs::kBefore ? yi <= xi : yi >= xi));
           const double v = static_cast<double>(s[t][i]) * scale;
           if (STATS) {
             s1 += ok ? v : 0.0;

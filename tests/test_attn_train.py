@@ -302,3 +302,33 @@ def test_score_std_with_common_components(q_off, k_off, orthogonal, D, L, causal
     for i, (mine, other) in enumerate(zip(*errs)):
         one = 4 * 2.0 ** -24 if dtype == torch.float32 or i == 0 else 2.0 ** -8
         assert mine <= max(1.1 * other, one), (("std", "dq", "dk")[i], mine, other)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_score_std_past_the_lengths(value):
+    """Rows outside the valid pairs hold anything: past their length, and for the
+    std (whose gradient multiplies them by 0) keys that no query sees."""
+    from selective_attention.kernels.attention import score_stats
+    b, H, L, D = 3, 2, 900, 64
+    g = torch.Generator().manual_seed(1)
+    q, k = (torch.randn(b, H, L, D, generator=g).cuda() for _ in range(2))
+    ql, kl = torch.tensor([900, 300, 0]).cuda(), torch.tensor([700, 600, 0]).cuda()
+
+    def fill(x, q_len, k_len):
+        a, e = q.clone(), k.clone()
+        for i in range(b):
+            a[i, :, int(q_len[i]):] = x
+            e[i, :, int(k_len[i]):] = x
+        return a.requires_grad_(True), e.requires_grad_(True)
+    want = M.ScoreStdFn.apply(*fill(0.0, ql, kl), ql, kl)
+    unseen = fill(value, ql, torch.minimum(ql, kl))
+    assert torch.equal(M.ScoreStdFn.apply(*unseen, ql, kl), want) and torch.isfinite(want).all()
+    torch.testing.assert_close(M.score_moments(*unseen, ql, kl)[0], score_stats(*unseen, ql, kl),
+                               rtol=1e-6, atol=1e-2)
+    grads = []
+    for x in (0.0, value):
+        ts = fill(x, ql, kl)
+        grads.append(torch.autograd.grad(M.ScoreStdFn.apply(*ts, ql, kl).sum(), ts))
+    for a, e in zip(*grads):
+        assert torch.isfinite(a).all() and torch.equal(a, e)
