@@ -142,6 +142,10 @@ class SelectiveMHA(nn.Module):
             kept = kept.any()
         v = self.v_proj(hidden_states)
         any_kept = _later_bool(kept)
+        # with every key dropped each query attends only itself (:208-209): told
+        # after the launches where these cannot refuse, before them elsewhere
+        if not (kept.is_cuda and D in (64, 128) and b * L > 0) and not any_kept():
+            return self.out_proj(v * out_gate)
         q, k = self.rope.rotate_qk(self.q_proj(hidden_states).view(b, L, H, D),
                                    self.k_proj(hidden_states).view(b, L, H, D), None, L)
         q, k = q.transpose(1, 2), k.transpose(1, 2)                   # (b, H, L, D) views

@@ -366,3 +366,19 @@ def test_prefill_with_every_key_dropped(causal):
         got = m(x, attn_gate_threshold=2.0, cache=cache)
         exp = m.out_proj(m.v_proj(x) * m._gates(x)[1])
     assert torch.equal(got, exp) and cache.pages is None
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("head_dim,L", [(32, 5), (64, 5), (64, 0)])
+def test_prompt_with_every_key_dropped(head_dim, L, device, causal):
+    """Each query attends itself alone: no attention runs, so any head_dim, an
+    empty prompt and a module on the CPU do."""
+    from selective_attention.modules.selective_attention import SelectiveMHA
+    torch.manual_seed(0)
+    m = SelectiveMHA(0, 128, head_dim, 2.0, is_causal=causal).to(device).eval()
+    x = torch.randn(2, L, 128, device=device)
+    with torch.no_grad():
+        out = m(x, attn_gate_threshold=2.0)
+        gate = torch.sigmoid(m.gate_proj(x))[..., m.num_heads:]
+        torch.testing.assert_close(out, m.out_proj(m.v_proj(x) * gate))
