@@ -410,7 +410,7 @@ class PagedSelectiveAttnCache:
             lens = torch.tensor(self.lens, dtype=torch.int32).to(self.device)
             paged_kv_append(k_rot, v, log_gate, self.page_table(), lens, self.k_pages,
                             self.v_pages, self.gate_pages)
-            self.lens = [n + 1 for n in self.lens]
+            self.lens[:] = [n + 1 for n in self.lens]   # (in place, as everywhere)
             self._sl, self._sl_dirty = lens, False
             return
         idx = torch.tensor(slots, dtype=torch.int64).to(self.device)

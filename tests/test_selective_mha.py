@@ -382,3 +382,17 @@ def test_prompt_with_every_key_dropped(head_dim, L, device, causal):
         out = m(x, attn_gate_threshold=2.0)
         gate = torch.sigmoid(m.gate_proj(x))[..., m.num_heads:]
         torch.testing.assert_close(out, m.out_proj(m.v_proj(x) * gate))
+
+
+@pytest.mark.gpu
+def test_append_advances_the_lengths_in_place():
+    """cache.lens is one list for the cache's life, as a caller may hold it; the
+    lengths that seq_lens handed out stay what they were."""
+    cache = PagedSelectiveAttnCache(2, 2, 64, max_tokens=128, device="cuda")
+    held, before = cache.lens, cache.seq_lens()
+    for n in (1, 2):
+        t = torch.zeros(2, 2, 64, device="cuda", dtype=torch.bfloat16)
+        cache.append(t, t, torch.zeros(2, 2, device="cuda"))
+        assert held is cache.lens and held == [n, n] and cache.seq_lens().tolist() == [n, n]
+        assert before.tolist() == [n - 1, n - 1]
+        before = cache.seq_lens()
