@@ -339,7 +339,7 @@ def test_score_std_past_the_lengths(value):
 @pytest.mark.parametrize("L,D", [(500, 128), (2048, 64), (4096, 32)])
 def test_no_further_off_than_the_dense_form(L, D, causal):
     """Long sums: every output's error against fp64 is that of the dense fp32 form
-    (torch's own sums over queries and keys), within the 10 % by which one draw's
+    (torch's own sums over queries and keys), within the 5 % by which one draw's
     error scatters."""
     *ts, do = inputs(1, 4, L, D, seed=L + 1)
     want = grads(lambda *t: M._gated_attention_dense(*t, causal), ts, do, torch.float64)
@@ -349,4 +349,4 @@ def test_no_further_off_than_the_dense_form(L, D, causal):
         errs.append([float((a.detach().double() - e.detach()).norm() / e.detach().norm()) for a, e in zip(got, want)])
     print([f"{x:.2e}" for x in sum(errs, [])], flush=True)
     for name, mine, dense in zip(("out", "dq", "dk", "dv", "dlog_gate"), *errs):
-        assert mine <= 1.1 * dense, (name, mine, dense)
+        assert mine <= 1.05 * dense, (name, mine, dense)
