@@ -21,10 +21,11 @@
 // short of 128-query blocks.  Small packed launches keep the block-sparse
 // kernel's dense form.
 // Measured, block-sparse kernel -> here: causal rows b 4, H 16, L 8192 (ragged),
-// D 64: 545 -> 403 us (the whole op 597 -> 407); bidirectional, 4 sequences of
-// 1500 to 4096, H 16, D 64, biased: 261 -> 214 us.  The same with a maximum per
-// block instead of the sum test, the biases scaled by every wave and 168
-// instead of 128 VGPRs: 234, 224 and 226 us.
+// D 64, the whole op: 574 -> 412 us; bidirectional, 4 sequences of 1500 to 4096,
+// H 16, D 64, biased: 253 -> 219 us (2 us of either are the columns that raise
+// their reference one by one).  Before that, 214 us, with a maximum per block
+// instead of the sum test 234, the biases scaled by every wave 224, 168 instead
+// of 128 VGPRs 226 us.
 #include "attn_tile.h"
 #include "prof.h"
 

@@ -21,14 +21,15 @@
 //
 // A 256-thread block owns 64 queries (64 keys in the dk / dv kernel), 16 per
 // wave, and streams 64-row tiles of the other side through one LDS stage;
-// the next tile's loads are in flight during a tile's products.  35 KB of
-// LDS lets four blocks share a CU, whose waves cover each other's barriers
-// and softmax.  Causal blocks do unequal work; they are issued longest first
+// the next tile's loads are in flight during a tile's products.  Registers set
+// how many blocks share a CU and cover each other's barriers and softmax (35 KB
+// of LDS would let four): at D 64, causal, 166 VGPRs in the forward, 198 for dq,
+// 232 for dk / dv, so three, two and two.  Causal blocks do unequal work; they are issued longest first
 // with every other 256 reversed, so that the blocks of a CU add up to about
 // the same.
 //
 // Measured at b 4, H 8, L 2048, D 64, causal (67 M pairs): forward 185 us,
-// dq 275 us, dk / dv 361 us, 92 to 95 TFLOP/s of fp32 MFMA each, 59 % of the
+// dq 266 us, dk / dv 359 us, 93 to 97 TFLOP/s of fp32 MFMA each, 60 % of the
 // 155 TFLOP/s that a large fp32 GEMM reaches here.  The dense form took 3.9 ms
 // for the same (elementwise passes over 0.5 GB score matrices, and products
 // over the masked half).

@@ -34,10 +34,10 @@ __device__ __forceinline__ int v_swz(int r) {
   else return (((r >> 1) & 1) << 2) | (((r >> 3) & 1) << 1) | ((r >> 4) & 1);
 }
 
-// Online softmax of the block-sparse kernel, with a lazy reference.  s[kt][i] holds log2-domain scores of
-// this lane's keys for query column lane & 15 (-inf where masked).  The
-// running reference m of a column (log2 domain, shared by its
-// four lane groups) is raised, and O and the partial sums rescaled, only when
+// Online softmax of the block-sparse kernel, with a lazy reference.  s[kt][i]
+// holds log2-domain scores of this lane's keys for query column lane & 15 (-inf
+// where masked).  The running reference m of a column (log2 domain, shared by
+// its four lane groups) is raised, and O and the partial sums rescaled, only when
 // some score exceeds it by more than 2^8: the common block needs no cross-lane
 // reduction at all, and probabilities stay <= 256.  l is this lane's partial
 // row sum (its own keys); the four lane groups' parts are added at the end.
