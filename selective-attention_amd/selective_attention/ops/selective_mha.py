@@ -163,14 +163,15 @@ class GatedAttnTrainFn(torch.autograd.Function):
 
 
 def _train_kernel_ok(q, k, v, log_gate) -> bool:
-    """Whether the training kernels take this call: plain device tensors of equal
-    shapes (the dense form broadcasts), a head_dim they are built for, and
-    nothing that has to see the dense form's own ops (autocast, tracing,
-    functorch transforms, forward-mode AD, dispatch modes)."""
+    """Whether the training kernels take this call: plain tensors of equal shapes
+    (the dense form broadcasts) on the current device (a launch does not switch
+    to another), a head_dim they are built for, and nothing that has to see the
+    dense form's own ops (autocast, tracing, functorch transforms, forward-mode
+    AD, dispatch modes)."""
     ts = (q, k, v, log_gate)
     return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda
                 and t.is_floating_point() and t.device == q.device for t in ts)
-            and q.dim() == 4 and q.shape == k.shape == v.shape and log_gate.shape == q.shape[:3]
+            and q.device.index == torch.cuda.current_device() and q.dim() == 4 and q.shape == k.shape == v.shape and log_gate.shape == q.shape[:3]
             and q.shape[-1] in TRAIN_HEAD_DIMS and 0 < q.numel()
             and q.shape[0] * q.shape[1] * ((q.shape[2] + 63) // 64) < 2 ** 31
             and not torch.is_autocast_enabled("cuda")

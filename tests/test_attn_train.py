@@ -122,8 +122,10 @@ def test_second_derivative_matches_dense():
 ])
 def test_score_std_through_gram_matrices(dtype, b, H, Lq, Lk, D, causal, ql, kl):
     """Counts exact; std and its gradient against the fp64 oracle at the edges of
-    the 64-row tiles and 256-row chunks.  fp32 sums of at most 2500 rows:
-    2500^0.5 * 2^-24 = 3e-6 relative on a Gram entry, 1e-5 with the products."""
+    the 64-row tiles and 256-row chunks, on vectors that share little (for what
+    cancels see test_score_std_with_common_components).  The scores are fp32
+    products of at most 128 terms, (128 / 4)^0.5 * 2^-24 = 3e-7 of the score,
+    and a tile's gradient sum the same; 1e-5 leaves room for single entries."""
     from oracle import attn as ref
     g = torch.Generator().manual_seed(Lq)
     q = (torch.randn(b, H, Lq, D, generator=g) + 0.2).to(dtype)
@@ -350,3 +352,13 @@ def test_no_further_off_than_the_dense_form(L, D, causal):
     print([f"{x:.2e}" for x in sum(errs, [])], flush=True)
     for name, mine, dense in zip(("out", "dq", "dk", "dv", "dlog_gate"), *errs):
         assert mine <= 1.05 * dense, (name, mine, dense)
+
+
+@pytest.mark.gpu
+def test_another_current_device_takes_the_dense_form(monkeypatch):
+    *ts, _ = inputs(1, 2, 40, 64, seed=4)
+    assert M._train_kernel_ok(*ts)
+    want = M._gated_attention_dense(*ts, True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    assert not M._train_kernel_ok(*ts)
+    assert torch.equal(gated_attention_train(*ts), want)
