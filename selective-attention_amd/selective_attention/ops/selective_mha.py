@@ -120,16 +120,17 @@ def _gated_attention_dense(q, k, v, log_gate, causal):
     return torch.matmul(torch.softmax(s, dim=-1), v)
 
 
-def _needs_torch_ops(t: torch.Tensor) -> bool:
-    """Whether something has to see torch's own ops on t, which a kernel launch
-    hides or cannot serve: a functorch or legacy batched wrapper (vmap,
-    is_grads_batched), forward-mode AD, a dispatch mode, tracing."""
-    return (torch._C._functorch.is_functorch_wrapped_tensor(t)
-            or torch._C._functorch.is_legacy_batchedtensor(t)
-            or torch._C._are_functorch_transforms_active()
+def _needs_torch_ops(*ts: torch.Tensor) -> bool:
+    """Whether something has to see torch's own ops on ts, which a kernel launch
+    hides or cannot serve: forward-mode AD, a dispatch mode, tracing, a functorch
+    transform, or a legacy batched tensor (is_grads_batched)."""
+    return (torch._C._are_functorch_transforms_active()
             or torch.autograd.forward_ad._current_level >= 0
             or torch._C._len_torch_dispatch_stack() > 0
-            or torch.compiler.is_compiling() or torch.jit.is_tracing())
+            or torch.compiler.is_compiling() or torch.jit.is_tracing()
+            # (on the tensors too: a GPU backward runs on a thread of its own)
+            or any(torch._C._functorch.is_functorch_wrapped_tensor(t)
+                   or torch._C._functorch.is_legacy_batchedtensor(t) for t in ts))
 
 
 class GatedAttnTrainFn(torch.autograd.Function):
@@ -175,7 +176,7 @@ def _train_kernel_ok(q, k, v, log_gate) -> bool:
             and q.shape[-1] in TRAIN_HEAD_DIMS and 0 < q.numel()
             and q.shape[0] * q.shape[1] * ((q.shape[2] + 63) // 64) < 2 ** 31
             and not torch.is_autocast_enabled("cuda")
-            and not any(_needs_torch_ops(t) for t in ts))
+            and not _needs_torch_ops(*ts))
 
 
 def gated_attention_train(q_rot, k_rot, v, log_gate, causal=True):
